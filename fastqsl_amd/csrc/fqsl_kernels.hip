@@ -5,7 +5,7 @@
 //   k_scott_persistent     Scott tracer, persistent grid, per-lane refill
 //                          from a device work queue (one line per lane)
 //   k_scott_per_line       Scott tracer, one thread per line
-//   k_plain_persistent / k_plain_per_line   position-only tracer (grid-index
+//   k_plain_quads / k_plain_sides   position-only tracer (grid-index
 //                          coordinates, or a stretched grid's own coordinates)
 //   k_qcalc_plane          QCalcPlane (FastQSL.py:65-117)
 //   k_pseudo_*             CookPseudoLine compaction (FastQSL.py:4-57)
@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "fqsl.h"
+#include "fqsl_quad.h"
 #include "fqsl_stretch.h"
 #include "fqsl_tracer.h"
 
@@ -404,7 +405,7 @@ extern "C" int fqsl_field_stretched(const fqsl_field* f) { return f && f->stretc
 
 // ------------------------------------------------------------- tuning knobs
 // Read by every launch, written by fqsl_tune_set from any host thread.
-static std::atomic<int> g_tune[FQSL_TUNE_COUNT] = {3, 100, 1, 8, 1, 64, 64, 1};
+static std::atomic<int> g_tune[FQSL_TUNE_COUNT] = {3, 100, 1, 8, 1, 64, 32, 1};
 
 extern "C" int fqsl_tune_set(int knob, int value) {
     if (knob < 0 || knob >= FQSL_TUNE_COUNT) return set_err(FQSL_ERR_INVALID, "tuning knob %d", knob);
@@ -904,132 +905,12 @@ k_scott_per_line_w3(F f, ScottParams P, Seeds s, unsigned long long n, ScottOut 
 }
 
 // ------------------------------------------------------------ plain kernels
-template <typename R, class F>
-__device__ __forceinline__ void plain_write(const PlainLine<R>& L, const F& f, const PlainParams& P,
-                                            unsigned long long i, const PlainOut& o, const DevScalars& ds) {
-    const float xs[3] = {(float)L.xs[0], (float)L.xs[1], (float)L.xs[2]};
-    const float xe[3] = {(float)L.xe[0], (float)L.xe[1], (float)L.xe[2]};
-    if (o.sx) { o.sx[i] = xs[0]; o.sy[i] = xs[1]; o.sz[i] = xs[2]; }
-    if (o.ex) { o.ex[i] = xe[0]; o.ey[i] = xe[1]; o.ez[i] = xe[2]; }
-    if (o.fs) o.fs[i] = L.flag_s;
-    if (o.fe) o.fe[i] = L.flag_e;
-    if (o.len) o.len[i] = L.len_total;
-    if (o.evals) o.evals[i] = L.evals;
-    if (o.tw) o.tw[i] = L.tw;
-    float b[3];
-    if (o.bsx) { b_clamped<R>(f, xs, b); o.bsx[i] = b[0]; o.bsy[i] = b[1]; o.bsz[i] = b[2]; }
-    if (o.bex) { b_clamped<R>(f, xe, b); o.bex[i] = b[0]; o.bey[i] = b[1]; o.bez[i] = b[2]; }
-    b_clamped<R>(f, L.p0, b);
-    if (o.btx) { o.btx[i] = b[0]; o.bty[i] = b[1]; o.btz[i] = b[2]; }
-    if (o.bflag) {
-        // TraceBlineAdaptive.cu:498-501, in float as the reference
-        const float bn = fabsf(b[0] * P.ncross[0] + b[1] * P.ncross[1] + b[2] * P.ncross[2]) * 100.f;
-        o.bflag[i] = bn < sqrtf(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]) ? 1 : 0;
-    }
-}
-
-// The stretched tracer writes B_start / B_end / B_this by the stretched
-// Interp3dxyzn (raw, TraceBlineAdaptiveStretch.cu:463-496).
-template <typename R, class F, bool kL = false>
-__device__ __forceinline__ void stretch_write(const PlainLine<R>& L, const F& f, const FQSL_CONST StretchGrid<R>& g,
-                                              const PlainParams& P, unsigned long long i, const PlainOut& o) {
-    const float xs[3] = {(float)L.xs[0], (float)L.xs[1], (float)L.xs[2]};
-    const float xe[3] = {(float)L.xe[0], (float)L.xe[1], (float)L.xe[2]};
-    if (o.sx) { o.sx[i] = xs[0]; o.sy[i] = xs[1]; o.sz[i] = xs[2]; }
-    if (o.ex) { o.ex[i] = xe[0]; o.ey[i] = xe[1]; o.ez[i] = xe[2]; }
-    if (o.fs) o.fs[i] = L.flag_s;
-    if (o.fe) o.fe[i] = L.flag_e;
-    if (o.len) o.len[i] = L.len_total;
-    if (o.evals) o.evals[i] = L.evals;
-    if (o.tw) o.tw[i] = L.tw;
-    double B[3];
-    if (o.bsx) {
-        const double p[3] = {xs[0], xs[1], xs[2]};
-        stretch_raw_at<R, F, kL>(f, g, p, B);
-        o.bsx[i] = (float)B[0]; o.bsy[i] = (float)B[1]; o.bsz[i] = (float)B[2];
-    }
-    if (o.bex) {
-        const double p[3] = {xe[0], xe[1], xe[2]};
-        stretch_raw_at<R, F, kL>(f, g, p, B);
-        o.bex[i] = (float)B[0]; o.bey[i] = (float)B[1]; o.bez[i] = (float)B[2];
-    }
-    const double p0[3] = {L.p0[0], L.p0[1], L.p0[2]};
-    stretch_raw_at<R, F, kL>(f, g, p0, B);
-    const float b[3] = {(float)B[0], (float)B[1], (float)B[2]};
-    if (o.btx) { o.btx[i] = b[0]; o.bty[i] = b[1]; o.btz[i] = b[2]; }
-    if (o.bflag) {
-        const float bn = fabsf(b[0] * P.ncross[0] + b[1] * P.ncross[1] + b[2] * P.ncross[2]) * 100.f;
-        o.bflag[i] = bn < sqrtf(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]) ? 1 : 0;
-    }
-}
-
-// Geometry of the plain tracer: grid-index coordinates (the uniform tracers)
-// or a stretched grid; the overloads pick the line driver.
-struct UniformGrid {};
-
-template <typename R, class F>
-__device__ __forceinline__ void line_init(PlainLine<R>& L, const F& f, const UniformGrid&, const PlainParams& P,
-                                          float x, float y, float z) {
-    plain_init<R>(L, f, P, x, y, z);
-}
 template <typename R>
 __device__ __forceinline__ const FQSL_CONST StretchGrid<R>& grid_of(const StretchRef<R>& g) {
     return *(const FQSL_CONST StretchGrid<R>*)g.g;
 }
-
-template <typename R, class F>
-__device__ __forceinline__ void line_init(PlainLine<R>& L, const F& f, const StretchRef<R>& g, const PlainParams& P,
-                                          float x, float y, float z) {
-    stretch_init<R, F>(L, f, grid_of(g), P, x, y, z);
-}
-template <typename R, class F, class FJ>
-__device__ __forceinline__ void line_attempt(PlainLine<R>& L, const F& f, const UniformGrid&, const PlainParams& P,
-                                             const FJ& fj) {
-    plain_attempt<R, F, FJ>(L, f, P, fj);
-}
-template <typename R, class F, class FJ>
-__device__ __forceinline__ void line_attempt(PlainLine<R>& L, const F& f, const StretchRef<R>& g,
-                                             const PlainParams& P, const FJ& fj) {
-    stretch_attempt<R, F, FJ>(L, f, grid_of(g), P, fj);
-}
-template <typename R, class F>
-__device__ __forceinline__ void line_write(const PlainLine<R>& L, const F& f, const UniformGrid&, const PlainParams& P,
-                                           unsigned long long i, const PlainOut& o, const DevScalars& ds) {
-    plain_write<R>(L, f, P, i, o, ds);
-}
-template <typename R, class F>
-__device__ __forceinline__ void line_write(const PlainLine<R>& L, const F& f, const StretchRef<R>& g,
-                                           const PlainParams& P, unsigned long long i, const PlainOut& o,
-                                           const DevScalars&) {
-    stretch_write<R>(L, f, grid_of(g), P, i, o);
-}
-
-// A float stretched grid whose compact lookup table each workgroup copies to
-// LDS at the start (`lds_bytes` of dynamic shared memory): the bin record of
-// a stage point is then an LDS read instead of a global load that the cell
-// load has to wait for.
-struct StretchLds {
-    const StretchGrid<float>* g;
-    int lds_bytes;
-};
 __device__ __forceinline__ const FQSL_CONST StretchGrid<float>& grid_of(const StretchLds& g) {
     return *(const FQSL_CONST StretchGrid<float>*)g.g;
-}
-template <typename R, class F>
-__device__ __forceinline__ void line_init(PlainLine<R>& L, const F& f, const StretchLds& g, const PlainParams& P,
-                                          float x, float y, float z) {
-    stretch_init<R, F, true>(L, f, grid_of(g), P, x, y, z);
-}
-template <typename R, class F, class FJ>
-__device__ __forceinline__ void line_attempt(PlainLine<R>& L, const F& f, const StretchLds& g,
-                                             const PlainParams& P, const FJ& fj) {
-    stretch_attempt<R, F, FJ, true>(L, f, grid_of(g), P, fj);
-}
-template <typename R, class F>
-__device__ __forceinline__ void line_write(const PlainLine<R>& L, const F& f, const StretchLds& g,
-                                           const PlainParams& P, unsigned long long i, const PlainOut& o,
-                                           const DevScalars&) {
-    stretch_write<R, F, true>(L, f, grid_of(g), P, i, o);
 }
 
 // Kernel prologue per geometry: the LDS grid copies its table (every thread
@@ -1062,75 +943,209 @@ __device__ __forceinline__ void apply_plain_scalars(F& f, PlainParams& P, unsign
     P.ncross[0] = ncross[0]; P.ncross[1] = ncross[1]; P.ncross[2] = ncross[2];
 }
 
-// Persistent plain tracing: each lane owns one line (forward, then backward)
-// and writes its outputs when it ends; idle lanes take the next queue
-// entries once at least `refill_min` of the wavefront's lanes are idle (or
-// all are), so refills and their setup run together.
-template <typename R, class F, class FJ, class G>
-__global__ void __launch_bounds__(256) k_plain_persistent(F f, PlainParams P, Seeds s, unsigned long long n,
-                                                          PlainOut out, DevScalars ds, const float* ncross,
-                                                          unsigned long long* queue, int refill_min, FJ fj, G g) {
+// B at a seed: Interp3d's clamped value on a uniform grid, the raw interpolant
+// on a stretched one (TraceBlineAdaptiveStretch.cu:463-496).
+template <typename R, class F>
+__device__ __forceinline__ void seed_b(const F& f, const UniformGrid&, const float* p, float b[3]) {
+    b_clamped<R>(f, p, b);
+}
+template <typename R, class F, class G>
+__device__ __forceinline__ void seed_b(const F& f, const G& g, const float* p, float b[3]) {
+    const double q[3] = {p[0], p[1], p[2]};
+    double B[3];
+    stretch_raw_at<R, F>(f, grid_of(g), q, B);
+    b[0] = (float)B[0]; b[1] = (float)B[1]; b[2] = (float)B[2];
+}
+
+// The lines of an RKF45 trace that are nearly tangent to the plane: their
+// tolerance is 8000 times smaller (bn <= 0.05, TraceBlineAdaptive.cu:356), so
+// they take up to ten times the steps of any other line.  `count` of them are
+// listed, and marked per line.
+struct TangentLines {
+    unsigned* list;           // NULL: no split
+    unsigned char* marked;
+    unsigned long long* count;
+};
+
+// Outputs of a plain trace that belong to the line and not to one side (B at
+// the seed and B_flag, and zeros where the two sides add their share), and the
+// list of the tangent lines.
+template <typename R, class F, class G>
+__global__ void __launch_bounds__(256) k_plain_prep(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o,
+                                                    DevScalars ds, const float* ncross, TangentLines tl, G g) {
+#if defined(__HIP_DEVICE_COMPILE__)
     apply_plain_scalars(f, P, n, ds, ncross);
-    fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];  // J lives on B's grid
     grid_prologue(g);
-    PlainLine<R> L;
-    bool active = false;
-    bool drained = false;
-    unsigned long long idx = 0;
-    const int lane = __lane_id();
-    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (;;) {
-        if (!drained) {
-            const unsigned long long need = __ballot(!active);
-            const int cnt = __popcll(need);
-            if (cnt >= refill_min || need == ~0ull) {
-                const int leader = __ffsll((long long)need) - 1;
-                unsigned long long base = 0;
-                if (lane == leader) base = atomicAdd(queue, (unsigned long long)cnt);
-                base = bcast64(base, leader);
-                if (base + (unsigned long long)cnt >= n) drained = true;
-                if (!active) {
-                    idx = base + (unsigned long long)__popcll(need & below);
-                    if (idx < n) {
-                        line_init<R>(L, f, g, P, s.x[idx], s.y[idx], s.z[idx]);
-                        if (L.done) line_write<R>(L, f, g, P, idx, out, ds);
-                        else active = true;
-                    }
+    const SideTracer<3, R, F, NoCurrent, G> T(f, g, P, 0);
+    const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
+    for (unsigned long long i0 = blockIdx.x * (unsigned long long)blockDim.x; i0 < n; i0 += stride) {
+        const unsigned long long i = i0 + threadIdx.x;
+        const bool in = i < n;
+        bool tangent = false;
+        if (in) {
+            if (o.len) o.len[i] = 0.0;
+            if (o.tw) o.tw[i] = 0.0;
+            if (o.evals) o.evals[i] = 0u;
+            const float p0[3] = {s.x[i], s.y[i], s.z[i]};
+            if (tl.list) {
+                tangent = T.slope(p0) <= 0.05;
+                tl.marked[i] = tangent ? 1 : 0;
+            }
+            if (o.btx || o.bflag) {
+                float b[3];
+                seed_b<R, F>(f, g, p0, b);
+                if (o.btx) { o.btx[i] = b[0]; o.bty[i] = b[1]; o.btz[i] = b[2]; }
+                if (o.bflag) {
+                    // TraceBlineAdaptive.cu:498-501, in float as the reference
+                    const float bn = fabsf(b[0] * P.ncross[0] + b[1] * P.ncross[1] + b[2] * P.ncross[2]) * 100.f;
+                    o.bflag[i] = bn < sqrtf(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]) ? 1 : 0;
                 }
             }
         }
-        if (!__any(active)) {
-            if (drained) break;
-            continue;
+        const unsigned long long m = __ballot(tangent);
+        if (m != 0ull) {
+            const int lane = __lane_id(), leader = __ffsll((long long)m) - 1;
+            unsigned long long base = 0;
+            if (lane == leader) base = atomicAdd(tl.count, (unsigned long long)__popcll(m));
+            base = bcast64(base, leader);
+            if (tangent) tl.list[base + (unsigned long long)__popcll(m & ((1ull << lane) - 1ull))] = (unsigned)i;
         }
-        if (active) {
-            line_attempt<R, F, FJ>(L, f, g, P, fj);
-            if (L.done) {
-                line_write<R>(L, f, g, P, idx, out, ds);
-                active = false;
+    }
+#endif
+}
+
+// One pass over the sides of `n` lines (task t: forward or backward side of line
+// t / 2, or of list[t / 2]; lines with skip[line] set are left out): K = 3, every lane of the wavefront owns a side; K = 1, every quad
+// of the first `width` ones does.  Ended sides are landed and free places
+// refilled together, once `refill_min` places of the wavefront need it or none
+// is tracing, so the code either side of the stepping runs for several at a
+// time.  Places take their sides from the wavefront's own run of tasks; a run is
+// claimed from the queue a share of what is left at a time, because claims of
+// one counter pass at ~8 ns each (a claim per 16 sides of a 1024^2 map is itself
+// a millisecond).
+template <int K, typename R, class F, class FJ, class G>
+__device__ __forceinline__ void trace_sides(const F& f, const PlainParams& P, const Seeds& s, unsigned long long n,
+                                            const PlainOut& o, unsigned long long* queue, int width, int refill_min,
+                                            const unsigned* __restrict__ list, const unsigned char* __restrict__ skip,
+                                            const FJ& fj, const G& g) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int lane = __lane_id(), a = first_axis<K>();
+    const SideTracer<K, R, F, FJ, G> T(f, g, P, a);
+    const SideField<K, FJ> J(fj, a);
+    const unsigned long long places = K == 3 ? ~0ull : 0x1111111111111111ull;  // one lane of each place
+    const bool mine = (K == 3 ? lane : lane >> 2) < width;
+    const unsigned long long below = (1ull << (K == 3 ? lane : lane & ~3)) - 1ull;
+    const unsigned long long tasks = 2ull * n;
+    // a claim takes 1/4 of a wavefront's even share of the rest
+    const int share_shift = 66 - __clzll((long long)gridDim.x * (blockDim.x >> 6));
+    unsigned long long line = 0, next = 0, end = 0;
+    bool drained = false;
+    Side<K, R> L;
+    L.pend = kSideIdle;
+    for (;;) {
+        unsigned long long act = __ballot(L.pend == kSideActive);
+        const unsigned long long done = __ballot(L.pend >= 0);
+        const unsigned long long idle = drained ? 0ull : __ballot(L.pend == kSideIdle && mine);
+        int wait = __popcll((done | idle) & places);
+        while (act != 0ull && wait < refill_min) {
+            if (L.pend == kSideActive) T.attempt(L, J);
+            const unsigned long long now = __ballot(L.pend == kSideActive);
+            wait += __popcll((act ^ now) & places);
+            act = now;
+        }
+        if (act == 0ull && wait == 0) break;
+        if (L.pend >= 0) {
+            double x[K];
+            T.land(L, J, x);
+            const bool fwd = L.dir > 0;
+            float* px[3] = {fwd ? o.ex : o.sx, fwd ? o.ey : o.sy, fwd ? o.ez : o.sz};
+            float* pb[3] = {fwd ? o.bex : o.bsx, fwd ? o.bey : o.bsy, fwd ? o.bez : o.bsz};
+            int32_t* pf = fwd ? o.fe : o.fs;
+            if (px[0]) {
+#pragma unroll
+                for (int q = 0; q < K; ++q) (K == 3 ? px[q] : axis_of(px[0], px[1], px[2], a))[line] = (float)x[q];
+            }
+            if (pb[0]) {
+                double xo[K];
+                R B[K];
+#pragma unroll
+                for (int q = 0; q < K; ++q) xo[q] = T.geo.out_point(q, (float)x[q]);
+                T.template raw_at<F>(T.f, xo, B);
+#pragma unroll
+                for (int q = 0; q < K; ++q) (K == 3 ? pb[q] : axis_of(pb[0], pb[1], pb[2], a))[line] = (float)B[q];
+            }
+            if (K == 3 || (lane & 3) == 0) {
+                if (pf) pf[line] = L.pend;
+                if (o.len) atomicAdd(o.len + line, L.len);
+                if (o.evals) atomicAdd(o.evals + line, L.evals);
+                if (o.tw) atomicAdd(o.tw + line, L.tw);
+            }
+            L.pend = kSideIdle;
+        }
+        const unsigned long long need = __ballot(L.pend == kSideIdle && mine) & places;
+        if (need != 0ull && next == end && !drained) {
+            unsigned long long run = (tasks - end) >> share_shift;
+            run = run < (unsigned)width ? (unsigned)width : (run > 256ull ? 256ull : run);
+            unsigned long long base = 0;
+            if (lane == 0) base = atomicAdd(queue, run);
+            base = bcast64(base, 0);
+            next = base < tasks ? base : tasks;
+            end = base + run < tasks ? base + run : tasks;
+            if (next == end) drained = true;
+        }
+        if (need != 0ull && next != end) {
+            const unsigned long long t = next + (unsigned long long)__popcll(need & below);
+            next += (unsigned long long)__popcll(need);
+            if (next > end) next = end;
+            if (L.pend == kSideIdle && mine && t < end) {
+                line = list ? (unsigned long long)list[t >> 1] : t >> 1;
+                if (!skip || !skip[line]) {
+                    const float p0[3] = {K == 3 ? s.x[line] : axis_of(s.x, s.y, s.z, a)[line],
+                                         K == 3 ? s.y[line] : 0.f, K == 3 ? s.z[line] : 0.f};
+                    T.init(L, p0, (t & 1ull) ? -1 : 1);
+                }
             }
         }
     }
+#endif
 }
 
-// One thread per line.  Two waves per SIMD as the register target: the FP64
-// variants otherwise take 256 VGPRs plus AGPRs and run one wave per SIMD
-// (1.2-1.3x slower); the FP32 variants fit two waves either way.
+// Plain tracing, persistent (fqsl_quad.h), every side by a quad of lanes.
+// `spread` wavefronts share few sides before a wavefront takes a second one, so
+// that none waits for another's branch.  Bound by the dependent instructions of
+// the longest side, 0.17 (RK4) to 0.21 us (RKF45) an evaluation; one thread per
+// line took 1.05 us, its three axes in turn on one lane with a branch tree each.
+// 233 x 191 lines on a 128 x 130 x 96 multipole: 1.9 -> 0.6 ms.
 template <typename R, class F, class FJ, class G>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-k_plain_per_line(F f, PlainParams P, Seeds s, unsigned long long n,
-                                                        PlainOut out, DevScalars ds, const float* ncross, FJ fj,
-                                                        G g) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 2)))
+k_plain_quads(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, DevScalars ds, const float* ncross,
+              unsigned long long* queue, int spread, FJ fj, G g) {
     apply_plain_scalars(f, P, n, ds, ncross);
     fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];  // J lives on B's grid
     grid_prologue(g);
-    const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
-    for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < n; i += stride) {
-        PlainLine<R> L;
-        line_init<R>(L, f, g, P, s.x[i], s.y[i], s.z[i]);
-        while (!L.done) line_attempt<R, F, FJ>(L, f, g, P, fj);
-        line_write<R>(L, f, g, P, i, out, ds);
-    }
+    const unsigned long long share = (2ull * n + (unsigned)spread - 1) / (unsigned)spread;
+    const int width = share > 16ull ? 16 : (share < 1ull ? 1 : (int)share);
+    trace_sides<1, R, F, FJ, G>(f, P, s, n, o, queue, width, 4 < width ? 4 : width, nullptr, nullptr, fj, g);
+}
+
+// Many RKF45 sides: the listed tangent lines, whose long chains set the time,
+// go first, by quads, in the first `tangent_blocks` workgroups (one a CU: more
+// wavefronts would slow each other's chains, fewer start them late); a
+// wavefront that has none left goes on to all others, one side per lane.  On the
+// 1024^2 neighbour map (multipole 256^3; longest line 5,048 evaluations, mean
+// 103) 5.3 -> 1.8 ms, on the stretched 256^3 map 12.5 -> 5.0 ms; all sides by
+// quads take 2.4 and 5.9 ms, all by lanes 2.7 ms on the first.
+template <typename R, class F, class FJ, class G>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 2)))
+k_plain_sides(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, DevScalars ds, const float* ncross,
+              unsigned long long* queue, int refill_min, int tangent_blocks, TangentLines tl, FJ fj, G g) {
+    apply_plain_scalars(f, P, n, ds, ncross);
+    fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];
+    grid_prologue(g);
+    if (tl.list && blockIdx.x < (unsigned)tangent_blocks)
+        trace_sides<1, R, F, FJ, G>(f, P, s, *tl.count, o, queue, 16, 4, tl.list, nullptr, fj, g);
+    trace_sides<3, R, F, FJ, G>(f, P, s, n, o, queue + 1, 64, refill_min, nullptr,
+                                       tl.list ? tl.marked : nullptr, fj, g);
 }
 
 // ------------------------------------------------------------- launching
@@ -1360,47 +1375,66 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
     return set_err(FQSL_ERR_INVALID, "schedule %d", schedule);
 }
 
-// Workgroup size of the one-thread-per-line plain kernel: one wavefront on a
-// uniform grid (a finished wavefront frees its slot at once: 14.8 -> 12.7 ms
-// on 1024^2 lines of ~470 evaluations), four on a stretched grid, where the
-// four wavefronts of adjacent seeds sharing a CU's L1 outweigh that (16.5
-// against 16.7 ms; FP64 27.0 against 30.3 ms).
-static int per_line_block(const UniformGrid&) { return 64; }
-template <typename R>
-static int per_line_block(const StretchRef<R>&) { return 256; }
-static int per_line_block(const StretchLds&) { return 256; }
+// Wavefronts per SIMD over which few sides are spread before a wavefront takes
+// a second one.
+constexpr int kPlainSpread = 2;
+// Sides up to which an RKF45 launch is traced by quads alone, two per resident
+// quad.  On the multipole 256^3 field (s_len 1/8, tol_coef 0.5; ms by quads /
+// tangent lines by quads and the rest by lanes): 65 k sides 0.72 / 0.73, 131 k
+// 0.68 / 0.70, 262 k 0.90 / 0.84, 1.0 M 1.57 / 1.25, 2.1 M 2.38 / 1.74.  RK4
+// lines have no tangent class and all go by quads, whose two loads a stage touch
+// a third of the cache lines of a lane's six (2.1 M sides 10.4 against 11.9 ms).
+constexpr unsigned long long kPlainQuadSides = 131072;
 
+// Both schedules run the same kernels; a line's result does not depend on which
+// lanes trace it.
 template <typename R, class F, class FJ = NoCurrent, class G = UniformGrid>
 static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsigned long long n, const PlainOut& o,
                         const DevScalars& ds, const float* ncross, int schedule, hipStream_t st,
                         unsigned long long n_hint, const FJ& fj = FJ{}, const G& g = G{}) {
-    if (schedule == FQSL_SCHED_PERSISTENT) {
-        unsigned long long* q = nullptr;
-        int rc = queue_slot(&q);
-        if (rc) return rc;
-        int grid = 0;
-        const int lds = grid_lds_bytes(g);
-        rc = persistent_grid(k_plain_persistent<R, F, FJ, G>, &grid, lds);
-        if (rc) return rc;
+    (void)schedule;
+    unsigned long long* q = nullptr;
+    int rc = queue_slot(&q);
+    if (rc) return rc;
+    const int lds = grid_lds_bytes(g);
+    // The tangent lines of a large RKF45 launch are listed in a workspace of
+    // 5 bytes a line; a capturing stream takes no allocation and traces by quads.
+    TangentLines tl{nullptr, nullptr, q + 2};
+    char* ws = nullptr;
+    if (P.method == kRKF45 && 2ull * n_hint > kPlainQuadSides && n_hint < (1ull << 32)) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(hipStreamIsCapturing(st, &cap));
+        if (cap == hipStreamCaptureStatusNone) {
+            HIP_TRY(hipMallocAsync((void**)&ws, 5 * (size_t)n_hint, st));
+            tl.list = (unsigned*)ws;
+            tl.marked = (unsigned char*)ws + 4 * (size_t)n_hint;
+        }
+    }
+    int grid = 0;
+    rc = tl.list ? persistent_grid(k_plain_sides<R, F, FJ, G>, &grid, lds)
+                 : persistent_grid(k_plain_quads<R, F, FJ, G>, &grid, lds);
+    const unsigned long long blocks = (2ull * n_hint + 3) / 4;  // one side per wavefront at the least
+    if (blocks < (unsigned long long)grid) grid = (int)(blocks < 1 ? 1 : blocks);
+    if (rc == FQSL_OK) {
         k_zero_u64<<<1, 64, 0, st>>>(q, kQueueSlotWidth);
-        HIP_TRY(hipGetLastError());
         rc = record_start(st);
-        if (rc) return rc;
-        k_plain_persistent<R, F, FJ, G><<<grid, 256, lds, st>>>(f, P, s, n, o, ds, ncross, q,
-                                                             g_tune[FQSL_TUNE_PLAIN_REFILL], fj, g);
-        HIP_TRY(hipGetLastError());
-        return record_end(st);
     }
-    if (schedule == FQSL_SCHED_PER_LINE) {
-        int rc = record_start(st);
-        if (rc) return rc;
-        const int block = per_line_block(g);
-        k_plain_per_line<R, F, FJ, G><<<per_line_grid(n_hint, block, ds), block, grid_lds_bytes(g), st>>>(
-            f, P, s, n, o, ds, ncross, fj, g);
-        HIP_TRY(hipGetLastError());
-        return record_end(st);
+    if (rc == FQSL_OK && (tl.list || o.len || o.evals || o.tw || o.btx || o.bflag))
+        k_plain_prep<R, F, G><<<per_line_grid(n_hint, 256, ds), 256, lds, st>>>(f, P, s, n, o, ds, ncross, tl, g);
+    if (rc == FQSL_OK) {
+        if (tl.list)
+            k_plain_sides<R, F, FJ, G><<<grid, 256, lds, st>>>(f, P, s, n, o, ds, ncross, q,
+                                                               g_tune[FQSL_TUNE_PLAIN_REFILL], cu_count(), tl, fj, g);
+        else
+            k_plain_quads<R, F, FJ, G><<<grid, 256, lds, st>>>(f, P, s, n, o, ds, ncross, q,
+                                                               cu_count() * 4 * kPlainSpread, fj, g);
+        rc = record_end(st);
     }
-    return set_err(FQSL_ERR_INVALID, "schedule %d", schedule);
+    const hipError_t e = hipGetLastError();
+    const hipError_t ef = ws ? hipFreeAsync(ws, st) : hipSuccess;
+    if (e != hipSuccess) return set_err(FQSL_ERR_HIP, "plain trace launch: %s", hipGetErrorString(e));
+    if (ef != hipSuccess) return set_err(FQSL_ERR_HIP, "hipFreeAsync: %s", hipGetErrorString(ef));
+    return rc;
 }
 
 static int check_common(int method, int precision, int schedule, bool scott = false) {

@@ -165,8 +165,10 @@ FQSL_COLD CellWeight<T> stretch_search(const FQSL_CONST StretchAxis<T>* A, int b
 // Cell and weight of the stage coordinate phi + plo along one axis (phi the
 // leading part, plo a small remainder: the weight is formed as
 // ((phi - a[m]) + plo) / width so it keeps the remainder's resolution).
-template <typename T>
-FQSL_HD void stretch_locate(const FQSL_CONST StretchAxis<T>& A, int rule, T phi, T plo, int& c, T& w) {
+// `A` is the axis as the caller holds it (by reference into the grid, or a
+// lane's own copy), `ax` its place in the grid, for the search fallback.
+template <typename T, class AX>
+FQSL_HD void stretch_locate(const AX& A, const FQSL_CONST StretchAxis<T>* ax, int rule, T phi, T plo, int& c, T& w) {
     T p = phi + plo;
     if (!(p > A.lo)) { p = A.clo; phi = A.clo; plo = (T)0; }
     if (!(p < A.hi)) { p = A.chi; phi = A.chi; plo = (T)0; }
@@ -177,9 +179,14 @@ FQSL_HD void stretch_locate(const FQSL_CONST StretchAxis<T>& A, int rule, T phi,
     c = up ? br.m_hi : br.m_lo;
     w = ((phi - (up ? br.a_hi : br.a_lo)) + plo) * (up ? br.iw_hi : br.iw_lo);
     if (br.m_lo >= 0) return;
-    const CellWeight<T> s = stretch_search<T>(&A, b, rule, p, phi, plo);
+    const CellWeight<T> s = stretch_search<T>(ax, b, rule, p, phi, plo);
     c = s.c;
     w = s.w;
+}
+
+template <typename T>
+FQSL_HD void stretch_locate(const FQSL_CONST StretchAxis<T>& A, int rule, T phi, T plo, int& c, T& w) {
+    stretch_locate<T>(A, &A, rule, phi, plo, c, w);
 }
 
 FQSL_HD float float_of_bits(unsigned u) {
@@ -194,8 +201,9 @@ extern __shared__ uint2 fqsl_stretch_lds[];
 
 // stretch_locate<float> from the LDS copy: the same cell and weight bit for
 // bit (the same record fields, the same expressions).
-FQSL_HD void stretch_locate_lds(const FQSL_CONST StretchAxis<float>& A, int rule, float phi, float plo, int& c,
-                                float& w) {
+template <class AX>
+FQSL_HD void stretch_locate_lds(const AX& A, const FQSL_CONST StretchAxis<float>* ax, int rule, float phi, float plo,
+                                int& c, float& w) {
     float p = phi + plo;
     if (!(p > A.lo)) { p = A.clo; phi = A.clo; plo = 0.f; }
     if (!(p < A.hi)) { p = A.chi; phi = A.chi; plo = 0.f; }
@@ -209,7 +217,7 @@ FQSL_HD void stretch_locate_lds(const FQSL_CONST StretchAxis<float>& A, int rule
     const uint2 cw = fqsl_stretch_lds[A.lcell + c];
     w = ((phi - float_of_bits(cw.x)) + plo) * float_of_bits(cw.y);
     if (!multi) return;
-    const CellWeight<float> s = stretch_search<float>(&A, b, rule, p, phi, plo);
+    const CellWeight<float> s = stretch_search<float>(ax, b, rule, p, phi, plo);
     c = s.c;
     w = s.w;
 }
@@ -237,7 +245,7 @@ FQSL_HD void stretch_raw(const F& f, const FQSL_CONST StretchGrid<R>& g, const R
     R w[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        if constexpr (kL) stretch_locate_lds(g.ax[a], g.rule, phi[a], plo[a], c[a], w[a]);
+        if constexpr (kL) stretch_locate_lds(g.ax[a], &g.ax[a], g.rule, phi[a], plo[a], c[a], w[a]);
         else stretch_locate<R>(g.ax[a], g.rule, phi[a], plo[a], c[a], w[a]);
     }
     R cc[3][8];

@@ -315,26 +315,20 @@ FQSL_HD void coef_eval(const R c[3][8], R x, R y, R z, R B[3], R d[3][3]) {
     }
 }
 
+// Value of the trilinear interpolant only, one component.
 template <typename R>
-FQSL_HD void coef_value(const R c[3][8], R x, R y, R z, R B[3]) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const R A = (c[q][0] + c[q][2] * y) + x * (c[q][1] + c[q][4] * y);
-        const R C = (c[q][3] + c[q][5] * y) + x * (c[q][6] + c[q][7] * y);
-        B[q] = A + z * C;
-    }
+FQSL_HD R coef_value1(const R c[8], R x, R y, R z) {
+    const R A = (c[0] + c[2] * y) + x * (c[1] + c[4] * y);
+    const R C = (c[3] + c[5] * y) + x * (c[6] + c[7] * y);
+    return A + z * C;
 }
 
-// Value of the trilinear interpolant only.
 template <typename R>
-FQSL_HD void cell_value(const R c[3][8], R wx, R wy, R wz, R B[3]) {
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const R e00 = c[q][0] + wx * (c[q][1] - c[q][0]), e10 = c[q][2] + wx * (c[q][3] - c[q][2]);
-        const R e01 = c[q][4] + wx * (c[q][5] - c[q][4]), e11 = c[q][6] + wx * (c[q][7] - c[q][6]);
-        const R f0 = e00 + wy * (e10 - e00), f1 = e01 + wy * (e11 - e01);
-        B[q] = f0 + wz * (f1 - f0);
-    }
+FQSL_HD R cell_value1(const R c[8], R wx, R wy, R wz) {
+    const R e00 = c[0] + wx * (c[1] - c[0]), e10 = c[2] + wx * (c[3] - c[2]);
+    const R e01 = c[4] + wx * (c[5] - c[4]), e11 = c[6] + wx * (c[7] - c[6]);
+    const R f0 = e00 + wy * (e10 - e00), f1 = e01 + wy * (e11 - e01);
+    return f0 + wz * (f1 - f0);
 }
 
 // Edge derivative along axis J only (the d[J] of cell_eval / coef_eval).
@@ -371,8 +365,11 @@ FQSL_HD void field_eval(const R c[3][8], R wx, R wy, R wz, R B[3], R d[3][3]) {
 
 template <class F, typename R>
 FQSL_HD void field_value(const R c[3][8], R wx, R wy, R wz, R B[3]) {
-    if constexpr (F::kCoef) coef_value<R>(c, wx, wy, wz, B);
-    else cell_value<R>(c, wx, wy, wz, B);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        if constexpr (F::kCoef) B[q] = coef_value1<R>(c[q], wx, wy, wz);
+        else B[q] = cell_value1<R>(c[q], wx, wy, wz);
+    }
 }
 
 template <class F, int J, typename R>

@@ -51,6 +51,7 @@ extern "C" {
                              stage points, stage positions, increments, error norm), controller and Q */
 
 /* how lines are mapped to lanes */
+/* The Scott tracer's schedules; the plain tracers take either and run the same kernels. */
 #define FQSL_SCHED_PERSISTENT 0 /* persistent grid, each lane refills from a device queue */
 #define FQSL_SCHED_PER_LINE 1   /* one thread per line, one launch */
 
@@ -495,9 +496,9 @@ int fqsl_TraceAllBlineStretch(float *Bx, float *By, float *Bz, int *BshapeN, flo
                                    coarse length estimate, 1 (default) = longest first up to 64 lines per
                                    persistent lane (ordering changes timing, never results) */
 #define FQSL_TUNE_ORDER_BUCKETS 5 /* length buckets of that order: power of two in [2, 256], default 64 */
-#define FQSL_TUNE_PLAIN_REFILL 6  /* idle lanes a wavefront of the persistent plain tracer gathers before it
-                                     refills them (1..64, default 64: a wavefront claims new lines
-                                     once all its lanes are idle) */
+#define FQSL_TUNE_PLAIN_REFILL 6  /* ended line sides a wavefront of the plain tracer gathers before it lands
+                                     them and takes new ones, where it traces one side per lane (1..64,
+                                     default 32; wavefronts that trace by quads of lanes gather 4) */
 #define FQSL_TUNE_STRETCH_LDS 7   /* FP32 stretched tracer: 1 (default) = each workgroup copies the axis
                                      lookup table to LDS when it fits 64 KiB; 0 = global-memory tables */
 #define FQSL_TUNE_COUNT 8
