@@ -89,29 +89,55 @@ __global__ void k_convert_to_f64(const float* in, double* out, long n) {
         out[i] = (double)in[i];
 }
 
-// One thread per cell: gather the 8 corners of the 3 components into 8 float4.
-__global__ void k_build_cells(const float* __restrict__ bx, const float* __restrict__ by,
-                              const float* __restrict__ bz, int nx, int ny, int nz, float4* __restrict__ cells) {
-    const long cx = nx - 1, cy = ny - 1, cz = nz - 1;
-    const long ncell = cx * cy * cz;
+// Cells of trilinear coefficients from the float field T (float, or a double
+// field rounded to float first, as the float arrays hold it).  A thread gathers
+// the 8 corners of the 3 components of one cell; a wavefront's 64 records go
+// through LDS so that each store instruction writes 1 KiB in one piece (written
+// by the thread that formed it, a record takes six stores of 16 bytes 128 bytes
+// apart, and two of padding).  Bound by the write of 128 bytes a cell: 256^3
+// nodes 0.87 -> 0.54 ms, 320 x 320 x 256 0.87 ms, 4.2 TB/s where a large copy
+// reaches 4.75.
+constexpr int kCellLds = 28;  // floats a record takes in LDS: 24, and 4 so that rows start in different banks
+template <typename T>
+__global__ void __launch_bounds__(256) k_build_cells(const T* __restrict__ bx, const T* __restrict__ by,
+                                                     const T* __restrict__ bz, int nx, int ny, int nz,
+                                                     float4* __restrict__ cells) {
+    __shared__ __align__(16) float lds[256 * kCellLds];
+    const unsigned cx = nx - 1, cy = ny - 1, cz = nz - 1;
+    const unsigned ncell = cx * cy * cz;  // below 2^31, as the node count is
     const long nxy = (long)nx * ny;
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < ncell; t += (long)gridDim.x * blockDim.x) {
-        const long i = t % cx, j = (t / cx) % cy, k = t / (cx * cy);
-        const long base = k * nxy + j * nx + i;
-        const float* comp[3] = {bx, by, bz};
-        float4* o = cells + 8 * t;
+    const T* comp[3] = {bx, by, bz};
+    const int lane = threadIdx.x & 63;
+    float* rec = lds + threadIdx.x * kCellLds;
+    const float* wave = lds + (threadIdx.x & ~63) * kCellLds;
+    for (unsigned long long b0 = blockIdx.x * 256ull; b0 < ncell; b0 += gridDim.x * 256ull) {
+        const unsigned t = (unsigned)b0 + threadIdx.x;
+        if (t < ncell) {
+            const unsigned row = t / cx, i = t - row * cx, k = row / cy, j = row - k * cy;
+            const long base = k * nxy + (long)j * nx + i;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            const float* b = comp[q];
-            float v[8], c8[8];
+            for (int q = 0; q < 3; ++q) {
+                const T* b = comp[q] + base;
+                float v[8], c8[8];
 #pragma unroll
-            for (int c = 0; c < 8; ++c) v[c] = b[base + (c & 1) + ((c >> 1) & 1) * nx + ((c >> 2) & 1) * nxy];
-            cell_coefs(v, c8);
-            o[2 * q] = make_float4(c8[0], c8[1], c8[2], c8[3]);
-            o[2 * q + 1] = make_float4(c8[4], c8[5], c8[6], c8[7]);
+                for (int c = 0; c < 8; ++c) v[c] = (float)b[(c & 1) + ((c >> 1) & 1) * nx + ((c >> 2) & 1) * nxy];
+                cell_coefs(v, c8);
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    *(float4*)(rec + 8 * q + 4 * c) = make_float4(c8[4 * c], c8[4 * c + 1], c8[4 * c + 2], c8[4 * c + 3]);
+            }
         }
-        o[6] = make_float4(0.f, 0.f, 0.f, 0.f);
-        o[7] = make_float4(0.f, 0.f, 0.f, 0.f);
+        __syncthreads();
+        // the wavefront's records, eight lanes to one: parts 0..5 of it, then the padding
+        const unsigned first = (unsigned)b0 + (threadIdx.x & ~63);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const unsigned c = 8 * s + (lane >> 3), part = lane & 7;
+            if (first + c < ncell)
+                cells[8ull * (first + c) + part] =
+                    part < 6 ? *(const float4*)(wave + c * kCellLds + 4 * part) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        __syncthreads();
     }
 }
 
@@ -122,15 +148,123 @@ static int grid_for(long n, int block) {
     return (int)g;
 }
 
+// Device memory of fields.  A series of snapshots creates and destroys fields
+// of one size, and allocating gigabytes costs far more than filling them: the
+// driver clears memory that was in use before (a 320 x 320 x 256 field created,
+// mapped at 256^2 and destroyed over and over: 119.9 ms, 6.0 with the blocks kept).  Blocks of destroyed fields are therefore kept for the next ones:
+// at most kFieldCacheBytes per device, the oldest given back first, all of them
+// when an allocation fails, and only blocks of 1 MiB and more.  A block is
+// reused for requests it exceeds by less than an eighth.
+constexpr size_t kFieldCacheBytes = 8ull << 30;
+constexpr size_t kFieldCacheMin = 1u << 20;
+struct FieldBlock {
+    int device;
+    void* ptr;
+    size_t bytes;
+};
+static std::mutex g_field_mu;
+static std::vector<FieldBlock>& field_cache() {  // oldest first; not destroyed at exit, when HIP may be gone
+    static std::vector<FieldBlock>* c = new std::vector<FieldBlock>();
+    return *c;
+}
+static std::unordered_map<void*, size_t>& field_sizes() {  // blocks in use that may be kept
+    static std::unordered_map<void*, size_t>* m = new std::unordered_map<void*, size_t>();
+    return *m;
+}
+
+static void field_cache_drop(int device, size_t keep) {  // the lock is held
+    size_t held = 0;
+    std::vector<FieldBlock>& c = field_cache();
+    for (size_t i = c.size(); i-- > 0;) {
+        if (c[i].device != device) continue;
+        held += c[i].bytes;
+        if (held > keep) {
+            held -= c[i].bytes;
+            (void)hipFree(c[i].ptr);
+            c.erase(c.begin() + i);
+        }
+    }
+}
+
+template <typename T>
+static hipError_t field_malloc(int device, T** out, size_t bytes) {
+    *out = nullptr;
+    if (bytes < kFieldCacheMin) return hipMalloc((void**)out, bytes);
+    std::lock_guard<std::mutex> lk(g_field_mu);
+    std::vector<FieldBlock>& c = field_cache();
+    int best = -1;
+    for (int i = 0; i < (int)c.size(); ++i)
+        if (c[i].device == device && c[i].bytes >= bytes && c[i].bytes - bytes <= bytes / 8 &&
+            (best < 0 || c[i].bytes < c[best].bytes))
+            best = i;
+    void* p = nullptr;
+    size_t got = bytes;
+    if (best >= 0) {
+        p = c[best].ptr;
+        got = c[best].bytes;
+        c.erase(c.begin() + best);
+    } else {
+        hipError_t e = hipMalloc(&p, bytes);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            field_cache_drop(device, 0);
+            e = hipMalloc(&p, bytes);
+            if (e != hipSuccess) return e;
+        }
+    }
+    field_sizes()[p] = got;
+    *out = (T*)p;
+    return hipSuccess;
+}
+
+// As hipFree, which waits for the device before the memory can be used again.
+static void field_release(int device, void* p) {
+    if (!p) return;
+    size_t bytes = 0;
+    {
+        std::lock_guard<std::mutex> lk(g_field_mu);
+        auto it = field_sizes().find(p);
+        if (it != field_sizes().end()) {
+            bytes = it->second;
+            field_sizes().erase(it);
+        }
+    }
+    int cur = -1;
+    if (bytes == 0 || bytes > kFieldCacheBytes || hipGetDevice(&cur) != hipSuccess ||
+        (cur != device && hipSetDevice(device) != hipSuccess)) {
+        (void)hipFree(p);
+        return;
+    }
+    const hipError_t e = hipDeviceSynchronize();
+    if (cur != device) (void)hipSetDevice(cur);
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        return;
+    }
+    std::lock_guard<std::mutex> lk(g_field_mu);
+    field_cache().push_back(FieldBlock{device, p, bytes});
+    field_cache_drop(device, kFieldCacheBytes);
+}
+
+static void build_cells(const void* const* b, int dtype, const int* n, float4* cells) {
+    const int g = grid_for((long)(n[0] - 1) * (n[1] - 1) * (n[2] - 1), 256);
+    if (dtype == FQSL_DTYPE_F64)
+        k_build_cells<double><<<g, 256>>>((const double*)b[0], (const double*)b[1], (const double*)b[2], n[0], n[1], n[2],
+                                          cells);
+    else
+        k_build_cells<float><<<g, 256>>>((const float*)b[0], (const float*)b[1], (const float*)b[2], n[0], n[1], n[2],
+                                         cells);
+}
+
 static void field_free(fqsl_field* f) {
     for (int q = 0; q < 3; ++q) {
-        if (f->soa32[q]) (void)hipFree(f->soa32[q]);
-        if (f->soa64[q]) (void)hipFree(f->soa64[q]);
-        if (f->cur32[q]) (void)hipFree(f->cur32[q]);
-        if (f->cur64[q]) (void)hipFree(f->cur64[q]);
+        field_release(f->device, f->soa32[q]);
+        field_release(f->device, f->soa64[q]);
+        field_release(f->device, f->cur32[q]);
+        field_release(f->device, f->cur64[q]);
     }
-    if (f->cell32) (void)hipFree(f->cell32);
-    if (f->curcell) (void)hipFree(f->curcell);
+    field_release(f->device, f->cell32);
+    field_release(f->device, f->curcell);
     if (f->axes_mem) (void)hipFree(f->axes_mem);
     delete f;
 }
@@ -153,24 +287,22 @@ extern "C" int fqsl_field_create(const void* bx, const void* by, const void* bz,
     const size_t esz = dtype == FQSL_DTYPE_F64 ? 8 : 4;
     // stage the input on the device in its own dtype
     void* staged[3] = {nullptr, nullptr, nullptr};
-    int rc = FQSL_OK;
     auto fail = [&](int code, const char* what, hipError_t e) {
         for (int q = 0; q < 3; ++q)
-            if (staged[q] && !on_device) (void)hipFree(staged[q]);
+            if (staged[q] && !on_device) field_release(f->device, staged[q]);
         field_free(f);
         return set_err(code, "%s: %s", what, hipGetErrorString(e));
     };
     for (int q = 0; q < 3; ++q) {
         if (on_device) { staged[q] = const_cast<void*>(src[q]); continue; }
-        hipError_t e = hipMalloc(&staged[q], nn * esz);
+        hipError_t e = field_malloc(f->device, &staged[q], nn * esz);
         if (e != hipSuccess) return fail(FQSL_ERR_NOMEM, "hipMalloc(field staging)", e);
         e = hipMemcpy(staged[q], src[q], nn * esz, hipMemcpyHostToDevice);
         if (e != hipSuccess) return fail(FQSL_ERR_HIP, "hipMemcpy(field)", e);
     }
-    const bool need32 = (layouts & (FQSL_LAYOUT_SOA32 | FQSL_LAYOUT_CELL32)) != 0;
     for (int q = 0; q < 3; ++q) {
-        if (need32) {
-            hipError_t e = hipMalloc(&f->soa32[q], nn * 4);
+        if (layouts & FQSL_LAYOUT_SOA32) {
+            hipError_t e = field_malloc(f->device, &f->soa32[q], nn * 4);
             if (e != hipSuccess) return fail(FQSL_ERR_NOMEM, "hipMalloc(soa32)", e);
             if (dtype == FQSL_DTYPE_F32) e = hipMemcpy(f->soa32[q], staged[q], nn * 4, hipMemcpyDeviceToDevice);
             else {
@@ -181,7 +313,7 @@ extern "C" int fqsl_field_create(const void* bx, const void* by, const void* bz,
             f->bytes += nn * 4;
         }
         if (layouts & FQSL_LAYOUT_SOA64) {
-            hipError_t e = hipMalloc(&f->soa64[q], nn * 8);
+            hipError_t e = field_malloc(f->device, &f->soa64[q], nn * 8);
             if (e != hipSuccess) return fail(FQSL_ERR_NOMEM, "hipMalloc(soa64)", e);
             if (dtype == FQSL_DTYPE_F64) e = hipMemcpy(f->soa64[q], staged[q], nn * 8, hipMemcpyDeviceToDevice);
             else {
@@ -194,9 +326,9 @@ extern "C" int fqsl_field_create(const void* bx, const void* by, const void* bz,
     }
     if (layouts & FQSL_LAYOUT_CELL32) {
         const long ncell = (long)(nx - 1) * (ny - 1) * (nz - 1);
-        hipError_t e = hipMalloc(&f->cell32, ncell * 128);
+        hipError_t e = field_malloc(f->device, &f->cell32, ncell * 128);
         if (e != hipSuccess) return fail(FQSL_ERR_NOMEM, "hipMalloc(cell32)", e);
-        k_build_cells<<<grid_for(ncell, 256), 256>>>(f->soa32[0], f->soa32[1], f->soa32[2], nx, ny, nz, f->cell32);
+        build_cells(staged, dtype, f->n, f->cell32);
         e = hipGetLastError();
         if (e != hipSuccess) return fail(FQSL_ERR_HIP, "k_build_cells", e);
         f->bytes += ncell * 128;
@@ -204,12 +336,7 @@ extern "C" int fqsl_field_create(const void* bx, const void* by, const void* bz,
     hipError_t e = hipDeviceSynchronize();
     if (e != hipSuccess) return fail(FQSL_ERR_HIP, "field build", e);
     for (int q = 0; q < 3; ++q)
-        if (!on_device && staged[q]) (void)hipFree(staged[q]);
-    if (!(layouts & FQSL_LAYOUT_SOA32) && (layouts & FQSL_LAYOUT_CELL32)) {
-        // the float SoA copy was only needed to build the cells
-        for (int q = 0; q < 3; ++q) { (void)hipFree(f->soa32[q]); f->soa32[q] = nullptr; f->bytes -= nn * 4; }
-    }
-    (void)rc;
+        if (!on_device) field_release(f->device, staged[q]);
     *out = f;
     return FQSL_OK;
 }
@@ -232,22 +359,22 @@ extern "C" int fqsl_field_set_current(fqsl_field* f, const void* jx, const void*
     const void* src[3] = {jx, jy, jz};
     const long ncell = (long)(f->n[0] - 1) * (f->n[1] - 1) * (f->n[2] - 1);
     for (int q = 0; q < 3; ++q) {
-        if (f->cur32[q]) { (void)hipFree(f->cur32[q]); f->cur32[q] = nullptr; f->bytes -= nn * 4; }
-        if (f->cur64[q]) { (void)hipFree(f->cur64[q]); f->cur64[q] = nullptr; f->bytes -= nn * 8; }
+        if (f->cur32[q]) { field_release(f->device, f->cur32[q]); f->cur32[q] = nullptr; f->bytes -= nn * 4; }
+        if (f->cur64[q]) { field_release(f->device, f->cur64[q]); f->cur64[q] = nullptr; f->bytes -= nn * 8; }
     }
-    if (f->curcell) { (void)hipFree(f->curcell); f->curcell = nullptr; f->bytes -= ncell * 128; }
+    if (f->curcell) { field_release(f->device, f->curcell); f->curcell = nullptr; f->bytes -= ncell * 128; }
     for (int q = 0; q < 3; ++q) {
         void* staged = const_cast<void*>(src[q]);
         if (!on_device) {
-            HIP_TRY(hipMalloc(&staged, nn * esz));
+            HIP_TRY(field_malloc(f->device, &staged, nn * esz));
             hipError_t e = hipMemcpy(staged, src[q], nn * esz, hipMemcpyHostToDevice);
             if (e != hipSuccess) {
-                (void)hipFree(staged);
+                field_release(f->device, staged);
                 return set_err(FQSL_ERR_HIP, "hipMemcpy(current): %s", hipGetErrorString(e));
             }
         }
-        hipError_t e = hipMalloc(&f->cur32[q], nn * 4);
-        if (e == hipSuccess) e = hipMalloc(&f->cur64[q], nn * 8);
+        hipError_t e = field_malloc(f->device, &f->cur32[q], nn * 4);
+        if (e == hipSuccess) e = field_malloc(f->device, &f->cur64[q], nn * 8);
         if (e == hipSuccess) {
             if (dtype == FQSL_DTYPE_F64) {
                 e = hipMemcpy(f->cur64[q], staged, nn * 8, hipMemcpyDeviceToDevice);
@@ -259,15 +386,15 @@ extern "C" int fqsl_field_set_current(fqsl_field* f, const void* jx, const void*
             if (e == hipSuccess) e = hipGetLastError();
             if (e == hipSuccess) e = hipDeviceSynchronize();
         }
-        if (!on_device) (void)hipFree(staged);
+        if (!on_device) field_release(f->device, staged);
         if (e != hipSuccess) return set_err(FQSL_ERR_HIP, "current layout: %s", hipGetErrorString(e));
         f->bytes += nn * 12;
     }
     if (f->cell32) {  // the FP32 tracers read B from cells; J the same way (6 vector loads, not 24 gathers)
-        hipError_t e = hipMalloc(&f->curcell, ncell * 128);
+        hipError_t e = field_malloc(f->device, &f->curcell, ncell * 128);
         if (e != hipSuccess) return set_err(FQSL_ERR_NOMEM, "hipMalloc(current cells): %s", hipGetErrorString(e));
-        k_build_cells<<<grid_for(ncell, 256), 256>>>(f->cur32[0], f->cur32[1], f->cur32[2], f->n[0], f->n[1], f->n[2],
-                                                     f->curcell);
+        const void* cur[3] = {f->cur32[0], f->cur32[1], f->cur32[2]};
+        build_cells(cur, FQSL_DTYPE_F32, f->n, f->curcell);
         e = hipGetLastError();
         if (e == hipSuccess) e = hipDeviceSynchronize();
         if (e != hipSuccess) return set_err(FQSL_ERR_HIP, "current cells: %s", hipGetErrorString(e));

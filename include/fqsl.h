@@ -73,6 +73,10 @@ typedef struct fqsl_field fqsl_field;
  * upload of Bx/By/Bz (demo/Q_RKF45CuPyScott.ipynb cell [4]). */
 int fqsl_field_create(const void *bx, const void *by, const void *bz, int nx, int ny, int nz,
                       int dtype, int on_device, int layouts, fqsl_field **out);
+/* Waits for the device.  Up to 8 GiB per device of the layouts' memory is kept
+ * for the next fields (fields of a time series have one size, and allocating
+ * gigabytes anew costs far more than filling them); it is given back when an
+ * allocation for a field fails or other fields' memory takes its place. */
 int fqsl_field_destroy(fqsl_field *field);
 /* Device bytes held by the field's layouts. */
 size_t fqsl_field_bytes(const fqsl_field *field);
