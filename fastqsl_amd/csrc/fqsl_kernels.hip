@@ -2,8 +2,10 @@
 //
 // Kernels:
 //   k_build_cells          SoA float field -> 128-byte cells of trilinear coefficients
-//   k_scott_persistent     Scott tracer, persistent grid, per-lane refill
-//                          from a device work queue (one line per lane)
+//   k_scott_quads          Scott tracer, persistent grid, lines refilled from a
+//                          device work queue, one line per quad of lanes
+//   k_scott_persistent     the same with one line per lane: the mixed variant
+//                          and large FP64 launches
 //   k_scott_per_line       Scott tracer, one thread per line
 //   k_plain_quads / k_plain_sides   position-only tracer (grid-index
 //                          coordinates, or a stretched grid's own coordinates)
@@ -30,6 +32,7 @@
 
 #include "fqsl.h"
 #include "fqsl_quad.h"
+#include "fqsl_quad_scott.h"
 #include "fqsl_stretch.h"
 #include "fqsl_tracer.h"
 
@@ -893,7 +896,7 @@ __global__ void __launch_bounds__(256) k_scott_prep(F f, ScottParams P, Seeds s,
 // queue entries once at least `refill_min` lanes of the wavefront are idle (or
 // all are), so the setup of refilled lines runs once for the group.  A wave
 // exits once every queue is empty and all its lanes are idle.
-template <typename R, class F, class FJ, typename X, bool kRoll = false>
+template <typename R, class F, class FJ, typename X>
 __device__ __forceinline__ void scott_persistent_body(F f, ScottParams P, Seeds s, unsigned long long n,
                                                       const R* __restrict__ frames, ScottRec<R>* __restrict__ recs,
                                                       DevScalars ds, unsigned long long* queues, int nq,
@@ -938,7 +941,7 @@ __device__ __forceinline__ void scott_persistent_body(F f, ScottParams P, Seeds 
         }
         if (active) {
             ScottEnd<R> e;
-            const int st = scott_attempt<R, F, FJ, X, kRoll>(L, f, P, e, fj);
+            const int st = scott_attempt<R, F, FJ, X>(L, f, P, e, fj);
             if (st != kTracing) {
                 recs[idx] = ScottRec<R>{L.st, e, L.len, st, L.evals, L.tw};
                 active = false;
@@ -947,17 +950,6 @@ __device__ __forceinline__ void scott_persistent_body(F f, ScottParams P, Seeds 
     }
 }
 
-// W = waves per SIMD the register allocation targets.
-#define FQSL_PERSISTENT_KERNEL(W)                                                                     \
-    template <typename R, class F, class FJ, typename X>                                              \
-    __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W)))                \
-    k_scott_persistent_w##W(F f, ScottParams P, Seeds s, unsigned long long n, const R* frames,       \
-                            ScottRec<R>* recs, DevScalars ds, unsigned long long* queues, int nq,     \
-                            int refill_min, const unsigned* order, FJ fj) {                           \
-        scott_persistent_body<R, F, FJ, X, W == 3>(f, P, s, n, frames, recs, ds, queues, nq, refill_min, order, \
-                                                  fj);                                                \
-    }
-
 template <typename R, class F, class FJ, typename X>
 __global__ void __launch_bounds__(256) k_scott_persistent(F f, ScottParams P, Seeds s, unsigned long long n,
                                                           const R* frames, ScottRec<R>* recs, DevScalars ds,
@@ -965,8 +957,186 @@ __global__ void __launch_bounds__(256) k_scott_persistent(F f, ScottParams P, Se
                                                           const unsigned* order, FJ fj) {
     scott_persistent_body<R, F, FJ, X>(f, P, s, n, frames, recs, ds, queues, nq, refill_min, order, fj);
 }
-FQSL_PERSISTENT_KERNEL(2)
-FQSL_PERSISTENT_KERNEL(3)
+// The mixed variant, at two waves per SIMD.
+template <typename R, class F, class FJ, typename X>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_scott_persistent_w2(F f, ScottParams P, Seeds s, unsigned long long n, const R* frames, ScottRec<R>* recs,
+                      DevScalars ds, unsigned long long* queues, int nq, int refill_min, const unsigned* order,
+                      FJ fj) {
+    scott_persistent_body<R, F, FJ, X>(f, P, s, n, frames, recs, ds, queues, nq, refill_min, order, fj);
+}
+
+// Persistent stepping with one line per quad of lanes (fqsl_quad_scott.h), the
+// first `width` quads of a wavefront each.  `src` tells a line's seed, step and
+// tolerance and is told when it is done.  Ended sides are landed, second sides
+// begun and free quads refilled together, once `refill_min` quads wait or none
+// is tracing; free quads take lines from the wavefront's own run, claimed a
+// share of the rest at a time (see trace_sides).
+template <typename R, class F, class FJ, class Src>
+__device__ __forceinline__ void scott_quads_body(const F& f, Src src, unsigned long long n,
+                                                 const R* __restrict__ frames, ScottRec<R>* __restrict__ recs,
+                                                 unsigned long long* queue, int width, int refill_min, const FJ& fj) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int lane = __lane_id(), a = first_axis<1>();
+    const bool writes = (lane & 3) != 3, first = (lane & 3) == 0;
+    ScottParams P = src.params();
+    const QuadScott<R, F, FJ> T(f, P, a);
+    const SideField<1, FJ> J(fj, a);
+    const unsigned long long kQuads = 0x1111111111111111ull;  // one lane of each
+    const bool mine = (lane >> 2) < width;
+    const unsigned long long below = (1ull << (lane & ~3)) - 1ull;
+    const int share_shift = 66 - __clzll((long long)gridDim.x * (blockDim.x >> 6));
+    unsigned long long line = 0, next = 0, end = 0;
+    bool drained = false;
+    QuadLine<R> L;
+    L.pend = kSideIdle;
+    for (;;) {
+        unsigned long long act = __ballot(L.pend == kSideActive);
+        const unsigned long long done = __ballot(L.pend >= 0);
+        const unsigned long long idle = drained ? 0ull : __ballot(L.pend == kSideIdle && mine);
+        int wait = __popcll((done | idle) & kQuads);
+        while (act != 0ull && wait < refill_min) {
+            if (L.pend == kSideActive) T.attempt(L, J);
+            const unsigned long long now = __ballot(L.pend == kSideActive);
+            wait += __popcll((act ^ now) & kQuads);
+            act = now;
+        }
+        if (act == 0ull && wait == 0) break;
+        bool begin = false;  // start the side L.dir
+        int status = kTracing;
+        if (L.pend >= 0) {
+            R fx, fu, fv;
+            T.land(L, fx, fu, fv);
+            ScottEnd<R>* e = L.dir < 0 ? &recs[line].st : &recs[line].en;
+            if (writes) { e->x[a] = fx; e->u[a] = fu; e->v[a] = fv; }
+            if (first) e->flag = L.pend;
+            if (L.pend == kClassOther) {  // q = 0; a forward side never traced keeps the seed
+                status = kAborted;
+                if (L.dir < 0) {
+                    e = &recs[line].en;
+                    if (writes) { e->x[a] = L.p0; e->u[a] = (R)0; e->v[a] = (R)0; }
+                    if (first) e->flag = kClassOther;
+                }
+            } else if (L.dir < 0) {
+                L.dir = 1;
+                begin = true;
+            } else {
+                status = kFinished;
+            }
+            L.pend = status == kTracing ? kSideActive : kSideIdle;
+        }
+        const unsigned long long need = __ballot(L.pend == kSideIdle && mine) & kQuads;
+        if (need != 0ull && next == end && !drained) {
+            unsigned long long run = (n - end) >> share_shift;
+            run = run < (unsigned)width ? (unsigned)width : (run > 128ull ? 128ull : run);
+            unsigned long long base = 0;
+            if (lane == 0) base = atomicAdd(queue, run);
+            base = bcast64(base, 0);
+            next = base < n ? base : n;
+            end = base + run < n ? base + run : n;
+            if (next == end) drained = true;
+        }
+        // an ended line is closed before its quad takes the next one
+        if (status != kTracing) {
+            if (first) {
+                ScottRec<R>& r = recs[line];
+                r.len = L.len; r.status = status; r.evals = L.evals; r.tw = L.tw;
+                src.done(line);
+            }
+            status = kTracing;
+        }
+        if (need != 0ull && next != end) {
+            const unsigned long long t = next + (unsigned long long)__popcll(need & below);
+            next += (unsigned long long)__popcll(need);
+            if (next > end) next = end;
+            if (L.pend == kSideIdle && mine && t < end) {
+                line = src.line(t);
+                L.p0 = src.seed(line, a, P);
+                L.len = 0.0;
+                L.tw = 0.0;
+                L.steps = 0; L.attempts = 0; L.evals = 0;
+                L.s = P.s0;
+                L.dir = -1;
+                L.pend = kSideActive;
+                if (quad_lane<2>(L.p0) < (R)-1e-8f) {  // TraceBlineScott.cu:366
+                    ScottRec<R>& r = recs[line];
+                    if (writes) { r.st.x[a] = L.p0; r.en.x[a] = L.p0; }
+                    if (first) r.st.flag = r.en.flag = kClassBelow;
+                    status = kFinished;
+                } else {
+                    begin = true;
+                }
+            }
+        }
+        // scott_begin_dir: the z0 shortcut (TraceBlineScott.cu:396-401) and sides
+        // that cannot take a step record their footpoint at once
+        while (begin) {
+            const R* fr = frames + (unsigned long long)kFrameWords * line;
+            const R u0 = fr[a], v0 = fr[3 + a], b0z = fr[6];
+            L.x.set_f((float)L.p0);
+            L.u = u0;
+            L.v = v0;
+            int cls = 5;
+            if (!((float)quad_lane<2>(L.p0) < 1e-6f && (double)b0z * L.dir < 0)) {
+                L.s = fabs(L.s);
+                if (T.can_step(L)) break;
+                cls = kClassLimit;
+            }
+            ScottEnd<R>* e = L.dir < 0 ? &recs[line].st : &recs[line].en;
+            if (writes) { e->x[a] = L.p0; e->u[a] = u0; e->v[a] = v0; }
+            if (first) e->flag = cls;
+            if (L.dir > 0) { status = kFinished; break; }
+            L.dir = 1;
+        }
+        if (status != kTracing) {
+            if (first) {
+                ScottRec<R>& r = recs[line];
+                r.len = L.len; r.status = status; r.evals = L.evals; r.tw = L.tw;
+                src.done(line);
+            }
+            L.pend = kSideIdle;
+        }
+    }
+#endif
+}
+
+// Lines of one request, in seed order or as `order` lists them.
+struct ScottLines {
+    Seeds s;
+    ScottParams P;
+    const unsigned* __restrict__ order;
+    __device__ __forceinline__ ScottParams params() const { return P; }
+    __device__ __forceinline__ unsigned long long line(unsigned long long t) const {
+        return order ? (unsigned long long)order[t] : t;
+    }
+    __device__ __forceinline__ float seed(unsigned long long i, int a, ScottParams&) const {
+        return a == 0 ? s.x[i] : (a == 1 ? s.y[i] : s.z[i]);
+    }
+    __device__ __forceinline__ void done(unsigned long long) const {}
+};
+
+// The lines of few launches fill the chip with one line a lane, and one lane
+// does a stage's three components in turn: a line's chain took 1.3 us an
+// evaluation, its six cell loads touch 384 cache lines a wavefront.  By quads
+// 0.5 us and a third of the cache lines, for 1.5 times the instructions a line;
+// FP32c launches of every size gain or stay (multipole 256^3, RKF45 1e-6, ms
+// before and after: 64 lines 1.87 / 0.78, 256^2 4.5 / 2.05, 512^2 5.9 / 3.0,
+// 1024^2 9.2 / 8.7; 512^2 with twist 5.2 / 3.1; cell cube of 8.4 M lines
+// 217 / 193).  Four wavefronts a SIMD: from 512^2 lines on bound by vector
+// instruction issue (98 instructions a stage of 16 lines, all issue slots
+// taken).  `spread` wavefronts share few lines before one takes a second.
+template <typename R, class F, class FJ>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1)))
+k_scott_quads(F f, ScottParams P, Seeds s, unsigned long long n, const R* frames, ScottRec<R>* recs, DevScalars ds,
+              unsigned long long* queue, int spread, int refill_min, const unsigned* order, FJ fj) {
+    apply_scalars(f, P, n, ds);
+    fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];  // J lives on B's grid
+    P.ctl = scott_ctl(P.tol);  // on the device, so every path forms the same bits
+    const unsigned long long share = (n + (unsigned)spread - 1) / (unsigned)spread;
+    const int width = share > 16ull ? 16 : (share < 1ull ? 1 : (int)share);
+    scott_quads_body<R, F, FJ>(f, ScottLines{s, P, order}, n, frames, recs, queue, width,
+                               refill_min < width ? refill_min : width, fj);
+}
 
 // Q assembly and output, one thread per line (TraceBlineScott.cu:475-508,
 // outputs as TraceAllBlineScott :565-582).
@@ -1372,26 +1542,61 @@ static int scott_waves(unsigned long long n) {
     return (w == 3 && n <= small_launch_lines()) ? 2 : w;
 }
 
-// Stepping kernel and grid of the persistent Scott schedule.
+// Stepping kernel and grid of the persistent Scott schedule; kern == nullptr: by
+// quads.  `lines`: how many are traced at a time.
 template <typename R, class F, class FJ, typename X>
-static int scott_persistent_kernel(decltype(&k_scott_persistent<R, F, FJ, X>)* kern, int* grid,
-                                   unsigned long long n) {
-    const int waves = scott_waves<R, X, FJ>(n);
-    *kern = waves == 2 ? k_scott_persistent_w2<R, F, FJ, X>
-          : waves == 3 ? k_scott_persistent_w3<R, F, FJ, X>
-                       : k_scott_persistent<R, F, FJ, X>;
-    int rc = persistent_grid(*kern, grid);
+struct ScottStepping {
+    decltype(&k_scott_persistent<R, F, FJ, X>) kern = nullptr;
+    int grid = 0;
+    unsigned long long lines = 0;
+};
+
+// FP64 lines up to which a launch goes by quads, eight a resident quad: above
+// it the quads' extra instructions cost more than their shorter chain gives (RK4
+// and RKF45 on a 128^3 field, ms by quads / by lanes: 16 k lines 4.0 / 7.3 and
+// 4.9 / 10.7, 102 k 4.7 / 7.6 and 7.4 / 12.0, 147 k 7.0 / 7.5 and 10.0 / 12.1,
+// 200 k 8.4 / 7.4 and 12.8 / 12.3).
+constexpr unsigned long long kScottQuadLinesFp64 = 131072;
+// Wavefronts per SIMD over which few lines are spread before a wavefront takes a
+// second one, and the quads that wait before ended sides are landed and free
+// quads refilled: every wait of an FP32c quad is an issue slot of the others
+// (1024^2 RK4 map 11.7 ms at one, 12.3 at two); the long FP64 service pays for
+// two (102 k lines 5.2 / 4.7 ms at one / two, 200 k 8.4 at both).
+constexpr int kScottSpread = 2;
+constexpr int kScottQuadRefillFp32 = 1, kScottQuadRefillFp64 = 2;
+
+template <typename R, class F, class FJ, typename X>
+static int scott_stepping(ScottStepping<R, F, FJ, X>* st, unsigned long long n) {
+    unsigned long long per_block = 64;  // quads
+    int rc = FQSL_OK;
+    st->kern = nullptr;
+    if constexpr (!std::is_same<R, X>::value) st->kern = k_scott_persistent_w2<R, F, FJ, X>;
+    else if constexpr (sizeof(R) == 8)
+        if (n > kScottQuadLinesFp64) st->kern = k_scott_persistent<R, F, FJ, X>;
+    if (st->kern) {
+        per_block = 256;
+        rc = persistent_grid(st->kern, &st->grid);
+    } else if constexpr (std::is_same<R, X>::value) {
+        rc = persistent_grid(k_scott_quads<R, F, FJ>, &st->grid);
+    }
     if (rc) return rc;
-    *grid = (int)((long)*grid * g_tune[FQSL_TUNE_GRID_PCT] / 100);
-    if (*grid < 1) *grid = 1;
+    st->grid = (int)((long)st->grid * g_tune[FQSL_TUNE_GRID_PCT] / 100);
+    if (st->grid < 1) st->grid = 1;
+    st->lines = per_block * (unsigned long long)st->grid;
     return FQSL_OK;
 }
 
-template <typename R>
-static bool scott_ordered(const DevScalars& ds, unsigned long long n_hint, int grid) {
+// Quads: not where every line is begun at once, nor with more than 16 lines a
+// quad, where the tail is short and the lost locality of the seeds costs more
+// (ms ordered / in seed order: 512^2 map 3.0 / 3.5, 1024^2 8.7 / 9.3, its RK4
+// 11.7 / 14.0; 2048^2 32.0 / 32.1, cube of 8.4 M lines 207 / 193; 64 lines
+// 0.83 / 0.78).  Lanes: up to 64 lines each.
+template <typename R, class F, class FJ, typename X>
+static bool scott_ordered(const DevScalars& ds, unsigned long long n_hint, const ScottStepping<R, F, FJ, X>& st) {
     const int om = g_tune[FQSL_TUNE_ORDER];
     return !ds.shape && n_hint < (1ull << 32) &&
-           (om == 2 || (om == 1 && n_hint <= 64ull * 256ull * (unsigned long long)grid));
+           (om == 2 || (om == 1 && (st.kern ? n_hint <= 64ull * st.lines
+                                            : n_hint > st.lines && n_hint <= 16ull * st.lines)));
 }
 
 // The persistent schedule's launches on `st` over a workspace `ws` laid out
@@ -1402,7 +1607,7 @@ static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, co
                                             const ScottOut& o, const DevScalars& ds, hipStream_t st,
                                             unsigned long long n_hint, const FJ& fj, char* ws, const ScottWs& w,
                                             bool ordered, unsigned long long* q,
-                                            decltype(&k_scott_persistent<R, F, FJ, X>) kern, int grid, bool timed) {
+                                            const ScottStepping<R, F, FJ, X>& step, bool timed) {
     R* frames = (R*)(ws + w.frames);
     ScottRec<R>* recs = (ScottRec<R>*)(ws + w.recs);
     unsigned* order = ordered ? (unsigned*)(ws + w.order) : nullptr;
@@ -1424,7 +1629,17 @@ static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, co
     }
     k_scott_prep<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(f, P, s, n, frames, o, ds);
     if (timed) e = hipEventRecord(g_evs0, st);
-    kern<<<grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, nq, refill_min, order, fj);
+    if constexpr (std::is_same<R, X>::value) {
+        if (!step.kern) {
+            const unsigned long long wanted = (n_hint + 3) / 4;  // one line per wavefront at the least
+            const int grid = wanted < (unsigned long long)step.grid ? (int)wanted : step.grid;
+            const int waves = std::min(step.grid, cu_count() * kScottSpread) * 4;
+            k_scott_quads<R, F, FJ><<<grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, waves,
+                                                          sizeof(R) == 4 ? kScottQuadRefillFp32 : kScottQuadRefillFp64,
+                                                          order, fj);
+        }
+    }
+    if (step.kern) step.kern<<<step.grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, nq, refill_min, order, fj);
     if (timed && e == hipSuccess) e = hipEventRecord(g_evs1, st);
     if (timed && e == hipSuccess) g_evs_valid = true;
     k_scott_finish<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(f, P, n, frames, recs, o, ds);
@@ -1457,11 +1672,10 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
     if (schedule == FQSL_SCHED_PERSISTENT) {
         // n_hint: number of lines, known on the host (sizes the workspace)
         if (n_hint == 0) return FQSL_OK;
-        decltype(&k_scott_persistent<R, F, FJ, X>) kern = nullptr;
-        int grid = 0;
-        int rc = scott_persistent_kernel<R, F, FJ, X>(&kern, &grid, n_hint);
+        ScottStepping<R, F, FJ, X> step;
+        int rc = scott_stepping<R, F, FJ, X>(&step, n_hint);
         if (rc) return rc;
-        const bool ordered = scott_ordered<R>(ds, n_hint, grid);
+        const bool ordered = scott_ordered(ds, n_hint, step);
         const ScottWs w = scott_ws_layout<R>(n_hint, ordered);
         if (noalloc) {  // device address of this device's scratch array: no allocation, no events
             if (w.bytes > kNoAllocScratchBytes - kNoAllocQueueBytes)
@@ -1471,7 +1685,7 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
             g_evs_valid = false;
             const hipError_t e = scott_persistent_launches<R, F, FJ, X>(
                 f, P, s, n, o, ds, st, n_hint, fj, noalloc + kNoAllocQueueBytes, w, ordered,
-                (unsigned long long*)noalloc, kern, grid, false);
+                (unsigned long long*)noalloc, step, false);
             if (e != hipSuccess) return set_err(FQSL_ERR_HIP, "Scott trace launch: %s", hipGetErrorString(e));
             return FQSL_OK;
         }
@@ -1481,7 +1695,7 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
         void* ws = nullptr;
         HIP_TRY(hipMallocAsync(&ws, w.bytes, st));
         const hipError_t e = scott_persistent_launches<R, F, FJ, X>(f, P, s, n, o, ds, st, n_hint, fj, (char*)ws,
-                                                                    w, ordered, q, kern, grid, true);
+                                                                    w, ordered, q, step, true);
         const hipError_t ef = hipFreeAsync(ws, st);
         if (e != hipSuccess) return set_err(FQSL_ERR_HIP, "Scott trace launch: %s", hipGetErrorString(e));
         if (ef != hipSuccess) return set_err(FQSL_ERR_HIP, "hipFreeAsync: %s", hipGetErrorString(ef));

@@ -73,6 +73,39 @@ __device__ __forceinline__ T pick_axis(const T* v, int dim) {
     all_axes<K>(v, a);
     return dim == 0 ? a[0] : (dim == 1 ? a[1] : a[2]);
 }
+// Float arithmetic on values of the quad's other lanes, as DPP operands of the
+// multiply-adds themselves.  (The compiler moves such operands to registers
+// first: it selects the three-address multiply-add, which has no DPP form.)  Two
+// wait states separate a register's last write from its reading by DPP; the
+// compiler cannot see into the block, so each begins with them.
+#define FQSL_Q0 " quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define FQSL_Q1 " quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define FQSL_Q2 " quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+
+// Sum over the three axes, on every lane.
+__device__ __forceinline__ int quad_sum(int v) {
+    int r;
+    asm("s_nop 1\n\t"
+        "v_add_u32_dpp %0, %1, %1 quad_perm:[1,2,0,1] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+        "v_add_u32_dpp %0, %1, %0 quad_perm:[2,0,1,2] row_mask:0xf bank_mask:0xf bound_ctrl:1"
+        : "=&v"(r) : "v"(v));
+    return r;
+}
+// coef_value1 with this lane's component c and the weight each lane holds.
+__device__ __forceinline__ float quad_coef_value(const float c[8], float w) {
+    float c0 = c[0], c1 = c[1], c3 = c[3], c6 = c[6];
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %4, %5" FQSL_Q1  // c0 + c2 y
+        "v_fmac_f32_dpp %1, %4, %6" FQSL_Q1  // c1 + c4 y
+        "v_fmac_f32_dpp %3, %4, %8" FQSL_Q1  // c6 + c7 y
+        "v_fmac_f32_dpp %2, %4, %7" FQSL_Q1  // c3 + c5 y
+        "v_fmac_f32_dpp %0, %4, %1" FQSL_Q0  // A
+        "v_fmac_f32_dpp %2, %4, %3" FQSL_Q0  // C
+        "v_fmac_f32_dpp %0, %4, %2" FQSL_Q2  // A + z C
+        : "+v"(c0), "+v"(c1), "+v"(c3), "+v"(c6) : "v"(w), "v"(c[2]), "v"(c[4]), "v"(c[5]), "v"(c[7]));
+    return c0;
+}
+
 // First of the axes a lane holds: its own of a quad (lane 3 repeats axis 0), 0
 // when it holds all.
 template <int K>
@@ -142,15 +175,22 @@ struct SideField<K, FieldSoA<T>> {
     }
 };
 
+// Index of the record at the cells the lanes hold.
+template <int K, class F>
+__device__ __forceinline__ unsigned record_index(const SideField<K, F>& f, const int* c) {
+    if constexpr (K == 1) return (unsigned)quad_sum(c[0] * f.stride[0]);
+    else return (unsigned)(c[0] * f.stride[0] + c[1] * f.stride[1] + c[2] * f.stride[2]);
+}
+
 // This lane's components of B at the cells and weights the lanes hold.
 template <int K, class F, typename R>
 __device__ __forceinline__ void side_value(const SideField<K, F>& f, const int* c, const R* w, R B[K]) {
-    int part[K], all[3];
     R k[K][8], x[3];
-#pragma unroll
-    for (int q = 0; q < K; ++q) part[q] = c[q] * f.stride[q];
-    all_axes<K>(part, all);
-    f.template load<R>((unsigned)(all[0] + all[1] + all[2]), k);
+    f.template load<R>(record_index<K, F>(f, c), k);
+    if constexpr (K == 1 && F::kCoef && sizeof(R) == 4) {
+        B[0] = quad_coef_value(k[0], w[0]);
+        return;
+    }
     all_axes<K>(w, x);
 #pragma unroll
     for (int q = 0; q < K; ++q) {
@@ -179,6 +219,25 @@ __device__ __forceinline__ void clamp_cell(int i, R r, int n, int& c, R& w) {
     c = max(min(i, n - 2), 0);
     w = clamp01(r + (R)(i - c)) + (r - r);
 }
+
+// The same for x = f + r with the whole part held as a float (exact below 2^24;
+// beyond, only its side of the box counts), top = n - 2: a NaN gives weight 0.
+__device__ __forceinline__ void clamp_cell_f(float f, float r, float top, int& c, float& w) {
+    const float cf = __builtin_amdgcn_fmed3f(f, 0.f, top);
+    c = (int)cf;
+    w = clamp01(r + (f - cf));
+}
+
+// a + b of two whole numbers held as floats, as an integer.  The conversion and
+// the sum saturate (to_int's limits lie in the same direction of the array), and
+// NaN gives 0: its weight is NaN in any cell.
+__device__ __forceinline__ int cvt_int(float v) {
+    int i;
+    asm("v_cvt_i32_f32_e32 %0, %1" : "=v"(i) : "v"(v));
+    return i;
+}
+__device__ __forceinline__ int sum_int(float a, float b) { return __builtin_elementwise_add_sat(cvt_int(a), cvt_int(b)); }
+__device__ __forceinline__ bool any_lane(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0ull; }
 
 // ------------------------------------------------------- positions
 // One coordinate: a compensated float pair, or a double.
@@ -228,7 +287,7 @@ struct SideGeom<K, UniformGrid, R> {
             const float fh = floorf(x.hi);
             const float u = (x.hi - fh) + (x.lo + d);
             const float fu = floorf(u);
-            clamp_cell<R>(to_int(fh) + to_int(fu), u - fu, na[q], c, w);
+            clamp_cell<R>(sum_int(fh, fu), u - fu, na[q], c, w);
         } else {
             const double v = x.x + d;
             const double f = floor(v);

@@ -4,16 +4,19 @@ The knobs (``_lib.TUNE_KNOBS``) change speed only -- a line's result does not
 depend on the lane, wave, queue or launch that traces it -- so they can be
 picked per workload by measurement:
 
-* ``scott_waves``  waves per SIMD the FP32c Scott stepping kernel is built for
-                   (3 = 168 VGPRs per lane, 2 = 256; 0 = the compiler's choice);
-* ``refill_min``   idle lanes a wavefront gathers before it claims new lines
-                   (the queue chunk: one atomic per chunk);
-* ``queues``       one seed queue, or one per XCD (8), the launch's blocks
-                   spread over them;
+* ``scott_waves``  waves per SIMD the FP32c Scott kernels with one line per lane
+                   (per-line schedule, batches) are built for (3 = 168 VGPRs per
+                   lane, 2 = 256; 0 = the compiler's choice);
+* ``refill_min``   idle lanes a wavefront of a persistent kernel with one line per
+                   lane (mixed, large FP64 launches, batches) gathers before it
+                   claims new lines (the queue chunk: one atomic per chunk);
+* ``queues``       one seed queue of such a kernel, or one per XCD (8), the
+                   launch's blocks spread over them;
 * ``grid_pct``     persistent grid size in % of one full occupancy wave;
 * ``order``        queue order: 2 = longest line first (by a coarse length
                    estimate), 0 = seed order, 1 = longest first only up to 64
-                   lines per persistent lane;
+                   lines per persistent lane, or from one to 16 per quad of
+                   lanes where lines are traced by quads;
 * ``order_buckets``length classes of that order (fewer keep more locality).
 
 ``autotune`` runs coordinate descent over these on the actual request, or on
