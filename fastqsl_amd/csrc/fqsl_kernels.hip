@@ -967,8 +967,9 @@ k_scott_persistent_w2(F f, ScottParams P, Seeds s, unsigned long long n, const R
 }
 
 // Persistent stepping with one line per quad of lanes (fqsl_quad_scott.h), the
-// first `width` quads of a wavefront each.  `src` tells a line's seed, step and
-// tolerance and is told when it is done.  Ended sides are landed, second sides
+// first `width` quads of a wavefront each.  `src` gives a quad its next line (the
+// seed and, where they differ, its field, method, step and tolerance) and is told
+// when the line is done.  Ended sides are landed, second sides
 // begun and free quads refilled together, once `refill_min` quads wait or none
 // is tracing; free quads take lines from the wavefront's own run, claimed a
 // share of the rest at a time (see trace_sides).
@@ -980,7 +981,7 @@ __device__ __forceinline__ void scott_quads_body(const F& f, Src src, unsigned l
     const int lane = __lane_id(), a = first_axis<1>();
     const bool writes = (lane & 3) != 3, first = (lane & 3) == 0;
     ScottParams P = src.params();
-    const QuadScott<R, F, FJ> T(f, P, a);
+    QuadScott<R, F, FJ> T(f, P, a);
     const SideField<1, FJ> J(fj, a);
     const unsigned long long kQuads = 0x1111111111111111ull;  // one lane of each
     const bool mine = (lane >> 2) < width;
@@ -1051,7 +1052,7 @@ __device__ __forceinline__ void scott_quads_body(const F& f, Src src, unsigned l
             if (next > end) next = end;
             if (L.pend == kSideIdle && mine && t < end) {
                 line = src.line(t);
-                L.p0 = src.seed(line, a, P);
+                L.p0 = src.take(line, a, P, T);
                 L.len = 0.0;
                 L.tw = 0.0;
                 L.steps = 0; L.attempts = 0; L.evals = 0;
@@ -1109,7 +1110,8 @@ struct ScottLines {
     __device__ __forceinline__ unsigned long long line(unsigned long long t) const {
         return order ? (unsigned long long)order[t] : t;
     }
-    __device__ __forceinline__ float seed(unsigned long long i, int a, ScottParams&) const {
+    template <class T>
+    __device__ __forceinline__ float take(unsigned long long i, int a, ScottParams&, T&) const {
         return a == 0 ? s.x[i] : (a == 1 ? s.y[i] : s.z[i]);
     }
     __device__ __forceinline__ void done(unsigned long long) const {}
@@ -2085,23 +2087,48 @@ extern "C" int fqsl_slog10q(uint64_t n, const float* q, const float* bn, const i
 
 // ----------------------------------------------------------------- batches
 // A batch of Scott requests, each with its own field, method, step,
-// tolerance, seeds and outputs.  Requests are grouped by (field, method); the
-// lines of a group form one contiguous range [base, base + n) of the batch's
-// line index and are drained by one persistent launch.  A line finds its
-// request by binary search over the requests' first-line offsets and takes
-// that request's step and tolerance, so one launch mixes requests of any
-// size.  All state lives in a workspace laid out at plan time, and a run only
-// launches kernels (the counters are cleared by a kernel), so a run can be
-// captured in a graph and replayed.
+// tolerance, seeds and outputs.  Requests are sorted by (layout of the field,
+// method, field), and the lines of consecutive requests form one contiguous
+// range of the batch's line index.  A line finds its request by binary search
+// over the requests' first-line offsets and takes that request's field, method,
+// step and tolerance.  Where lines are traced by quads of lanes, each quad holds
+// its own field's pointers and one launch traces all requests of a layout
+// (k_batch_quads); one line per lane, a launch per (field, method) keeps the
+// field in scalar registers (k_batch_step).  All state lives in a workspace laid
+// out at plan time, and a run only launches kernels (the counters are cleared by
+// a kernel), so a run can be captured in a graph and replayed.
+struct BatchField {
+    const void* p[3];  // cell records, or the three component arrays
+    int n[3], kind;
+};
+enum : int { kBatchCell32 = 0, kBatchSoA32 = 1, kBatchSoA64 = 2 };
+
 struct BatchReq {
     Seeds s;
     ScottOut o;
+    BatchField f;
     double step, tol;
     unsigned long long n;
+    int method;
+};
+
+template <class F>
+struct BatchFieldOf;
+template <>
+struct BatchFieldOf<FieldCell32> {
+    static __host__ __device__ __forceinline__ FieldCell32 get(const BatchField& b) {
+        return FieldCell32{(const float4*)b.p[0], {b.n[0], b.n[1], b.n[2]}};
+    }
+};
+template <typename T>
+struct BatchFieldOf<FieldSoA<T>> {
+    static __host__ __device__ __forceinline__ FieldSoA<T> get(const BatchField& b) {
+        return FieldSoA<T>{(const T*)b.p[0], (const T*)b.p[1], (const T*)b.p[2], {b.n[0], b.n[1], b.n[2]}};
+    }
 };
 
 struct BatchCtl {
-    unsigned long long* queues;     // one counter per group
+    unsigned long long* queues;     // one counter per launch
     unsigned long long* remaining;  // lines of each request not yet finished
     unsigned long long* stamps;     // [r]: device wall clock when request r's last line
                                     // finished stepping; [nreq]: start of the run
@@ -2142,12 +2169,13 @@ struct BatchGroupArgs {
 };
 
 template <typename R, class F>
-__global__ void __launch_bounds__(256) k_batch_prep(F f, BatchGroupArgs g, R* __restrict__ frames) {
+__global__ void __launch_bounds__(256) k_batch_prep(BatchGroupArgs g, R* __restrict__ frames) {
     for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < g.n;
          i += (unsigned long long)gridDim.x * blockDim.x) {
         const unsigned long long gi = g.base + i;
         const int r = batch_find(g.offs, g.r0, g.r1, gi);
         const unsigned long long li = gi - g.offs[r];
+        const F f = BatchFieldOf<F>::get(g.reqs[r].f);
         const Seeds s = g.reqs[r].s;
         const float p0[3] = {s.x[li], s.y[li], s.z[li]};
         R u0[3], v0[3], b0z;
@@ -2167,9 +2195,47 @@ __global__ void __launch_bounds__(256) k_batch_prep(F f, BatchGroupArgs g, R* __
     }
 }
 
+// Lines of a range of requests, for scott_quads_body.
+template <class F>
+struct BatchLines {
+    BatchGroupArgs g;
+    BatchCtl c;
+    __device__ __forceinline__ ScottParams params() const { return ScottParams{g.reqs[g.r0].method, 0.0, 0.0, 0.0}; }
+    __device__ __forceinline__ unsigned long long line(unsigned long long t) const { return g.base + t; }
+    template <class T>
+    __device__ __forceinline__ float take(unsigned long long i, int a, ScottParams& P, T& tracer) const {
+        const int r = batch_find(g.offs, g.r0, g.r1, i);
+        const BatchReq& q = g.reqs[r];
+        const unsigned long long li = i - g.offs[r];
+        P.method = q.method;
+        P.s0 = q.step;
+        P.tol = q.tol;
+        P.ctl = scott_ctl(P.tol);
+        tracer.set_field(BatchFieldOf<F>::get(q.f), a);
+        return a == 0 ? q.s.x[li] : (a == 1 ? q.s.y[li] : q.s.z[li]);
+    }
+    __device__ __forceinline__ void done(unsigned long long i) const {
+        batch_line_done(c, batch_find(g.offs, g.r0, g.r1, i));
+    }
+};
+
+// All requests of a layout, whatever their fields and methods, in one launch with
+// a single tail: a launch per (field, method) ended six times with a few long
+// lines in an empty chip, and its lanes were held back by their cell loads (see
+// k_scott_quads).  12 requests of 64^2 to 700^2 lines over three fields: 19
+// launches, 50.6 ms -> 4 launches, 42.5 ms; bound by vector instruction issue.
+template <typename R, class F>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1)))
+k_batch_quads(BatchGroupArgs g, const R* frames, ScottRec<R>* recs, BatchCtl c, int qi, int spread, int refill_min) {
+    const unsigned long long share = (g.n + (unsigned)spread - 1) / (unsigned)spread;
+    const int width = share > 16ull ? 16 : (share < 1ull ? 1 : (int)share);
+    scott_quads_body<R, F, NoCurrent>(BatchFieldOf<F>::get(g.reqs[g.r0].f), BatchLines<F>{g, c}, g.n, frames, recs,
+                                      c.queues + qi, width, refill_min < width ? refill_min : width, NoCurrent{});
+}
+
 // Persistent stepping over one group: as scott_persistent_body, with the
 // step and tolerance of each lane's request.
-template <typename R, class F, typename X, bool kRoll = false>
+template <typename R, class F, typename X>
 __device__ __forceinline__ void scott_batch_body(F f, int method, BatchGroupArgs g, const R* __restrict__ frames,
                                                  ScottRec<R>* __restrict__ recs, BatchCtl c, int qi,
                                                  int refill_min) {
@@ -2217,7 +2283,7 @@ __device__ __forceinline__ void scott_batch_body(F f, int method, BatchGroupArgs
         }
         if (active) {
             ScottEnd<R> e;
-            const int st = scott_attempt<R, F, NoCurrent, X, kRoll>(L, f, P, e);
+            const int st = scott_attempt<R, F, NoCurrent, X>(L, f, P, e);
             if (st != kTracing) {
                 recs[idx] = ScottRec<R>{L.st, e, L.len, st, L.evals, L.tw};
                 active = false;
@@ -2240,21 +2306,15 @@ k_batch_step_w2(F f, int method, BatchGroupArgs g, const R* frames, ScottRec<R>*
     scott_batch_body<R, F, X>(f, method, g, frames, recs, c, qi, refill_min);
 }
 
-template <typename R, class F, typename X>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
-k_batch_step_w3(F f, int method, BatchGroupArgs g, const R* frames, ScottRec<R>* recs, BatchCtl c, int qi,
-                int refill_min) {
-    scott_batch_body<R, F, X, true>(f, method, g, frames, recs, c, qi, refill_min);
-}
-
 template <typename R, class F>
-__global__ void __launch_bounds__(256) k_batch_finish(F f, BatchGroupArgs g, const R* __restrict__ frames,
+__global__ void __launch_bounds__(256) k_batch_finish(BatchGroupArgs g, const R* __restrict__ frames,
                                                       const ScottRec<R>* __restrict__ recs) {
     for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < g.n;
          i += (unsigned long long)gridDim.x * blockDim.x) {
         const unsigned long long gi = g.base + i;
         const int r = batch_find(g.offs, g.r0, g.r1, gi);
         const unsigned long long li = gi - g.offs[r];
+        const F f = BatchFieldOf<F>::get(g.reqs[r].f);
         const ScottOut o = g.reqs[r].o;
         const ScottRec<R> rec = recs[gi];
         double q0, qp;
@@ -2272,8 +2332,10 @@ __global__ void __launch_bounds__(256) k_batch_finish(F f, BatchGroupArgs g, con
     }
 }
 
+// Consecutive requests of the batch order and their lines: of one layout, or of
+// one field and method.
 struct BatchGroup {
-    const fqsl_field* field;
+    BatchField f;
     int method;
     int r0, r1;
     unsigned long long base, n;
@@ -2284,8 +2346,8 @@ struct fqsl_scott_batch {
     int precision;
     int nreq;
     int refill_min;
-    int waves;
-    std::vector<BatchGroup> groups;
+    std::vector<BatchGroup> layouts;  // by layout
+    std::vector<BatchGroup> groups;   // by field and method
     std::vector<int> order;  // batch position -> caller's request index
     char* ws;                // caller's workspace
     BatchReq* reqs;
@@ -2340,33 +2402,82 @@ int check_request(const fqsl_scott_request& q, int precision, int k) {
     return FQSL_OK;
 }
 
-// Requests in batch order: grouped by (field, method), stable within a group.
+// The layout a request is traced on.
+BatchField batch_field(const fqsl_scott_request& q, int precision) {
+    const fqsl_field* f = q.field;
+    BatchField b{{nullptr, nullptr, nullptr}, {f->n[0], f->n[1], f->n[2]}, kBatchCell32};
+    if (precision != FQSL_PREC_FP64 && f->cell32) {
+        b.p[0] = f->cell32;
+        return b;
+    }
+    b.kind = precision == FQSL_PREC_FP64 ? kBatchSoA64 : kBatchSoA32;
+    for (int a = 0; a < 3; ++a)
+        b.p[a] = precision == FQSL_PREC_FP64 ? (const void*)f->soa64[a] : (const void*)f->soa32[a];
+    return b;
+}
+
+// Requests in batch order: by layout, then RK4 first (a fixed step takes several
+// times the evaluations of an adaptive one, and the longest lines are better
+// begun early), then by field; stable within these.
 std::vector<int> batch_order(const fqsl_scott_request* reqs, int nreq) {
     std::vector<int> ord(nreq);
     for (int k = 0; k < nreq; ++k) ord[k] = k;
     std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) {
-        if (reqs[a].field != reqs[b].field) return reqs[a].field < reqs[b].field;
-        return reqs[a].method < reqs[b].method;
+        const fqsl_scott_request &p = reqs[a], &q = reqs[b];
+        const bool pc = p.field->cell32 != nullptr, qc = q.field->cell32 != nullptr;
+        if (pc != qc) return pc;
+        if (p.method != q.method) return p.method == FQSL_METHOD_RK4;
+        return std::less<const fqsl_field*>()(p.field, q.field);
     });
     return ord;
 }
 
-template <typename R, class F, typename X = R>
-int batch_launch_group(const fqsl_scott_batch* b, const BatchGroup& G, int gi, const F& f, hipStream_t st) {
-    BatchGroupArgs g{b->reqs, b->offs, G.r0, G.r1, G.base, G.n};
-    R* frames = (R*)b->frames;
-    ScottRec<R>* recs = (ScottRec<R>*)b->recs;
-    const int knob = sizeof(R) != 4 ? 0 : (sizeof(X) == 8 ? 2 : b->waves);
-    const int waves = (knob == 3 && G.n <= small_launch_lines()) ? 2 : knob;
-    auto kern = waves == 2 ? k_batch_step_w2<R, F, X> : waves == 3 ? k_batch_step_w3<R, F, X> : k_batch_step<R, F, X>;
+template <typename R, class F, typename X>
+int batch_step_groups(const fqsl_scott_batch* b, const BatchGroup& S, hipStream_t st) {
+    auto kern = std::is_same<R, X>::value ? k_batch_step<R, F, X> : k_batch_step_w2<R, F, X>;
     int grid = 0;
     int rc = persistent_grid(kern, &grid);
     if (rc) return rc;
     grid = (int)((long)grid * g_tune[FQSL_TUNE_GRID_PCT] / 100);
     if (grid < 1) grid = 1;
-    k_batch_prep<R, F><<<grid_for((long)G.n, 256), 256, 0, st>>>(f, g, frames);
-    kern<<<grid, 256, 0, st>>>(f, G.method, g, frames, recs, b->ctl, gi, b->refill_min);
-    k_batch_finish<R, F><<<grid_for((long)G.n, 256), 256, 0, st>>>(f, g, frames, recs);
+    for (size_t gi = 0; gi < b->groups.size(); ++gi) {
+        const BatchGroup& G = b->groups[gi];
+        if (G.n == 0 || G.r0 < S.r0 || G.r0 >= S.r1) continue;
+        kern<<<grid, 256, 0, st>>>(BatchFieldOf<F>::get(G.f), G.method,
+                                   BatchGroupArgs{b->reqs, b->offs, G.r0, G.r1, G.base, G.n}, (const R*)b->frames,
+                                   (ScottRec<R>*)b->recs, b->ctl, (int)gi, b->refill_min);
+    }
+    return FQSL_OK;
+}
+
+// The requests of one layout: by quads where a trace of as many lines goes by
+// quads (scott_stepping), in one launch.
+template <typename R, class F, typename X = R>
+int batch_launch(const fqsl_scott_batch* b, const BatchGroup& S, int qi, hipStream_t st) {
+    const BatchGroupArgs g{b->reqs, b->offs, S.r0, S.r1, S.base, S.n};
+    R* frames = (R*)b->frames;
+    ScottRec<R>* recs = (ScottRec<R>*)b->recs;
+    k_batch_prep<R, F><<<grid_for((long)S.n, 256), 256, 0, st>>>(g, frames);
+    int rc = FQSL_OK;
+    bool quads = false;
+    if constexpr (std::is_same<R, X>::value) {
+        quads = sizeof(R) == 4 || S.n <= kScottQuadLinesFp64;
+        if (quads) {
+            int full = 0;
+            rc = persistent_grid(k_batch_quads<R, F>, &full);
+            if (rc) return rc;
+            full = (int)((long)full * g_tune[FQSL_TUNE_GRID_PCT] / 100);
+            if (full < 1) full = 1;
+            const unsigned long long wanted = (S.n + 3) / 4;  // one line per wavefront at the least
+            const int grid = wanted < (unsigned long long)full ? (int)wanted : full;
+            const int waves = std::min(full, cu_count() * kScottSpread) * 4;
+            k_batch_quads<R, F><<<grid, 256, 0, st>>>(g, frames, recs, b->ctl, qi, waves,
+                                                      sizeof(R) == 4 ? kScottQuadRefillFp32 : kScottQuadRefillFp64);
+        }
+    }
+    if (!quads) rc = batch_step_groups<R, F, X>(b, S, st);
+    if (rc) return rc;
+    k_batch_finish<R, F><<<grid_for((long)S.n, 256), 256, 0, st>>>(g, frames, recs);
     HIP_TRY(hipGetLastError());
     return FQSL_OK;
 }
@@ -2404,25 +2515,28 @@ extern "C" int fqsl_scott_batch_create(const fqsl_scott_request* reqs, int nreq,
     b->precision = precision;
     b->nreq = nreq;
     b->refill_min = g_tune[FQSL_TUNE_REFILL_MIN];
-    b->waves = g_tune[FQSL_TUNE_SCOTT_WAVES];
     b->order = batch_order(reqs, nreq);
     std::vector<BatchReq> table(nreq);
     std::vector<unsigned long long> offs(nreq);
     unsigned long long lines = 0;
     for (int k = 0; k < nreq; ++k) {
         const fqsl_scott_request& q = reqs[b->order[k]];
-        if (k == 0 || q.field != b->groups.back().field || q.method != b->groups.back().method)
-            b->groups.push_back(BatchGroup{q.field, q.method, k, k, lines, 0});
-        BatchGroup& G = b->groups.back();
-        G.r1 = k + 1;
-        G.n += q.n;
+        const BatchField f = batch_field(q, precision);
+        const bool layout = k == 0 || f.kind != b->layouts.back().f.kind;
+        if (layout) b->layouts.push_back(BatchGroup{f, q.method, k, k, lines, 0});
+        if (layout || q.field != reqs[b->order[k - 1]].field || q.method != b->groups.back().method)
+            b->groups.push_back(BatchGroup{f, q.method, k, k, lines, 0});
+        for (BatchGroup* G : {&b->layouts.back(), &b->groups.back()}) {
+            G->r1 = k + 1;
+            G->n += q.n;
+        }
         offs[k] = lines;
         const fqsl_scott_out& o = q.out;
         table[k] = BatchReq{Seeds{q.x, q.y, q.z},
                             ScottOut{o.start_x, o.start_y, o.start_z, o.end_x, o.end_y, o.end_z, o.flag_start,
                                      o.flag_end, o.b_this_x, o.b_this_y, o.b_this_z, o.q_0, o.q_perp, o.line_len,
                                      o.evals, nullptr},
-                            q.step, q.method == FQSL_METHOD_RKF45 ? q.tol : 0.0, q.n};
+                            f, q.step, q.method == FQSL_METHOD_RKF45 ? q.tol : 0.0, q.n, q.method};
         lines += q.n;
     }
     const BatchLayout L = batch_layout(nreq, (int)b->groups.size(), lines, precision);
@@ -2461,23 +2575,18 @@ extern "C" int fqsl_scott_batch_run(const fqsl_scott_batch* b, void* stream) {
     k_batch_reset<<<grid_for((long)(b->nreq + 1 > ng ? b->nreq + 1 : ng), 256), 256, 0, st>>>(b->ctl, b->reqs, b->nreq,
                                                                                              ng);
     HIP_TRY(hipGetLastError());
-    for (int gi = 0; gi < ng; ++gi) {
-        const BatchGroup& G = b->groups[gi];
-        if (G.n == 0) continue;
-        const fqsl_field* fd = G.field;
+    const bool mixed = b->precision == FQSL_PREC_MIXED;
+    for (size_t k = 0; k < b->layouts.size(); ++k) {
+        const BatchGroup& S = b->layouts[k];
+        if (S.n == 0) continue;
+        const int qi = (int)k;
         int rc;
-        if (b->precision == FQSL_PREC_FP64) {
-            FieldSoA<double> f{fd->soa64[0], fd->soa64[1], fd->soa64[2], {fd->n[0], fd->n[1], fd->n[2]}};
-            rc = batch_launch_group<double>(b, G, gi, f, st);
-        } else if (fd->cell32) {
-            FieldCell32 f{fd->cell32, {fd->n[0], fd->n[1], fd->n[2]}};
-            rc = b->precision == FQSL_PREC_MIXED ? batch_launch_group<float, FieldCell32, double>(b, G, gi, f, st)
-                                                 : batch_launch_group<float>(b, G, gi, f, st);
-        } else {
-            FieldSoA<float> f{fd->soa32[0], fd->soa32[1], fd->soa32[2], {fd->n[0], fd->n[1], fd->n[2]}};
-            rc = b->precision == FQSL_PREC_MIXED ? batch_launch_group<float, FieldSoA<float>, double>(b, G, gi, f, st)
-                                                 : batch_launch_group<float>(b, G, gi, f, st);
-        }
+        if (S.f.kind == kBatchSoA64) rc = batch_launch<double, FieldSoA<double>>(b, S, qi, st);
+        else if (S.f.kind == kBatchCell32)
+            rc = mixed ? batch_launch<float, FieldCell32, double>(b, S, qi, st) : batch_launch<float, FieldCell32>(b, S, qi, st);
+        else
+            rc = mixed ? batch_launch<float, FieldSoA<float>, double>(b, S, qi, st)
+                       : batch_launch<float, FieldSoA<float>>(b, S, qi, st);
         if (rc) return rc;
     }
     if (timed) return record_end(st);

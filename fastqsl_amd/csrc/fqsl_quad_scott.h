@@ -147,9 +147,16 @@ struct QuadScott {
     float top;  // the last cell of the lane's axis
     const ScottParams& P;
 
-    __device__ __forceinline__ QuadScott(const F& ff, const ScottParams& p, int a)
-        : f(ff, a), na(axis_of(ff.n[0], ff.n[1], ff.n[2], a)), len_lim(scott_len_lim(ff)), P(p) {
+    __device__ __forceinline__ QuadScott(const F& ff, const ScottParams& p, int a) : f(ff, a), P(p) { set_box(ff, a); }
+    // another field, for this lane's quad (lines of several fields in one launch)
+    __device__ __forceinline__ void set_field(const F& ff, int a) {
+        f = SideField<1, F>(ff, a);
+        set_box(ff, a);
+    }
+    __device__ __forceinline__ void set_box(const F& ff, int a) {
+        na = axis_of(ff.n[0], ff.n[1], ff.n[2], a);
         top = (float)(na - 2);
+        len_lim = scott_len_lim(ff);
         n[0] = ff.n[0]; n[1] = ff.n[1]; n[2] = ff.n[2];
     }
 
