@@ -1430,7 +1430,9 @@ k_plain_quads(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, Dev
 // Many RKF45 sides: the listed tangent lines, whose long chains set the time,
 // go first, by quads, in the first `tangent_blocks` workgroups (one a CU: more
 // wavefronts would slow each other's chains, fewer start them late); a
-// wavefront that has none left goes on to all others, one side per lane.  On the
+// wavefront that has none left goes on to all others, one side per lane.  Few of
+// them are spread over all of these wavefronts, as in k_plain_quads (the pseudo
+// lines of a 233 x 191 map, 1,000 in arrays of 178,000: 2.08 -> 1.50 ms).  On the
 // 1024^2 neighbour map (multipole 256^3; longest line 5,048 evaluations, mean
 // 103) 5.3 -> 1.8 ms, on the stretched 256^3 map 12.5 -> 5.0 ms; all sides by
 // quads take 2.4 and 5.9 ms, all by lanes 2.7 ms on the first.
@@ -1441,8 +1443,12 @@ k_plain_sides(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, Dev
     apply_plain_scalars(f, P, n, ds, ncross);
     fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];
     grid_prologue(g);
-    if (tl.list && blockIdx.x < (unsigned)tangent_blocks)
-        trace_sides<1, R, F, FJ, G>(f, P, s, *tl.count, o, queue, 16, 4, tl.list, nullptr, fj, g);
+    if (tl.list && blockIdx.x < (unsigned)tangent_blocks) {
+        const unsigned long long m = *tl.count, waves = 4ull * (unsigned)tangent_blocks;
+        const unsigned long long share = (2ull * m + waves - 1) / waves;
+        const int width = share > 16ull ? 16 : (share < 1ull ? 1 : (int)share);
+        trace_sides<1, R, F, FJ, G>(f, P, s, m, o, queue, width, 4 < width ? 4 : width, tl.list, nullptr, fj, g);
+    }
     trace_sides<3, R, F, FJ, G>(f, P, s, n, o, queue + 1, 64, refill_min, nullptr,
                                        tl.list ? tl.marked : nullptr, fj, g);
 }
