@@ -144,6 +144,23 @@ __global__ void __launch_bounds__(256) k_build_cells(const T* __restrict__ bx, c
     }
 }
 
+// Pairs (FieldPairs) of the float field.  Bound by memory: 12 bytes read and 32
+// written a node, 256^3 nodes 0.2 ms.
+__global__ void __launch_bounds__(256) k_build_pairs(const float* __restrict__ bx, const float* __restrict__ by,
+                                                     const float* __restrict__ bz, unsigned nodes,
+                                                     float4* __restrict__ pairs) {
+    const float* comp[3] = {bx, by, bz};
+    for (unsigned long long i = blockIdx.x * 256ull + threadIdx.x; i < nodes; i += gridDim.x * 256ull) {
+        // the pair past a row's end (and the array's) is in no cell
+        const unsigned long long j = i + 1 < nodes ? i + 1 : i;
+        float v[3], w[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) { v[q] = comp[q][i]; w[q] = comp[q][j]; }
+        pairs[2 * i] = make_float4(v[0], w[0], v[1], w[1]);
+        pairs[2 * i + 1] = make_float4(v[2], w[2], 0.f, 0.f);
+    }
+}
+
 static int grid_for(long n, int block) {
     long g = (n + block - 1) / block;
     if (g > 65535L * 16) g = 65535L * 16;
@@ -220,8 +237,9 @@ static hipError_t field_malloc(int device, T** out, size_t bytes) {
     return hipSuccess;
 }
 
-// As hipFree, which waits for the device before the memory can be used again.
-static void field_release(int device, void* p) {
+// As hipFree, which waits for the device before the memory can be used again;
+// `done`: the work that used it is known to have ended.
+static void field_release(int device, void* p, bool done = false) {
     if (!p) return;
     size_t bytes = 0;
     {
@@ -238,7 +256,7 @@ static void field_release(int device, void* p) {
         (void)hipFree(p);
         return;
     }
-    const hipError_t e = hipDeviceSynchronize();
+    const hipError_t e = done ? hipSuccess : hipDeviceSynchronize();
     if (cur != device) (void)hipSetDevice(cur);
     if (e != hipSuccess) {
         (void)hipFree(p);
@@ -1600,9 +1618,9 @@ static int scott_stepping(ScottStepping<R, F, FJ, X>* st, unsigned long long n) 
 // 11.7 / 14.0; 2048^2 32.0 / 32.1, cube of 8.4 M lines 207 / 193; 64 lines
 // 0.83 / 0.78).  Lanes: up to 64 lines each.
 template <typename R, class F, class FJ, typename X>
-static bool scott_ordered(const DevScalars& ds, unsigned long long n_hint, const ScottStepping<R, F, FJ, X>& st) {
+static bool scott_ordered(const DevScalars& ds, const F& f, unsigned long long n_hint, const ScottStepping<R, F, FJ, X>& st) {
     const int om = g_tune[FQSL_TUNE_ORDER];
-    return !ds.shape && n_hint < (1ull << 32) &&
+    return (!ds.shape || f.n[0] > 0) && n_hint < (1ull << 32) &&
            (om == 2 || (om == 1 && (st.kern ? n_hint <= 64ull * st.lines
                                             : n_hint > st.lines && n_hint <= 16ull * st.lines)));
 }
@@ -1610,12 +1628,14 @@ static bool scott_ordered(const DevScalars& ds, unsigned long long n_hint, const
 // The persistent schedule's launches on `st` over a workspace `ws` laid out
 // by scott_ws_layout and the queue counters `q` (kQueueSlotWidth words).
 // `timed` records the trace and stepping-kernel events of this thread.
+// `pairs`: the field's node pairs, which the quads then read in place of F.
 template <typename R, class F, class FJ, typename X>
 static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, const Seeds& s, unsigned long long n,
                                             const ScottOut& o, const DevScalars& ds, hipStream_t st,
                                             unsigned long long n_hint, const FJ& fj, char* ws, const ScottWs& w,
                                             bool ordered, unsigned long long* q,
-                                            const ScottStepping<R, F, FJ, X>& step, bool timed) {
+                                            const ScottStepping<R, F, FJ, X>& step, bool timed,
+                                            const float2* pairs = nullptr) {
     R* frames = (R*)(ws + w.frames);
     ScottRec<R>* recs = (ScottRec<R>*)(ws + w.recs);
     unsigned* order = ordered ? (unsigned*)(ws + w.order) : nullptr;
@@ -1642,9 +1662,17 @@ static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, co
             const unsigned long long wanted = (n_hint + 3) / 4;  // one line per wavefront at the least
             const int grid = wanted < (unsigned long long)step.grid ? (int)wanted : step.grid;
             const int waves = std::min(step.grid, cu_count() * kScottSpread) * 4;
-            k_scott_quads<R, F, FJ><<<grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, waves,
-                                                          sizeof(R) == 4 ? kScottQuadRefillFp32 : kScottQuadRefillFp64,
-                                                          order, fj);
+            const int refill = sizeof(R) == 4 ? kScottQuadRefillFp32 : kScottQuadRefillFp64;
+            bool done = false;
+            if constexpr (std::is_same<F, FieldSoA<float>>::value) {
+                if (pairs) {
+                    k_scott_quads<R, FieldPairs, FJ><<<grid, 256, 0, st>>>(
+                        FieldPairs{pairs, {f.n[0], f.n[1], f.n[2]}}, P, s, n, frames, recs, ds, q, waves, refill, order, fj);
+                    done = true;
+                }
+            }
+            if (!done)
+                k_scott_quads<R, F, FJ><<<grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, waves, refill, order, fj);
         }
     }
     if (step.kern) step.kern<<<step.grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, nq, refill_min, order, fj);
@@ -1676,14 +1704,14 @@ static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 template <typename R, class F, class FJ = NoCurrent, typename X = R>
 static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsigned long long n, const ScottOut& o,
                         const DevScalars& ds, int schedule, hipStream_t st, unsigned long long n_hint,
-                        char* noalloc, const FJ& fj = FJ{}) {
+                        char* noalloc, const FJ& fj = FJ{}, const float2* pairs = nullptr) {
     if (schedule == FQSL_SCHED_PERSISTENT) {
         // n_hint: number of lines, known on the host (sizes the workspace)
         if (n_hint == 0) return FQSL_OK;
         ScottStepping<R, F, FJ, X> step;
         int rc = scott_stepping<R, F, FJ, X>(&step, n_hint);
         if (rc) return rc;
-        const bool ordered = scott_ordered(ds, n_hint, step);
+        const bool ordered = scott_ordered<R, F, FJ, X>(ds, f, n_hint, step);
         const ScottWs w = scott_ws_layout<R>(n_hint, ordered);
         if (noalloc) {  // device address of this device's scratch array: no allocation, no events
             if (w.bytes > kNoAllocScratchBytes - kNoAllocQueueBytes)
@@ -1703,7 +1731,7 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
         void* ws = nullptr;
         HIP_TRY(hipMallocAsync(&ws, w.bytes, st));
         const hipError_t e = scott_persistent_launches<R, F, FJ, X>(f, P, s, n, o, ds, st, n_hint, fj, (char*)ws,
-                                                                    w, ordered, q, step, true);
+                                                                    w, ordered, q, step, true, pairs);
         const hipError_t ef = hipFreeAsync(ws, st);
         if (e != hipSuccess) return set_err(FQSL_ERR_HIP, "Scott trace launch: %s", hipGetErrorString(e));
         if (ef != hipSuccess) return set_err(FQSL_ERR_HIP, "hipFreeAsync: %s", hipGetErrorString(ef));
@@ -3079,6 +3107,20 @@ extern "C" int fqsl_trace_plain_n(const fqsl_field* field, const fqsl_plain_para
 // 256 is only the cap passed as the line-count hint.
 static constexpr int kPerLineMaxBlocks = 65536;
 
+// Whether the Scott entry pairs the nodes of the in-place field first.  Quads
+// reading three component arrays touch twelve cache lines an evaluation, most of
+// them missing L1 (vector instructions took 0.2 of the issue slots); four with
+// pairs.  Whole calls, in place / by pairs: 256^3 nodes, 147 k lines 5.1 / 2.3 ms,
+// 66 k 2.6 / 1.75, 128^3 147 k 2.8 / 1.5, 9 k 1.02 / 0.97, 64^3 147 k 2.0 / 1.3;
+// with fewer lines than a 512th of the nodes (256^3, 26 k: 1.4) the pairing is
+// not earned back.  Fields below the size whose memory is kept stay in place, and
+// those above 2^27 nodes (4 GiB of pairs, half of what is kept).
+static bool dropin_by_pairs(const int* n, unsigned long long lines) {
+    if (n[0] < 2 || n[1] < 2 || n[2] < 2) return false;
+    const double nodes = (double)n[0] * n[1] * n[2];
+    return nodes >= (double)(kFieldCacheMin / 32) && nodes <= (double)(1 << 27) && (double)lines * 512.0 >= nodes;
+}
+
 extern "C" int fqsl_TraceAllBlineScott(float* Bx, float* By, float* Bz, int* BshapeN, float* curB_x, float* curB_y,
                                        float* curB_z, double* twist, bool* curB_flag, float* inp_x, float* inp_y,
                                        float* inp_z, float* inp_cross_dir, float* start_x, float* start_y,
@@ -3106,24 +3148,45 @@ extern "C" int fqsl_TraceAllBlineScott(float* Bx, float* By, float* Bz, int* Bsh
                q_0, q_perp, LineLen, nullptr, twist_on ? twist : nullptr};
     DevScalars ds{BshapeN, s_len, N, tol_coef, curB_flag, twist};
     FieldSoA<float> f{Bx, By, Bz, {2, 2, 2}};
-    unsigned long long n_hint = (unsigned long long)kPerLineMaxBlocks * 256;
+    unsigned long long n_hint = (unsigned long long)kPerLineMaxBlocks * 256, n = 0;
+    const hipStream_t st = (hipStream_t)stream;
+    bool by_pairs = false;
     if (schedule == FQSL_SCHED_PERSISTENT) {
         // the persistent path sizes its workspace from N: read it (synchronises the stream)
-        HIP_TRY(hipMemcpyAsync(&n_hint, N, sizeof(n_hint), hipMemcpyDeviceToHost, (hipStream_t)stream));
-        HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+        int shape[3] = {0, 0, 0};
+        HIP_TRY(hipMemcpyAsync(&n_hint, N, sizeof(n_hint), hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipMemcpyAsync(shape, BshapeN, sizeof(shape), hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipStreamSynchronize(st));
+        n = n_hint;
+        for (int q = 0; q < 3; ++q) f.n[q] = shape[q];
+        by_pairs = precision == FQSL_PREC_FP32C && dropin_by_pairs(f.n, n);
     }
-    const hipStream_t st = (hipStream_t)stream;
+    int dev = 0;
+    float2* pairs = nullptr;
+    if (by_pairs && hipGetDevice(&dev) == hipSuccess) {
+        const unsigned nodes = (unsigned)f.n[0] * (unsigned)f.n[1] * (unsigned)f.n[2];
+        if (field_malloc(dev, &pairs, 32ull * nodes) == hipSuccess)
+            k_build_pairs<<<grid_for((long)nodes, 256), 256, 0, st>>>(Bx, By, Bz, nodes, (float4*)pairs);
+        else
+            (void)hipGetLastError();  // no room: the field is read in place
+    }
     if (twist_on) {
         const FieldSoA<float> fj{curB_x, curB_y, curB_z, {2, 2, 2}};  // shape taken from B's on the device
-        if (precision == FQSL_PREC_MIXED)
-            return launch_scott<float, FieldSoA<float>, FieldSoA<float>, double>(f, P, s, 0ull, o, ds, schedule, st,
-                                                                                 n_hint, nullptr, fj);
-        return launch_scott<float>(f, P, s, 0ull, o, ds, schedule, st, n_hint, nullptr, fj);
+        rc = precision == FQSL_PREC_MIXED
+                 ? launch_scott<float, FieldSoA<float>, FieldSoA<float>, double>(f, P, s, n, o, ds, schedule, st, n_hint,
+                                                                                 nullptr, fj)
+                 : launch_scott<float>(f, P, s, n, o, ds, schedule, st, n_hint, nullptr, fj, pairs);
+    } else {
+        rc = precision == FQSL_PREC_MIXED
+                 ? launch_scott<float, FieldSoA<float>, NoCurrent, double>(f, P, s, n, o, ds, schedule, st, n_hint, nullptr)
+                 : launch_scott<float>(f, P, s, n, o, ds, schedule, st, n_hint, nullptr, NoCurrent{}, pairs);
     }
-    if (precision == FQSL_PREC_MIXED)
-        return launch_scott<float, FieldSoA<float>, NoCurrent, double>(f, P, s, 0ull, o, ds, schedule, st, n_hint,
-                                                                       nullptr);
-    return launch_scott<float>(f, P, s, 0ull, o, ds, schedule, st, n_hint, nullptr);
+    if (pairs) {  // other streams may take the block once this one is done with it
+        const hipError_t e = hipStreamSynchronize(st);
+        field_release(dev, pairs, e == hipSuccess);
+        if (rc == FQSL_OK && e != hipSuccess) return set_err(FQSL_ERR_HIP, "Scott trace: %s", hipGetErrorString(e));
+    }
+    return rc;
 }
 
 extern "C" int fqsl_TraceAllBline(int method, float* Bx, float* By, float* Bz, int* BshapeN, float* curB_x,

@@ -175,6 +175,26 @@ struct SideField<K, FieldSoA<T>> {
     }
 };
 
+template <>
+struct SideField<1, FieldPairs> {
+    const FQSL_GLOBAL float2* base;
+    int stride[1], nx, nxy;
+    __device__ __forceinline__ SideField(const FieldPairs& f, int a)
+        : base((const FQSL_GLOBAL float2*)f.pairs + a), nx(f.n[0]), nxy(f.n[0] * f.n[1]) {
+        stride[0] = axis_of(1, nx, nxy, a);
+    }
+    template <typename R>
+    __device__ __forceinline__ void load(unsigned node, R c[1][8]) const {
+        const FQSL_GLOBAL float2* p = base + 4 * (unsigned long long)node;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float2 v = p[4 * ((k & 1) * (long)nx + (k >> 1) * (long)nxy)];
+            c[0][2 * k] = (R)v.x;
+            c[0][2 * k + 1] = (R)v.y;
+        }
+    }
+};
+
 // Index of the record at the cells the lanes hold.
 template <int K, class F>
 __device__ __forceinline__ unsigned record_index(const SideField<K, F>& f, const int* c) {

@@ -160,6 +160,15 @@ struct FieldSoA {
     }
 };
 
+// Pairs of nodes adjacent in x, the components of a pair together: record (i, j, k)
+// is [Bx(i) Bx(i+1)] [By ..] [Bz ..] [pad], 32 bytes.  The values of FieldSoA from
+// four cache lines a cell instead of twelve, and twice its memory.
+struct FieldPairs {
+    static constexpr bool kCoef = false;
+    const float2* pairs;
+    int n[3];
+};
+
 // Trilinear coefficients of one cell from its corners v[a + 2b + 4c]:
 //   B(x, y, z) = c0 + c1 x + c2 y + c3 z + c4 xy + c5 yz + c6 xz + c7 xyz
 // for (x, y, z) in [0, 1]^3, formed in double and rounded once.

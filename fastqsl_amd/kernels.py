@@ -63,6 +63,9 @@ SCOTT_PARAMS = _COMMON_HEAD + [
     ("s_len", _F32, False), ("N", _U64, False), ("LineLen", _F64, True), ("tol_coef", _F32, False)]
 
 
+_UNUSED = object()  # an argument the library does not read in this call
+
+
 class _Binding:
     """Holds device views of the call's arrays and copies host outputs back."""
 
@@ -73,6 +76,9 @@ class _Binding:
         self.copy_back = []
         self.keep = []
         for (name, dt, is_out), a in zip(params, args):
+            if a is _UNUSED:
+                self.ptrs.append(None)
+                continue
             if isinstance(a, torch.Tensor):
                 if not a.is_cuda:
                     raise ValueError(f"{name}: CPU tensors are not accepted; pass a CUDA tensor or NumPy array")
@@ -128,8 +134,7 @@ class _Kernel:
         if not flag_val:
             # twist off: the notebooks pass float32 dummies for curB and twist,
             # which the library never reads
-            twist_i = self._twist_i
-            args = args[:twist_i] + (np.zeros(1, np.float64),) + args[twist_i + 1:]
+            args = args[:self._twist_i] + (_UNUSED,) + args[self._twist_i + 1:]
         b = _Binding(self.params, args)
         st = stream if stream is not None else torch.cuda.current_stream()
         L = _lib.lib()
@@ -142,7 +147,10 @@ class _Kernel:
         else:
             rc = L.fqsl_TraceAllBline(self.method, *b.ptrs, prec, sched, ctypes.c_void_p(st.cuda_stream))
         _lib.check(rc)
-        if b.copy_back:
+        # host arrays: results are copied back and no copy outlives its use; another
+        # stream than torch's: the caller's tensors may be freed after the call.
+        # Otherwise nothing waits here, as with a launch of the reference's kernel.
+        if b.keep or stream is not None:
             b.finish(st)
         self._last = b  # device copies stay alive until the next call
 
