@@ -205,6 +205,59 @@ struct QuadScott {
         return D * t1 - S * t2;
     }
 
+    // Rows of the axes whose +-h samples leave the cell, every place being inside
+    // the box: axis_setup_sel's values without its places beyond the faces (at
+    // x = 0 its lower sample is clamped to weight 0, as r = 0 gives).
+    __device__ __forceinline__ void near_plane(unsigned cell, int i, R r, R w, R B, const R d[3], R J[3]) const {
+        const R h = (R)kFdH;
+        const bool down = !(r >= h), up = !(r + h <= (R)1);
+        Axis<R> own;
+        own.am = down ? r : h;
+        own.amp = (down && i >= 1) ? h - r : (R)0;
+        own.ap = up ? (R)1 - r : h;
+        own.apn = (up && i + 1 <= na - 2) ? (r + h) - (R)1 : (R)0;
+        const int code = down || up ? 1 : 0;
+        int codes[3];
+        all_axes<1>(&code, codes);
+        R x[3];
+        all_axes<1>(&w, x);
+        if (codes[0]) J[0] = quotient<0>(own, cell, x, B, d[0]);
+        if (codes[1]) J[1] = quotient<1>(own, cell, x, B, d[1]);
+        if (codes[2]) J[2] = quotient<2>(own, cell, x, B, d[2]);
+    }
+    // The same for places anywhere (NaN among them), and every axis in FP64.
+    __device__ __forceinline__ void any_place(unsigned cell, int i, R r, R w, const R bd[3], R& B, R& b, const R d[3],
+                                              R J[3]) const {
+        constexpr bool kExact = sizeof(R) == 8;
+        const R h = (R)kFdH;
+        int code = 2, codes[3] = {2, 2, 2};
+        if constexpr (!kExact) {
+            const bool odd = !((unsigned)i < (unsigned)(na - 1) && r >= h && r + h <= (R)1);
+            const bool below = i < -1 || (i == -1 && !(r > (R)1 - h));          // x <= -h
+            const bool above = i >= na - 1 && !(((R)(i - (na - 1)) + r) < h);  // x >= N-1+h
+            code = odd ? (r == r && (below || above) ? 1 : 2) : 0;
+            all_axes<1>(&code, codes);
+            const R bad = r - r;  // 0, or NaN, which the clamped weight does not keep
+            R bads[3];
+            all_axes<1>(&bad, bads);
+            const R any = bads[0] + bads[1] + bads[2];
+            if (any != any) B = b = any;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                if (codes[a] == 1) J[a] = (d[a] - b * bd[a]) * (R)0;
+                if (any != any) J[a] = any;
+            }
+        }
+        if (kExact || any_lane(code == 2)) {
+            const Axis<R> own = axis_setup_sel<R>(i, r, na);
+            R x[3];
+            all_axes<1>(&w, x);
+            if (codes[0] == 2) J[0] = quotient<0>(own, cell, x, B, d[0]);
+            if (codes[1] == 2) J[1] = quotient<1>(own, cell, x, B, d[1]);
+            if (codes[2] == 2) J[2] = quotient<2>(own, cell, x, B, d[2]);
+        }
+    }
+
     // scott_stage for this lane's components; b receives the unit field.
     __device__ __forceinline__ void stage(const QuadLine<R>& L, R dx, R du, R dv, R sc, R& kx, R& ku, R& kv, R& b) const {
         constexpr bool kExact = sizeof(R) == 8;
@@ -252,32 +305,15 @@ struct QuadScott {
         // (a weight nearer to a face than h + 1e-6, which NaN and places outside
         // have too, for the exact test to follow)
         if (kExact || any_lane(!(fabsf((float)w - 0.5f) <= (float)(0.5 - kFdH - 1e-6)))) {
-            int code = 2, codes[3] = {2, 2, 2};
             if constexpr (!kExact) {
                 i = sum_int(fh, fq);
-                const bool odd = !((unsigned)i < (unsigned)(na - 1) && r >= h && r + h <= (R)1);
-                const bool below = i < -1 || (i == -1 && !(r > (R)1 - h));          // x <= -h
-                const bool above = i >= na - 1 && !(((R)(i - (na - 1)) + r) < h);  // x >= N-1+h
-                code = odd ? (r == r && (below || above) ? 1 : 2) : 0;
-                all_axes<1>(&code, codes);
-                const R bad = r - r;  // 0, or NaN, which the clamped weight does not keep
-                R bads[3];
-                all_axes<1>(&bad, bads);
-                const R any = bads[0] + bads[1] + bads[2];
-                if (any != any) B = b = any;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    if (codes[a] == 1) J[a] = (d[a] - b * bd[a]) * (R)0;
-                    if (any != any) J[a] = any;
+                if (!any_lane(!((unsigned)i < (unsigned)(na - 1) && r == r))) {
+                    near_plane(cell, i, r, w, B, d, J);
+                } else {
+                    any_place(cell, i, r, w, bd, B, b, d, J);
                 }
-            }
-            if (kExact || any_lane(code == 2)) {
-                const Axis<R> own = axis_setup_sel<R>(i, r, na);
-                R x[3];
-                all_axes<1>(&w, x);
-                if (codes[0] == 2) J[0] = quotient<0>(own, cell, x, B, d[0]);
-                if (codes[1] == 2) J[1] = quotient<1>(own, cell, x, B, d[1]);
-                if (codes[2] == 2) J[2] = quotient<2>(own, cell, x, B, d[2]);
+            } else {
+                any_place(cell, i, r, w, bd, B, b, d, J);
             }
         }
         kx = sc * b;
