@@ -145,7 +145,7 @@ __global__ void __launch_bounds__(256) k_build_cells(const T* __restrict__ bx, c
 }
 
 // Pairs (FieldPairs) of the float field.  Bound by memory: 12 bytes read and 32
-// written a node, 256^3 nodes 0.2 ms.
+// written a node, 256^3 nodes 0.12 ms (6.2 TB/s).
 __global__ void __launch_bounds__(256) k_build_pairs(const float* __restrict__ bx, const float* __restrict__ by,
                                                      const float* __restrict__ bz, unsigned nodes,
                                                      float4* __restrict__ pairs) {
@@ -3701,6 +3701,54 @@ __global__ void k_scatter_f32(unsigned long long m, const uint64_t* __restrict__
     for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < m;
          i += (unsigned long long)gridDim.x * blockDim.x)
         target[pix[i]] = v[i];
+}
+
+// Per-line arrays into or out of the order `perm`, all of them in one launch: by
+// torch an array takes two (the index converted, then the copy), 40 for a map's
+// outputs.  Bound by memory, and for small maps by the launch: 1024^2 pixels, 20
+// outputs 0.28 -> 0.044 ms, 256^2 pixels, 15 outputs 0.13 -> 0.008 ms.
+constexpr int kPermuteMax = 24;
+struct PermuteArrays {
+    const char* src[kPermuteMax];
+    char* dst[kPermuteMax];
+    unsigned long long stride[kPermuteMax];  // of the source, in elements
+    int wide[kPermuteMax];                   // 8-byte elements
+    int count;
+};
+template <bool kScatter>
+__global__ void __launch_bounds__(256) k_permute(unsigned long long n, const int* __restrict__ perm, PermuteArrays a) {
+    for (unsigned long long i = blockIdx.x * 256ull + threadIdx.x; i < n; i += gridDim.x * 256ull) {
+        const unsigned long long p = (unsigned)perm[i], from = kScatter ? i : p, to = kScatter ? p : i;
+        for (int k = 0; k < a.count; ++k) {
+            if (a.wide[k])
+                ((unsigned long long*)a.dst[k])[to] = ((const unsigned long long*)a.src[k])[from * a.stride[k]];
+            else
+                ((unsigned*)a.dst[k])[to] = ((const unsigned*)a.src[k])[from * a.stride[k]];
+        }
+    }
+}
+
+extern "C" int fqsl_permute(uint64_t n, const int32_t* perm, int scatter, int count, const void* const* src,
+                            const uint64_t* src_stride, void* const* dst, const int32_t* elem_bytes, void* stream) {
+    if (count < 0 || count > kPermuteMax) return set_err(FQSL_ERR_INVALID, "%d arrays (at most %d)", count, kPermuteMax);
+    if (n == 0 || count == 0) return FQSL_OK;
+    if (!perm || !src || !src_stride || !dst || !elem_bytes) return set_err(FQSL_ERR_INVALID, "NULL argument");
+    PermuteArrays a{};
+    a.count = count;
+    for (int k = 0; k < count; ++k) {
+        if (!src[k] || !dst[k]) return set_err(FQSL_ERR_INVALID, "array %d is NULL", k);
+        if (elem_bytes[k] != 4 && elem_bytes[k] != 8)
+            return set_err(FQSL_ERR_INVALID, "array %d: elements of %d bytes", k, elem_bytes[k]);
+        a.src[k] = (const char*)src[k];
+        a.dst[k] = (char*)dst[k];
+        a.stride[k] = src_stride[k];
+        a.wide[k] = elem_bytes[k] == 8;
+    }
+    hipStream_t st = (hipStream_t)stream;
+    if (scatter) k_permute<true><<<grid_for((long)n, 256), 256, 0, st>>>(n, perm, a);
+    else k_permute<false><<<grid_for((long)n, 256), 256, 0, st>>>(n, perm, a);
+    HIP_TRY(hipGetLastError());
+    return FQSL_OK;
 }
 
 extern "C" int fqsl_bad_pixels(uint64_t n, const int32_t* b_flag, const float* q, const float* x, const float* y,

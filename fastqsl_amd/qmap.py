@@ -30,12 +30,19 @@ from .field import Field
 from .trace import trace_plain, trace_scott
 
 
-def _grid(seeds, shape):
+def _seed_rows(seeds, shape):
     import torch
     s = seeds if isinstance(seeds, torch.Tensor) else torch.as_tensor(np.asarray(seeds, np.float32))
     s = s.to(device="cuda", dtype=torch.float32).reshape(-1, 3)
     if s.shape[0] != int(np.prod(shape)):
         raise ValueError(f"{s.shape[0]} seeds do not fill a {shape} grid")
+    return s
+
+
+def _grid(seeds, shape, perm=None):
+    s = _seed_rows(seeds, shape)
+    if perm is not None:
+        return _permute([s[:, 0], s[:, 1], s[:, 2]], perm, scatter=False)
     return s[:, 0].contiguous(), s[:, 1].contiguous(), s[:, 2].contiguous()
 
 
@@ -46,10 +53,8 @@ def scott_qmap(field: Field, seeds, shape, method="rkf45", step=0.25, tol=1e-6,
     longest-first order then keeps blocks together within a length class,
     ~1 % on the 1024^2 multipole map); returns a dict of (rows, cols)
     tensors: q_0, q_perp, flag_start, flag_end, b_this_z, ..."""
-    x, y, z = _grid(seeds, shape)
     perm = block_order(shape, (tile, tile)) if tile and tile > 1 else None
-    if perm is not None:
-        x, y, z = x[perm], y[perm], z[perm]
+    x, y, z = _grid(seeds, shape, perm)
     r = trace_scott(field, x, y, z, method=method, step=step, tol=tol, precision=precision,
                     schedule=schedule)
     if perm is not None:
@@ -152,7 +157,7 @@ def scott_qcube(field: Field, x_axis, y_axis, z_axis, method="rkf45", step=0.25,
     x, y, z, shape = cube_seeds(x_axis, y_axis, z_axis)
     perm = block_order(shape, (brick,) * 3) if brick and brick > 1 else None
     if perm is not None:
-        x, y, z = x[perm], y[perm], z[perm]
+        x, y, z = _permute([x, y, z], perm, scatter=False)
     r = trace_scott(field, x, y, z, method=method, step=step, tol=tol, precision=precision,
                     schedule=schedule, outputs=outputs)
     if perm is not None:
@@ -233,17 +238,28 @@ def block_order(shape, block):
     return t
 
 
+def _permute(arrays, perm, scatter):
+    """1-D arrays (of any stride) in the order ``perm``, or back from it
+    (``scatter``), in one launch per 24 of them on the current stream."""
+    import ctypes
+    import torch
+    from . import _lib
+    from .trace import _stream
+    out = [torch.empty(v.shape, dtype=v.dtype, device=v.device) for v in arrays]
+    for k in range(0, len(arrays), 24):
+        src, dst = arrays[k:k + 24], out[k:k + 24]
+        m = len(src)
+        _lib.check(_lib.lib().fqsl_permute(
+            perm.numel(), perm.data_ptr(), int(scatter), m, (ctypes.c_void_p * m)(*[v.data_ptr() for v in src]),
+            (ctypes.c_uint64 * m)(*[v.stride(0) for v in src]), (ctypes.c_void_p * m)(*[v.data_ptr() for v in dst]),
+            (ctypes.c_int32 * m)(*[v.element_size() for v in src]), _stream(None)))
+    return out
+
+
 def _unpermute(r, perm):
     """Per-line outputs traced in ``perm`` order, back in seed order."""
-    import torch
-    out = {}
-    for k, v in r.items():
-        if k == "_seeds":
-            continue
-        u = torch.empty_like(v)
-        u[perm] = v
-        out[k] = u
-    return out
+    names = [k for k in r if k != "_seeds"]
+    return dict(zip(names, _permute([r[k] for k in names], perm, scatter=True)))
 
 
 def neighbour_qmap(field: Field, seeds, shape, stride, normal=(0.0, 0.0, 1.0), method="rkf45",
@@ -263,10 +279,8 @@ def neighbour_qmap(field: Field, seeds, shape, stride, normal=(0.0, 0.0, 1.0), m
     the number of pseudo pixels (``n_pseudo``, a CUDA int64 scalar written on
     the stream: ``int(res["n_pseudo"])`` waits for it)."""
     import torch
-    x, y, z = _grid(seeds, shape)
     perm = block_order(shape, (tile, tile)) if tile and tile > 1 else None
-    if perm is not None:
-        x, y, z = x[perm], y[perm], z[perm]
+    x, y, z = _grid(seeds, shape, perm)
     r = trace_plain(field, x, y, z, ncross=normal, method=method, step=step, tol_coef=tol_coef,
                     precision=precision, schedule=schedule)
     if perm is not None:  # back to pixel order

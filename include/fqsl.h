@@ -423,6 +423,13 @@ int fqsl_bad_pixels(uint64_t n, const int32_t *b_flag, const float *q, const flo
                     const float *z, uint64_t capacity, float *seed_x, float *seed_y, float *seed_z,
                     uint64_t *pixel, uint64_t *count_host, void *stream);
 
+/* `count` (at most 24) arrays of n elements of 4 or 8 bytes each, in one launch:
+ * dst[k][perm[i]] = src[k][i * src_stride[k]] (scatter), or
+ * dst[k][i] = src[k][perm[i] * src_stride[k]].  perm: a permutation of 0..n-1 on
+ * the device; the pointer tables are read on the host before the call returns. */
+int fqsl_permute(uint64_t n, const int32_t *perm, int scatter, int count, const void *const *src,
+                 const uint64_t *src_stride, void *const *dst, const int32_t *elem_bytes, void *stream);
+
 /* target[pixel[i]] = values[i] for i < m (the fix-up's
  * Qall_1d[idx_bad] = q_perp_bad, same cell). */
 int fqsl_scatter_f32(uint64_t m, const uint64_t *pixel, const float *values, float *target, void *stream);
