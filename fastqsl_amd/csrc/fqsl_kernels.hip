@@ -2521,11 +2521,13 @@ extern "C" size_t fqsl_scott_batch_workspace_bytes(const fqsl_scott_request* req
     if (!reqs || nreq <= 0) return 0;
     unsigned long long lines = 0;
     for (int k = 0; k < nreq; ++k) lines += reqs[k].n;
-    std::vector<int> ord = batch_order(reqs, nreq);
-    int ngroups = 0;
-    for (int k = 0; k < nreq; ++k)
-        if (k == 0 || reqs[ord[k]].field != reqs[ord[k - 1]].field || reqs[ord[k]].method != reqs[ord[k - 1]].method)
-            ++ngroups;
+    // the groups of batch_order, whose layouts go by the field, without reading a field
+    std::vector<std::pair<const fqsl_field*, int>> groups(nreq);
+    for (int k = 0; k < nreq; ++k) groups[k] = {reqs[k].field, reqs[k].method};
+    std::sort(groups.begin(), groups.end(), [](const auto& a, const auto& b) {
+        return a.first != b.first ? std::less<const fqsl_field*>()(a.first, b.first) : a.second < b.second;
+    });
+    const int ngroups = (int)(std::unique(groups.begin(), groups.end()) - groups.begin());
     return batch_layout(nreq, ngroups, lines, precision).total;
 }
 
