@@ -1427,9 +1427,12 @@ __device__ __forceinline__ void trace_sides(const F& f, const PlainParams& P, co
 #endif
 }
 
+// Sides a wavefront takes at the least (see kQuadMinFp32).
+constexpr int kPlainQuadMin = 4;
+
 // Plain tracing, persistent (fqsl_quad.h), every side by a quad of lanes.
 // `spread` wavefronts share few sides before a wavefront takes a second one, so
-// that none waits for another's branch.  Bound by the dependent instructions of
+// that few wait for another's branch.  Bound by the dependent instructions of
 // the longest side, 0.17 (RK4) to 0.21 us (RKF45) an evaluation; one thread per
 // line took 1.05 us, its three axes in turn on one lane with a branch tree each.
 // 233 x 191 lines on a 128 x 130 x 96 multipole: 1.9 -> 0.6 ms.
@@ -1441,7 +1444,7 @@ k_plain_quads(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, Dev
     fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];  // J lives on B's grid
     grid_prologue(g);
     const unsigned long long share = (2ull * n + (unsigned)spread - 1) / (unsigned)spread;
-    const int width = share > 16ull ? 16 : (share < 1ull ? 1 : (int)share);
+    const int width = share > 16ull ? 16 : (share < (unsigned)kPlainQuadMin ? kPlainQuadMin : (int)share);
     trace_sides<1, R, F, FJ, G>(f, P, s, n, o, queue, width, 4 < width ? 4 : width, nullptr, nullptr, fj, g);
 }
 
@@ -1464,7 +1467,7 @@ k_plain_sides(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, Dev
     if (tl.list && blockIdx.x < (unsigned)tangent_blocks) {
         const unsigned long long m = *tl.count, waves = 4ull * (unsigned)tangent_blocks;
         const unsigned long long share = (2ull * m + waves - 1) / waves;
-        const int width = share > 16ull ? 16 : (share < 1ull ? 1 : (int)share);
+        const int width = share > 16ull ? 16 : (share < (unsigned)kPlainQuadMin ? kPlainQuadMin : (int)share);
         trace_sides<1, R, F, FJ, G>(f, P, s, m, o, queue, width, 4 < width ? 4 : width, tl.list, nullptr, fj, g);
     }
     trace_sides<3, R, F, FJ, G>(f, P, s, n, o, queue + 1, 64, refill_min, nullptr,
@@ -1577,12 +1580,37 @@ struct ScottStepping {
     unsigned long long lines = 0;
 };
 
-// FP64 lines up to which a launch goes by quads, eight a resident quad: above
-// it the quads' extra instructions cost more than their shorter chain gives (RK4
-// and RKF45 on a 128^3 field, ms by quads / by lanes: 16 k lines 4.0 / 7.3 and
-// 4.9 / 10.7, 102 k 4.7 / 7.6 and 7.4 / 12.0, 147 k 7.0 / 7.5 and 10.0 / 12.1,
-// 200 k 8.4 / 7.4 and 12.8 / 12.3).
-constexpr unsigned long long kScottQuadLinesFp64 = 131072;
+// FP64 lines up to which a launch goes by quads, four a resident quad: above it
+// the quads' extra instructions cost more than their shorter chain gives, first
+// where seeds lie anywhere in the box and share no cells (ms by quads / by lanes,
+// RK4 on 108 x 66 x 51: 16 k lines 2.05 / 3.66, 33 k 3.2 / 3.7, 66 k 4.8 / 3.7, 131 k
+// 8.3 / 5.3; RKF45 66 k 10.5 / 11.7, 131 k 18.0 / 14.9), last on maps (128^3: 147 k
+// 7.0 / 7.5, 200 k 8.4 / 7.4).
+constexpr unsigned long long kScottQuadLinesFp64 = 65536;
+// Lines (or sides) a wavefront takes at the least.  With one or two quads of a
+// wavefront traced, few lines wait longer than in one wavefront: spread over every
+// CU and XCD, each starts on caches and address translations that no other line
+// has filled.  Lines in a 108 x 66 x 51 / 128^3 box, ms at least 1 / 2 / 4 / 8 / 16 a wavefront:
+// FP32c RKF45 64 lines .99 / 1.09 / .72 / .69 / .80 and 1.21 / 1.43 / .93 / .91 / .99, 1359
+// .92 / 1.04 / 1.00 / 1.03 / 1.10, 4096 1.13 / 1.05 / .99 / 1.04 / 1.16; FP64 RK4 64 lines
+// 3.44 / 4.23 / 2.23 / 1.53 / 1.49 (3.1 by lanes), 1359 4.24 / 4.34 / 2.49 / 1.95 / 1.91.
+constexpr int kQuadMinFp32 = 4, kQuadMinFp64 = 16;
+template <typename R>
+constexpr int quad_min() { return sizeof(R) == 4 ? kQuadMinFp32 : kQuadMinFp64; }
+// Workgroups, and wavefronts over which `n` lines are spread (`full`: a resident
+// grid, `spread`: wavefronts a SIMD).
+struct QuadGrid {
+    int blocks, waves;
+};
+static QuadGrid quad_grid(unsigned long long n, int full, int spread, int least) {
+    const unsigned long long wanted = (n + (unsigned)least - 1) / (unsigned)least;  // wavefronts
+    const unsigned long long blocks = (wanted + 3) / 4;
+    QuadGrid g;
+    g.blocks = blocks < (unsigned long long)full ? (int)std::max(blocks, 1ull) : full;
+    g.waves = (int)std::min<unsigned long long>((unsigned long long)std::min(full, cu_count() * spread) * 4,
+                                                std::max(wanted, 1ull));
+    return g;
+}
 // Wavefronts per SIMD over which few lines are spread before a wavefront takes a
 // second one, and the quads that wait before ended sides are landed and free
 // quads refilled: every wait of an FP32c quad is an issue slot of the others
@@ -1659,9 +1687,8 @@ static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, co
     if (timed) e = hipEventRecord(g_evs0, st);
     if constexpr (std::is_same<R, X>::value) {
         if (!step.kern) {
-            const unsigned long long wanted = (n_hint + 3) / 4;  // one line per wavefront at the least
-            const int grid = wanted < (unsigned long long)step.grid ? (int)wanted : step.grid;
-            const int waves = std::min(step.grid, cu_count() * kScottSpread) * 4;
+            const QuadGrid g = quad_grid(n_hint, step.grid, kScottSpread, quad_min<R>());
+            const int grid = g.blocks, waves = g.waves;
             const int refill = sizeof(R) == 4 ? kScottQuadRefillFp32 : kScottQuadRefillFp64;
             bool done = false;
             if constexpr (std::is_same<F, FieldSoA<float>>::value) {
@@ -2502,11 +2529,9 @@ int batch_launch(const fqsl_scott_batch* b, const BatchGroup& S, int qi, hipStre
             if (rc) return rc;
             full = (int)((long)full * g_tune[FQSL_TUNE_GRID_PCT] / 100);
             if (full < 1) full = 1;
-            const unsigned long long wanted = (S.n + 3) / 4;  // one line per wavefront at the least
-            const int grid = wanted < (unsigned long long)full ? (int)wanted : full;
-            const int waves = std::min(full, cu_count() * kScottSpread) * 4;
-            k_batch_quads<R, F><<<grid, 256, 0, st>>>(g, frames, recs, b->ctl, qi, waves,
-                                                      sizeof(R) == 4 ? kScottQuadRefillFp32 : kScottQuadRefillFp64);
+            const QuadGrid q = quad_grid(S.n, full, kScottSpread, quad_min<R>());
+            k_batch_quads<R, F><<<q.blocks, 256, 0, st>>>(g, frames, recs, b->ctl, qi, q.waves,
+                                                          sizeof(R) == 4 ? kScottQuadRefillFp32 : kScottQuadRefillFp64);
         }
     }
     if (!quads) rc = batch_step_groups<R, F, X>(b, S, st);
