@@ -993,10 +993,9 @@ def bench_trace(args, fq, torch, log, volume):
 
     classes, counts = np.unique(flags, return_counts=True)
     prof = "volume" if volume else "plane"
-    waves = fq._lib.tune_get("scott_waves") if args.precision == "fp32c" else 0
     roof = valu_roofline(prof, kms, evals, bpe, oracle_evals,
-                         kernel=("stepping kernel k_scott_persistent%s" % ("_w%d" % waves if waves else "")
-                                 if args.schedule == "persistent" else "k_scott_per_line"))
+                         kernel=("k_scott_per_line" if args.schedule != "persistent" else
+                                 "stepping kernel " + ("k_scott_quads" if args.precision == "fp32c" else "k_scott_persistent")))
     if not (args.precision == "fp32c" and args.schedule == "persistent" and (volume or args.pixels == 1024)):
         roof.update(achieved=None, frac=None, valu_insts_per_launch=None, traffic=None,
                     note="the profile covers the default FP32c persistent workload only")
