@@ -2296,7 +2296,7 @@ k_batch_quads(BatchGroupArgs g, const R* frames, ScottRec<R>* recs, BatchCtl c, 
 
 // Persistent stepping over one group: as scott_persistent_body, with the
 // step and tolerance of each lane's request.
-template <typename R, class F, typename X>
+template <typename R, class F, typename X, bool kRoll = false>
 __device__ __forceinline__ void scott_batch_body(F f, int method, BatchGroupArgs g, const R* __restrict__ frames,
                                                  ScottRec<R>* __restrict__ recs, BatchCtl c, int qi,
                                                  int refill_min) {
@@ -2344,7 +2344,7 @@ __device__ __forceinline__ void scott_batch_body(F f, int method, BatchGroupArgs
         }
         if (active) {
             ScottEnd<R> e;
-            const int st = scott_attempt<R, F, NoCurrent, X>(L, f, P, e);
+            const int st = scott_attempt<R, F, NoCurrent, X, kRoll>(L, f, P, e);
             if (st != kTracing) {
                 recs[idx] = ScottRec<R>{L.st, e, L.len, st, L.evals, L.tw};
                 active = false;
@@ -2365,6 +2365,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 k_batch_step_w2(F f, int method, BatchGroupArgs g, const R* frames, ScottRec<R>* recs, BatchCtl c, int qi,
                 int refill_min) {
     scott_batch_body<R, F, X>(f, method, g, frames, recs, c, qi, refill_min);
+}
+
+template <typename R, class F, typename X>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
+k_batch_step_w3(F f, int method, BatchGroupArgs g, const R* frames, ScottRec<R>* recs, BatchCtl c, int qi,
+                int refill_min) {
+    scott_batch_body<R, F, X, true>(f, method, g, frames, recs, c, qi, refill_min);
 }
 
 template <typename R, class F>
@@ -2495,7 +2502,8 @@ std::vector<int> batch_order(const fqsl_scott_request* reqs, int nreq) {
 
 template <typename R, class F, typename X>
 int batch_step_groups(const fqsl_scott_batch* b, const BatchGroup& S, hipStream_t st) {
-    auto kern = std::is_same<R, X>::value ? k_batch_step<R, F, X> : k_batch_step_w2<R, F, X>;
+    auto kern = sizeof(R) == 8 ? k_batch_step<R, F, X>
+              : std::is_same<R, X>::value ? k_batch_step_w3<R, F, X> : k_batch_step_w2<R, F, X>;
     int grid = 0;
     int rc = persistent_grid(kern, &grid);
     if (rc) return rc;
@@ -2511,8 +2519,14 @@ int batch_step_groups(const fqsl_scott_batch* b, const BatchGroup& S, hipStream_
     return FQSL_OK;
 }
 
-// The requests of one layout: by quads where a trace of as many lines goes by
-// quads (scott_stepping), in one launch.
+// FP32c lines of a layout up to which a batch goes by quads: 1.4 M lines over three
+// fields 41.1 ms against 48.9 by lanes, but 50.5 M lines in 256 requests 1.55 s
+// against 1.46: with hundreds of lines a quad no tail is left to shorten, and a
+// launch per (field, method) keeps to one field at a time.
+constexpr unsigned long long kBatchQuadLinesFp32 = 1ull << 24;
+
+// The requests of one layout: by quads, in one launch, up to the line counts above
+// (FP64: as a single trace, scott_stepping).
 template <typename R, class F, typename X = R>
 int batch_launch(const fqsl_scott_batch* b, const BatchGroup& S, int qi, hipStream_t st) {
     const BatchGroupArgs g{b->reqs, b->offs, S.r0, S.r1, S.base, S.n};
@@ -2522,7 +2536,7 @@ int batch_launch(const fqsl_scott_batch* b, const BatchGroup& S, int qi, hipStre
     int rc = FQSL_OK;
     bool quads = false;
     if constexpr (std::is_same<R, X>::value) {
-        quads = sizeof(R) == 4 || S.n <= kScottQuadLinesFp64;
+        quads = S.n <= (sizeof(R) == 4 ? kBatchQuadLinesFp32 : kScottQuadLinesFp64);
         if (quads) {
             int full = 0;
             rc = persistent_grid(k_batch_quads<R, F>, &full);
