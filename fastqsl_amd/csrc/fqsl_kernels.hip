@@ -33,6 +33,7 @@
 #include "fqsl.h"
 #include "fqsl_quad.h"
 #include "fqsl_quad_scott.h"
+#include "fqsl_route.h"
 #include "fqsl_stretch.h"
 #include "fqsl_tracer.h"
 
@@ -1256,7 +1257,7 @@ __device__ __forceinline__ void apply_plain_scalars(F& f, PlainParams& P, unsign
     f.n[0] = ds.shape[0]; f.n[1] = ds.shape[1]; f.n[2] = ds.shape[2];
     P.s0 = (double)ds.s_len[0];
     P.tol_coef = ds.tol_coef ? (double)ds.tol_coef[0] : 1.0;
-    n = ds.N[0];
+    if (ds.N) n = ds.N[0];
     P.ncross[0] = ncross[0]; P.ncross[1] = ncross[1]; P.ncross[2] = ncross[2];
 }
 
@@ -1782,16 +1783,9 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
 // Wavefronts per SIMD over which few sides are spread before a wavefront takes
 // a second one.
 constexpr int kPlainSpread = 2;
-// Sides up to which an RKF45 launch is traced by quads alone, two per resident
-// quad.  On the multipole 256^3 field (s_len 1/8, tol_coef 0.5; ms by quads /
-// tangent lines by quads and the rest by lanes): 65 k sides 0.72 / 0.73, 131 k
-// 0.68 / 0.70, 262 k 0.90 / 0.84, 1.0 M 1.57 / 1.25, 2.1 M 2.38 / 1.74.  RK4
-// lines have no tangent class and all go by quads, whose two loads a stage touch
-// a third of the cache lines of a lane's six (2.1 M sides 10.4 against 11.9 ms).
-constexpr unsigned long long kPlainQuadSides = 131072;
-
 // Both schedules run the same kernels; a line's result does not depend on which
-// lanes trace it.
+// lanes trace it.  `n_hint` is the number of lines (the capacity of the arrays
+// where ds.n_dev holds fewer); where ds.N holds it on the device, only a cap.
 template <typename R, class F, class FJ = NoCurrent, class G = UniformGrid>
 static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsigned long long n, const PlainOut& o,
                         const DevScalars& ds, const float* ncross, int schedule, hipStream_t st,
@@ -1805,13 +1799,14 @@ static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsign
     // 5 bytes a line; a capturing stream takes no allocation and traces by quads.
     TangentLines tl{nullptr, nullptr, q + 2};
     char* ws = nullptr;
-    if (P.method == kRKF45 && 2ull * n_hint > kPlainQuadSides && n_hint < (1ull << 32)) {
+    const unsigned long long listed = plain_listed_lines(P.method == kRKF45, n_hint, !ds.N);
+    if (listed) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         HIP_TRY(hipStreamIsCapturing(st, &cap));
         if (cap == hipStreamCaptureStatusNone) {
-            HIP_TRY(hipMallocAsync((void**)&ws, 5 * (size_t)n_hint, st));
+            HIP_TRY(hipMallocAsync((void**)&ws, 5 * (size_t)listed, st));
             tl.list = (unsigned*)ws;
-            tl.marked = (unsigned char*)ws + 4 * (size_t)n_hint;
+            tl.marked = (unsigned char*)ws + 4 * (size_t)listed;
         }
     }
     int grid = 0;
@@ -3142,10 +3137,11 @@ extern "C" int fqsl_trace_plain_n(const fqsl_field* field, const fqsl_plain_para
 }
 
 // ------------------------------------------- reference-shaped entry points
-// The seed count N lives on the device; the per-line launch needs a grid on
-// the host, so it runs a chip-sized grid (per_line_grid) whose grid-stride
-// loop covers any N, as the reference's fixed grids do.  kPerLineMaxBlocks *
-// 256 is only the cap passed as the line-count hint.
+// The seed count N lives on the device.  The plain entries read it with the
+// switches they wait for anyway; where a call has none, and in the Scott
+// entry's per-line launch, the grid is chip-sized (per_line_grid) and its
+// grid-stride loop or queue covers any N, as the reference's fixed grids do.
+// kPerLineMaxBlocks * 256 is then only the cap passed as the line-count hint.
 static constexpr int kPerLineMaxBlocks = 65536;
 
 // Whether the Scott entry pairs the nodes of the in-place field first.  Quads
@@ -3241,9 +3237,12 @@ extern "C" int fqsl_TraceAllBline(int method, float* Bx, float* By, float* Bz, i
     if (!Bx || !By || !Bz || !BshapeN || !inp_x || !inp_y || !inp_z || !inp_cross_dir || !s_len || !N)
         return set_err(FQSL_ERR_INVALID, "NULL required argument");
     bool twist_on = false;
-    if (curB_flag) {  // the switch is a device scalar: read it (synchronises the stream)
+    unsigned long long n = 0, n_hint = (unsigned long long)kPerLineMaxBlocks * 256;
+    if (curB_flag) {  // the switch is a device scalar: read it, and the line count (synchronises the stream)
         HIP_TRY(hipMemcpyAsync(&twist_on, curB_flag, sizeof(bool), hipMemcpyDeviceToHost, (hipStream_t)stream));
+        HIP_TRY(hipMemcpyAsync(&n, N, sizeof(n), hipMemcpyDeviceToHost, (hipStream_t)stream));
         HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+        n_hint = n;
     }
     if (twist_on && (!curB_x || !curB_y || !curB_z || !twist))
         return set_err(FQSL_ERR_INVALID, "curB_flag is set: curB_x/y/z and twist must be device arrays");
@@ -3259,14 +3258,13 @@ extern "C" int fqsl_TraceAllBline(int method, float* Bx, float* By, float* Bz, i
     PlainOut o{start_x, start_y, start_z, end_x, end_y, end_z, flag_start, flag_end, B_this_x, B_this_y, B_this_z,
                B_flag, B_start_x, B_start_y, B_start_z, B_end_x, B_end_y, B_end_z, LineLen, nullptr,
                twist_on ? twist : nullptr};
-    DevScalars ds{BshapeN, s_len, N, method == FQSL_METHOD_RKF45 ? tol_coef : nullptr, curB_flag, twist};
+    DevScalars ds{BshapeN, s_len, curB_flag ? nullptr : N, method == FQSL_METHOD_RKF45 ? tol_coef : nullptr, curB_flag, twist};
     FieldSoA<float> f{Bx, By, Bz, {2, 2, 2}};
-    const unsigned long long n_hint = (unsigned long long)kPerLineMaxBlocks * 256;
     if (twist_on) {
         const FieldSoA<float> fj{curB_x, curB_y, curB_z, {2, 2, 2}};  // shape taken from B's on the device
-        return launch_plain<float>(f, P, s, 0ull, o, ds, inp_cross_dir, schedule, (hipStream_t)stream, n_hint, fj);
+        return launch_plain<float>(f, P, s, n, o, ds, inp_cross_dir, schedule, (hipStream_t)stream, n_hint, fj);
     }
-    return launch_plain<float>(f, P, s, 0ull, o, ds, inp_cross_dir, schedule, (hipStream_t)stream, n_hint);
+    return launch_plain<float>(f, P, s, n, o, ds, inp_cross_dir, schedule, (hipStream_t)stream, n_hint);
 }
 
 // Lookup tables of the stretched drop-in, per device, kept while the axes
@@ -3299,10 +3297,12 @@ extern "C" int fqsl_TraceAllBlineStretch(float* Bx, float* By, float* Bz, int* B
     if (precision != FQSL_PREC_FP32C)
         return set_err(FQSL_ERR_UNSUPPORTED, "the in-place float field supports FQSL_PREC_FP32C only");
     hipStream_t st = (hipStream_t)stream;
-    // the shape and the two switches are device scalars: read them (synchronises the stream)
+    // the shape, the line count and the two switches are device scalars: read them (synchronises the stream)
     int shape[3] = {0, 0, 0};
+    unsigned long long n = 0;
     bool uni = false, twist_on = false;
     HIP_TRY(hipMemcpyAsync(shape, BshapeN, sizeof(shape), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(&n, N, sizeof(n), hipMemcpyDeviceToHost, st));
     if (flag_uni) HIP_TRY(hipMemcpyAsync(&uni, flag_uni, sizeof(bool), hipMemcpyDeviceToHost, st));
     if (curB_flag) HIP_TRY(hipMemcpyAsync(&twist_on, curB_flag, sizeof(bool), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
@@ -3357,17 +3357,16 @@ extern "C" int fqsl_TraceAllBlineStretch(float* Bx, float* By, float* Bz, int* B
     PlainOut o{start_x, start_y, start_z, end_x, end_y, end_z, flag_start, flag_end, B_this_x, B_this_y, B_this_z,
                B_flag, B_start_x, B_start_y, B_start_z, B_end_x, B_end_y, B_end_z, LineLen, nullptr,
                twist_on ? twist : nullptr};
-    DevScalars ds{BshapeN, s_len, N, tol_coef, curB_flag, twist};
+    DevScalars ds{BshapeN, s_len, nullptr, tol_coef, curB_flag, twist};
     FieldSoA<float> f{Bx, By, Bz, {shape[0], shape[1], shape[2]}};
-    const unsigned long long n_hint = (unsigned long long)kPerLineMaxBlocks * 256;
     const FieldSoA<float> fj{curB_x, curB_y, curB_z, {shape[0], shape[1], shape[2]}};
     if (stretch_lds_fits(lds_bytes)) {
         const StretchLds gl{g.g, lds_bytes};
-        if (twist_on) return launch_plain<float>(f, P, s, 0ull, o, ds, inp_cross_dir, schedule, st, n_hint, fj, gl);
-        return launch_plain<float>(f, P, s, 0ull, o, ds, inp_cross_dir, schedule, st, n_hint, NoCurrent{}, gl);
+        if (twist_on) return launch_plain<float>(f, P, s, n, o, ds, inp_cross_dir, schedule, st, n, fj, gl);
+        return launch_plain<float>(f, P, s, n, o, ds, inp_cross_dir, schedule, st, n, NoCurrent{}, gl);
     }
-    if (twist_on) return launch_plain<float>(f, P, s, 0ull, o, ds, inp_cross_dir, schedule, st, n_hint, fj, g);
-    return launch_plain<float>(f, P, s, 0ull, o, ds, inp_cross_dir, schedule, st, n_hint, NoCurrent{}, g);
+    if (twist_on) return launch_plain<float>(f, P, s, n, o, ds, inp_cross_dir, schedule, st, n, fj, g);
+    return launch_plain<float>(f, P, s, n, o, ds, inp_cross_dir, schedule, st, n, NoCurrent{}, g);
 }
 
 // ---------------------------------------------- neighbour-difference assembly
