@@ -2184,7 +2184,7 @@ struct BatchFieldOf<FieldSoA<T>> {
 };
 
 struct BatchCtl {
-    unsigned long long* queues;     // one counter per launch
+    unsigned long long* queues;     // one counter per group of requests, see BatchSpan
     unsigned long long* remaining;  // lines of each request not yet finished
     unsigned long long* stamps;     // [r]: device wall clock when request r's last line
                                     // finished stepping; [nreq]: start of the run
@@ -2395,13 +2395,10 @@ __global__ void __launch_bounds__(256) k_batch_finish(BatchGroupArgs g, const R*
     }
 }
 
-// Consecutive requests of the batch order and their lines: of one layout, or of
-// one field and method.
-struct BatchGroup {
+// A span with its layout or, where it has one field and method, these.
+struct BatchGroup : BatchSpan {
     BatchField f;
     int method;
-    int r0, r1;
-    unsigned long long base, n;
 };
 
 struct fqsl_scott_batch {
@@ -2504,12 +2501,11 @@ int batch_step_groups(const fqsl_scott_batch* b, const BatchGroup& S, hipStream_
     if (rc) return rc;
     grid = (int)((long)grid * g_tune[FQSL_TUNE_GRID_PCT] / 100);
     if (grid < 1) grid = 1;
-    for (size_t gi = 0; gi < b->groups.size(); ++gi) {
-        const BatchGroup& G = b->groups[gi];
+    for (const BatchGroup& G : b->groups) {
         if (G.n == 0 || G.r0 < S.r0 || G.r0 >= S.r1) continue;
         kern<<<grid, 256, 0, st>>>(BatchFieldOf<F>::get(G.f), G.method,
                                    BatchGroupArgs{b->reqs, b->offs, G.r0, G.r1, G.base, G.n}, (const R*)b->frames,
-                                   (ScottRec<R>*)b->recs, b->ctl, (int)gi, b->refill_min);
+                                   (ScottRec<R>*)b->recs, b->ctl, G.counter, b->refill_min);
     }
     return FQSL_OK;
 }
@@ -2523,7 +2519,7 @@ constexpr unsigned long long kBatchQuadLinesFp32 = 1ull << 24;
 // The requests of one layout: by quads, in one launch, up to the line counts above
 // (FP64: as a single trace, scott_stepping).
 template <typename R, class F, typename X = R>
-int batch_launch(const fqsl_scott_batch* b, const BatchGroup& S, int qi, hipStream_t st) {
+int batch_launch(const fqsl_scott_batch* b, const BatchGroup& S, hipStream_t st) {
     const BatchGroupArgs g{b->reqs, b->offs, S.r0, S.r1, S.base, S.n};
     R* frames = (R*)b->frames;
     ScottRec<R>* recs = (ScottRec<R>*)b->recs;
@@ -2539,7 +2535,7 @@ int batch_launch(const fqsl_scott_batch* b, const BatchGroup& S, int qi, hipStre
             full = (int)((long)full * g_tune[FQSL_TUNE_GRID_PCT] / 100);
             if (full < 1) full = 1;
             const QuadGrid q = quad_grid(S.n, full, kScottSpread, quad_min<R>());
-            k_batch_quads<R, F><<<q.blocks, 256, 0, st>>>(g, frames, recs, b->ctl, qi, q.waves,
+            k_batch_quads<R, F><<<q.blocks, 256, 0, st>>>(g, frames, recs, b->ctl, S.counter, q.waves,
                                                           sizeof(R) == 4 ? kScottQuadRefillFp32 : kScottQuadRefillFp64);
         }
     }
@@ -2588,18 +2584,16 @@ extern "C" int fqsl_scott_batch_create(const fqsl_scott_request* reqs, int nreq,
     b->order = batch_order(reqs, nreq);
     std::vector<BatchReq> table(nreq);
     std::vector<unsigned long long> offs(nreq);
+    std::vector<int> kind(nreq);
+    std::vector<char> other(nreq);
+    std::vector<unsigned long long> count(nreq);
     unsigned long long lines = 0;
     for (int k = 0; k < nreq; ++k) {
         const fqsl_scott_request& q = reqs[b->order[k]];
         const BatchField f = batch_field(q, precision);
-        const bool layout = k == 0 || f.kind != b->layouts.back().f.kind;
-        if (layout) b->layouts.push_back(BatchGroup{f, q.method, k, k, lines, 0});
-        if (layout || q.field != reqs[b->order[k - 1]].field || q.method != b->groups.back().method)
-            b->groups.push_back(BatchGroup{f, q.method, k, k, lines, 0});
-        for (BatchGroup* G : {&b->layouts.back(), &b->groups.back()}) {
-            G->r1 = k + 1;
-            G->n += q.n;
-        }
+        kind[k] = f.kind;
+        count[k] = q.n;
+        other[k] = k == 0 || q.field != reqs[b->order[k - 1]].field || q.method != table[k - 1].method;
         offs[k] = lines;
         const fqsl_scott_out& o = q.out;
         table[k] = BatchReq{Seeds{q.x, q.y, q.z},
@@ -2609,6 +2603,10 @@ extern "C" int fqsl_scott_batch_create(const fqsl_scott_request* reqs, int nreq,
                             f, q.step, q.method == FQSL_METHOD_RKF45 ? q.tol : 0.0, q.n, q.method};
         lines += q.n;
     }
+    std::vector<BatchSpan> layouts, groups;
+    batch_spans(nreq, kind.data(), other.data(), count.data(), layouts, groups);
+    for (const BatchSpan& v : layouts) b->layouts.push_back(BatchGroup{v, table[v.r0].f, table[v.r0].method});
+    for (const BatchSpan& v : groups) b->groups.push_back(BatchGroup{v, table[v.r0].f, table[v.r0].method});
     const BatchLayout L = batch_layout(nreq, (int)b->groups.size(), lines, precision);
     char* ws = (char*)workspace;
     b->ws = ws;
@@ -2646,17 +2644,15 @@ extern "C" int fqsl_scott_batch_run(const fqsl_scott_batch* b, void* stream) {
                                                                                              ng);
     HIP_TRY(hipGetLastError());
     const bool mixed = b->precision == FQSL_PREC_MIXED;
-    for (size_t k = 0; k < b->layouts.size(); ++k) {
-        const BatchGroup& S = b->layouts[k];
+    for (const BatchGroup& S : b->layouts) {
         if (S.n == 0) continue;
-        const int qi = (int)k;
         int rc;
-        if (S.f.kind == kBatchSoA64) rc = batch_launch<double, FieldSoA<double>>(b, S, qi, st);
+        if (S.f.kind == kBatchSoA64) rc = batch_launch<double, FieldSoA<double>>(b, S, st);
         else if (S.f.kind == kBatchCell32)
-            rc = mixed ? batch_launch<float, FieldCell32, double>(b, S, qi, st) : batch_launch<float, FieldCell32>(b, S, qi, st);
+            rc = mixed ? batch_launch<float, FieldCell32, double>(b, S, st) : batch_launch<float, FieldCell32>(b, S, st);
         else
-            rc = mixed ? batch_launch<float, FieldSoA<float>, double>(b, S, qi, st)
-                       : batch_launch<float, FieldSoA<float>>(b, S, qi, st);
+            rc = mixed ? batch_launch<float, FieldSoA<float>, double>(b, S, st)
+                       : batch_launch<float, FieldSoA<float>>(b, S, st);
         if (rc) return rc;
     }
     if (timed) return record_end(st);

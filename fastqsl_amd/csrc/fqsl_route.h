@@ -3,6 +3,8 @@
 // Plain host C++ without HIP, so that the CPU tests build and check the rules.
 #pragma once
 
+#include <vector>
+
 namespace fqsl {
 
 // Sides up to which an RKF45 launch is traced by quads alone, two per resident
@@ -21,6 +23,35 @@ constexpr unsigned long long kPlainQuadSides = 131072;
 inline unsigned long long plain_listed_lines(bool rkf45, unsigned long long lines, bool counted) {
     const bool list = rkf45 && counted && lines > kPlainQuadSides / 2 && lines < (1ull << 32);
     return list ? lines : 0ull;
+}
+
+// Consecutive requests of a batch and their lines: those of one layout, which a
+// launch by quads takes together, or of one field and method, which a launch by
+// lanes takes.  `counter` is the work counter of that launch.  Layouts of one
+// run go either way, each by its own line count, so both kinds of launches draw
+// from one numbering: a group's counter is its place among the groups, a
+// layout's that of its first group, which is not launched beside it.
+struct BatchSpan {
+    int r0, r1, counter;
+    unsigned long long base, n;
+};
+
+// Spans of requests in batch order: request k has n[k] lines on layout kind[k];
+// other[k]: its field or method is another than request k - 1's.
+inline void batch_spans(int nreq, const int* kind, const char* other, const unsigned long long* n,
+                        std::vector<BatchSpan>& layouts, std::vector<BatchSpan>& groups) {
+    unsigned long long lines = 0;
+    for (int k = 0; k < nreq; ++k) {
+        const bool layout = k == 0 || kind[k] != kind[k - 1];
+        const int next = (int)groups.size();
+        if (layout) layouts.push_back(BatchSpan{k, k, next, lines, 0});
+        if (layout || other[k]) groups.push_back(BatchSpan{k, k, next, lines, 0});
+        for (BatchSpan* s : {&layouts.back(), &groups.back()}) {
+            s->r1 = k + 1;
+            s->n += n[k];
+        }
+        lines += n[k];
+    }
 }
 
 }  // namespace fqsl

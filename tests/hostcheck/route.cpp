@@ -4,3 +4,30 @@
 extern "C" unsigned long long rt_plain_listed_lines(int rkf45, unsigned long long lines, int counted) {
     return fqsl::plain_listed_lines(rkf45 != 0, lines, counted != 0);
 }
+
+// Counter and first request of every launch of a batch in which layouts of at
+// most `quad_lines` lines are launched whole and larger ones group by group;
+// returns how many there are.
+extern "C" int rt_batch_launches(int nreq, const int* kind, const char* other, const unsigned long long* n,
+                                 unsigned long long quad_lines, int* counter, int* first, unsigned long long* lines) {
+    std::vector<fqsl::BatchSpan> layouts, groups;
+    fqsl::batch_spans(nreq, kind, other, n, layouts, groups);
+    int m = 0;
+    auto launch = [&](const fqsl::BatchSpan& v) {
+        counter[m] = v.counter;
+        first[m] = v.r0;
+        lines[m++] = v.n;
+    };
+    for (const fqsl::BatchSpan& s : layouts) {
+        if (s.n <= quad_lines) launch(s);
+        else
+            for (const fqsl::BatchSpan& g : groups)
+                if (g.r0 >= s.r0 && g.r0 < s.r1) launch(g);
+    }
+    return m;
+}
+extern "C" int rt_batch_groups(int nreq, const int* kind, const char* other, const unsigned long long* n) {
+    std::vector<fqsl::BatchSpan> layouts, groups;
+    fqsl::batch_spans(nreq, kind, other, n, layouts, groups);
+    return (int)groups.size();
+}

@@ -3,6 +3,7 @@ import ctypes
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -29,3 +30,27 @@ def test_every_line_a_plain_trace_may_mark_has_its_place(route, lines):
     assert f(0, lines, 1) == 0
     # a counted RKF45 launch lists all its lines or none; line numbers are 32 bits wide
     assert f(1, lines, 1) == (lines if 65536 < lines < 2 ** 32 else 0)
+
+
+@pytest.mark.parametrize("quad_lines", [0, 5, 20, 60, 10 ** 9])
+@pytest.mark.parametrize("seed", range(20))
+def test_launches_of_a_batch_share_no_counter(route, quad_lines, seed):
+    """Layouts launched whole and layouts launched by field and method in one
+    batch: every launch has its own work counter, inside the workspace's, and
+    every request lies in one launch."""
+    rng = np.random.default_rng(seed)
+    m = int(rng.integers(1, 12))
+    kind = np.sort(rng.integers(0, 3, m)).astype(np.int32)
+    other = rng.integers(0, 2, m).astype(np.int8)
+    other[0] = 1
+    n = rng.integers(0, 20, m).astype(np.uint64)
+    args = [m, kind.ctypes.data_as(ctypes.c_void_p), other.ctypes.data_as(ctypes.c_void_p), n.ctypes.data_as(ctypes.c_void_p)]
+    counter, first = np.empty(m, np.int32), np.empty(m, np.int32)
+    lines = np.empty(m, np.uint64)
+    k = route.rt_batch_launches(*args, ctypes.c_ulonglong(quad_lines), counter.ctypes.data_as(ctypes.c_void_p),
+                                first.ctypes.data_as(ctypes.c_void_p), lines.ctypes.data_as(ctypes.c_void_p))
+    counter, first, lines = counter[:k], first[:k], lines[:k]
+    assert len(set(counter)) == k and counter.min() >= 0 and counter.max() < route.rt_batch_groups(*args)
+    assert list(first) == sorted(first) and first[0] == 0
+    edges = list(first) + [m]
+    assert [n[a:b].sum() for a, b in zip(edges[:-1], edges[1:])] == list(lines)
