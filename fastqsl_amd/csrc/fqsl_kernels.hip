@@ -9,6 +9,7 @@
 //   k_scott_per_line       Scott tracer, one thread per line
 //   k_plain_quads / k_plain_sides   position-only tracer (grid-index
 //                          coordinates, or a stretched grid's own coordinates)
+//   k_plain_lines          the same, one thread per line: results over the seeds
 //   k_qcalc_plane          QCalcPlane (FastQSL.py:65-117)
 //   k_pseudo_*             CookPseudoLine compaction (FastQSL.py:4-57)
 //   k_qcut_scatter         Qcut + merge (demo/Q_RKF45CuPy.ipynb cells [10]-[11])
@@ -1261,6 +1262,12 @@ __device__ __forceinline__ void apply_plain_scalars(F& f, PlainParams& P, unsign
     P.ncross[0] = ncross[0]; P.ncross[1] = ncross[1]; P.ncross[2] = ncross[2];
 }
 
+// TraceBlineAdaptive.cu:498-501, in float as the reference.
+__device__ __forceinline__ int b_flag(const float b[3], const PlainParams& P) {
+    const float bn = fabsf(b[0] * P.ncross[0] + b[1] * P.ncross[1] + b[2] * P.ncross[2]) * 100.f;
+    return bn < sqrtf(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]) ? 1 : 0;
+}
+
 // B at a seed: Interp3d's clamped value on a uniform grid, the raw interpolant
 // on a stretched one (TraceBlineAdaptiveStretch.cu:463-496).
 template <typename R, class F>
@@ -1313,11 +1320,7 @@ __global__ void __launch_bounds__(256) k_plain_prep(F f, PlainParams P, Seeds s,
                 float b[3];
                 seed_b<R, F>(f, g, p0, b);
                 if (o.btx) { o.btx[i] = b[0]; o.bty[i] = b[1]; o.btz[i] = b[2]; }
-                if (o.bflag) {
-                    // TraceBlineAdaptive.cu:498-501, in float as the reference
-                    const float bn = fabsf(b[0] * P.ncross[0] + b[1] * P.ncross[1] + b[2] * P.ncross[2]) * 100.f;
-                    o.bflag[i] = bn < sqrtf(b[0] * b[0] + b[1] * b[1] + b[2] * b[2]) ? 1 : 0;
-                }
+                if (o.bflag) o.bflag[i] = b_flag(b, P);
             }
         }
         const unsigned long long m = __ballot(tangent);
@@ -1473,6 +1476,50 @@ k_plain_sides(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, Dev
     }
     trace_sides<3, R, F, FJ, G>(f, P, s, n, o, queue + 1, 64, refill_min, nullptr,
                                        tl.list ? tl.marked : nullptr, fj, g);
+}
+
+// One thread per line, which reads the seed once and writes the line's outputs
+// when both its sides have ended: for calls whose outputs lie on their seeds.
+// One line a thread is the slowest way to trace (1024^2 lines on a stretched
+// 256^3 grid 14.0 ms, 5.6 by k_plain_sides).  Two wavefronts per SIMD as the
+// register target: the FP64 variants otherwise run one (1.2-1.3 times slower).
+template <typename R, class F, class FJ, class G>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+k_plain_lines(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, DevScalars ds, const float* ncross, FJ fj,
+              G g) {
+    constexpr bool kUniform = std::is_same<G, UniformGrid>::value, kL = std::is_same<G, StretchLds>::value;
+    apply_plain_scalars(f, P, n, ds, ncross);
+    fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];  // J lives on B's grid
+    grid_prologue(g);
+    const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
+    for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < n; i += stride) {
+        const float p0[3] = {s.x[i], s.y[i], s.z[i]};
+        PlainLine<R> L;
+        if constexpr (kUniform) {
+            plain_init<R>(L, f, P, p0[0], p0[1], p0[2]);
+            while (!L.done) plain_attempt<R, F, FJ>(L, f, P, fj);
+        } else {
+            stretch_init<R, F, kL>(L, f, grid_of(g), P, p0[0], p0[1], p0[2]);
+            while (!L.done) stretch_attempt<R, F, FJ, kL>(L, f, grid_of(g), P, fj);
+        }
+        const float xs[3] = {(float)L.xs[0], (float)L.xs[1], (float)L.xs[2]};
+        const float xe[3] = {(float)L.xe[0], (float)L.xe[1], (float)L.xe[2]};
+        float b[3];
+        if (o.sx) { o.sx[i] = xs[0]; o.sy[i] = xs[1]; o.sz[i] = xs[2]; }
+        if (o.ex) { o.ex[i] = xe[0]; o.ey[i] = xe[1]; o.ez[i] = xe[2]; }
+        if (o.fs) o.fs[i] = L.flag_s;
+        if (o.fe) o.fe[i] = L.flag_e;
+        if (o.len) o.len[i] = L.len_total;
+        if (o.evals) o.evals[i] = L.evals;
+        if (o.tw) o.tw[i] = L.tw;
+        if (o.bsx) { seed_b<R, F>(f, g, xs, b); o.bsx[i] = b[0]; o.bsy[i] = b[1]; o.bsz[i] = b[2]; }
+        if (o.bex) { seed_b<R, F>(f, g, xe, b); o.bex[i] = b[0]; o.bey[i] = b[1]; o.bez[i] = b[2]; }
+        if (o.btx || o.bflag) {
+            seed_b<R, F>(f, g, p0, b);
+            if (o.btx) { o.btx[i] = b[0]; o.bty[i] = b[1]; o.btz[i] = b[2]; }
+            if (o.bflag) o.bflag[i] = b_flag(b, P);
+        }
+    }
 }
 
 // ------------------------------------------------------------- launching
@@ -1784,17 +1831,27 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
 // a second one.
 constexpr int kPlainSpread = 2;
 // Both schedules run the same kernels; a line's result does not depend on which
-// lanes trace it.  `n_hint` is the number of lines (the capacity of the arrays
+// lanes trace it.  Outputs on the seed arrays are traced one thread per line.  `n_hint` is the number of lines (the capacity of the arrays
 // where ds.n_dev holds fewer); where ds.N holds it on the device, only a cap.
 template <typename R, class F, class FJ = NoCurrent, class G = UniformGrid>
 static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsigned long long n, const PlainOut& o,
                         const DevScalars& ds, const float* ncross, int schedule, hipStream_t st,
                         unsigned long long n_hint, const FJ& fj = FJ{}, const G& g = G{}) {
     (void)schedule;
+    const int lds = grid_lds_bytes(g);
+    const void* const seeds[] = {s.x, s.y, s.z};
+    const void* const outs[] = {o.sx, o.sy, o.sz, o.ex, o.ey, o.ez, o.fs, o.fe, o.btx, o.bty, o.btz, o.bflag,
+                                o.bsx, o.bsy, o.bsz, o.bex, o.bey, o.bez, o.evals};
+    if (plain_in_place(seeds, 3, outs, sizeof(outs) / sizeof(outs[0]))) {
+        int rc = record_start(st);
+        if (rc) return rc;
+        k_plain_lines<R, F, FJ, G><<<per_line_grid(n_hint, 256, ds), 256, lds, st>>>(f, P, s, n, o, ds, ncross, fj, g);
+        HIP_TRY(hipGetLastError());
+        return record_end(st);
+    }
     unsigned long long* q = nullptr;
     int rc = queue_slot(&q);
     if (rc) return rc;
-    const int lds = grid_lds_bytes(g);
     // The tangent lines of a large RKF45 launch are listed in a workspace of
     // 5 bytes a line; a capturing stream takes no allocation and traces by quads.
     TangentLines tl{nullptr, nullptr, q + 2};

@@ -20,7 +20,10 @@
 // (each starts from the seed with the initial step), so they are separate
 // tasks of the queue.  Every value is formed by the same expression on the same
 // operands as in the one-thread-per-line code of fqsl_tracer.h /
-// fqsl_stretch.h, which the CPU tests build.
+// fqsl_stretch.h, which the CPU tests build.  FP32 lines have the same bits; of
+// FP64 lines on uniform grids, where the compiler fuses products and sums in
+// another order, one length in twenty differs in its last place; and the twists
+// of the two sides are summed apart, not one after the other.
 #pragma once
 
 #include "fqsl_stretch.h"

@@ -25,6 +25,18 @@ inline unsigned long long plain_listed_lines(bool rkf45, unsigned long long line
     return list ? lines : 0ull;
 }
 
+// Whether a plain trace writes a result where it reads its seeds.  The forward
+// and the backward side of a line are separate tasks, each of which reads the
+// seed when it begins, and the outputs that belong to the line are written
+// before either: only one thread that traces both sides, and writes when they
+// have ended, may overwrite them.
+inline bool plain_in_place(const void* const* seeds, int nseeds, const void* const* out, int nout) {
+    for (int i = 0; i < nout; ++i)
+        for (int k = 0; k < nseeds; ++k)
+            if (out[i] && out[i] == seeds[k]) return true;
+    return false;
+}
+
 // Consecutive requests of a batch and their lines: those of one layout, which a
 // launch by quads takes together, or of one field and method, which a launch by
 // lanes takes.  `counter` is the work counter of that launch.  Layouts of one

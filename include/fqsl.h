@@ -338,7 +338,10 @@ typedef struct {
 } fqsl_plain_out;
 
 /* Position-only tracing of n seeds, forward then backward.  Replaces a launch
- * of TraceAllBline (TraceBlineAdaptive.cu:429-510, TraceBline.cu:383-464). */
+ * of TraceAllBline (TraceBlineAdaptive.cu:429-510, TraceBline.cu:383-464).
+ * Arrays of 4-byte results may be the seed arrays themselves (the same start;
+ * here, in fqsl_trace_plain_n and in the reference-shaped entries): such a call
+ * runs one thread per line. */
 int fqsl_trace_plain(const fqsl_field *field, const fqsl_plain_params *params, uint64_t n,
                      const float *x, const float *y, const float *z, const fqsl_plain_out *out,
                      void *stream);

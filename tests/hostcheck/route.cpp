@@ -31,3 +31,7 @@ extern "C" int rt_batch_groups(int nreq, const int* kind, const char* other, con
     fqsl::batch_spans(nreq, kind, other, n, layouts, groups);
     return (int)groups.size();
 }
+
+extern "C" int rt_plain_in_place(const void* const* seeds, int nseeds, const void* const* out, int nout) {
+    return fqsl::plain_in_place(seeds, nseeds, out, nout) ? 1 : 0;
+}

@@ -54,3 +54,12 @@ def test_launches_of_a_batch_share_no_counter(route, quad_lines, seed):
     assert list(first) == sorted(first) and first[0] == 0
     edges = list(first) + [m]
     assert [n[a:b].sum() for a, b in zip(edges[:-1], edges[1:])] == list(lines)
+
+
+@pytest.mark.parametrize("out,expected", [([], 0), ([0, 0], 0), ([40, 0, 50], 0), ([10], 1), ([0, 40, 30], 1),
+                                          ([40, 20, 50], 1), ([11, 14], 0)])
+def test_results_over_the_seeds_are_seen(route, out, expected):
+    """Addresses of the result arrays against seeds at 10, 20 and 30; 0 is NULL."""
+    seeds = (ctypes.c_void_p * 3)(10, 20, 30)
+    arr = (ctypes.c_void_p * max(1, len(out)))(*out)
+    assert route.rt_plain_in_place(seeds, 3, arr, len(out)) == expected
