@@ -9,7 +9,8 @@
 //   k_scott_per_line       Scott tracer, one thread per line
 //   k_plain_quads / k_plain_sides   position-only tracer (grid-index
 //                          coordinates, or a stretched grid's own coordinates)
-//   k_plain_lines          the same, one thread per line: results over the seeds
+//   k_plain_lines          the same, one thread per line: results over the
+//                          seeds, captured per-line launches
 //   k_qcalc_plane          QCalcPlane (FastQSL.py:65-117)
 //   k_pseudo_*             CookPseudoLine compaction (FastQSL.py:4-57)
 //   k_qcut_scatter         Qcut + merge (demo/Q_RKF45CuPy.ipynb cells [10]-[11])
@@ -1479,8 +1480,8 @@ k_plain_sides(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, Dev
 }
 
 // One thread per line, which reads the seed once and writes the line's outputs
-// when both its sides have ended: for calls whose outputs lie on their seeds.
-// One line a thread is the slowest way to trace (1024^2 lines on a stretched
+// when both its sides have ended: for calls whose outputs lie on their seeds, and
+// for captured per-line launches (plain_by_lines).  One line a thread is the slowest way to trace (1024^2 lines on a stretched
 // 256^3 grid 14.0 ms, 5.6 by k_plain_sides).  Two wavefronts per SIMD as the
 // register target: the FP64 variants otherwise run one (1.2-1.3 times slower).
 template <typename R, class F, class FJ, class G>
@@ -1830,19 +1831,25 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
 // Wavefronts per SIMD over which few sides are spread before a wavefront takes
 // a second one.
 constexpr int kPlainSpread = 2;
+
 // Both schedules run the same kernels; a line's result does not depend on which
-// lanes trace it.  Outputs on the seed arrays are traced one thread per line.  `n_hint` is the number of lines (the capacity of the arrays
-// where ds.n_dev holds fewer); where ds.N holds it on the device, only a cap.
+// lanes trace it.  Outputs on the seed arrays, and the per-line schedule on a
+// capturing stream, are traced one thread per line.  `n_hint` is the number of
+// lines (the capacity of the arrays where ds.n_dev holds fewer); where ds.N holds
+// it on the device, only a cap.
 template <typename R, class F, class FJ = NoCurrent, class G = UniformGrid>
 static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsigned long long n, const PlainOut& o,
                         const DevScalars& ds, const float* ncross, int schedule, hipStream_t st,
                         unsigned long long n_hint, const FJ& fj = FJ{}, const G& g = G{}) {
-    (void)schedule;
     const int lds = grid_lds_bytes(g);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(st, &cap));
+    const bool capturing = cap != hipStreamCaptureStatusNone;
     const void* const seeds[] = {s.x, s.y, s.z};
     const void* const outs[] = {o.sx, o.sy, o.sz, o.ex, o.ey, o.ez, o.fs, o.fe, o.btx, o.bty, o.btz, o.bflag,
                                 o.bsx, o.bsy, o.bsz, o.bex, o.bey, o.bez, o.evals};
-    if (plain_in_place(seeds, 3, outs, sizeof(outs) / sizeof(outs[0]))) {
+    const bool in_place = plain_in_place(seeds, 3, outs, sizeof(outs) / sizeof(outs[0]));
+    if (plain_by_lines(in_place, schedule == FQSL_SCHED_PER_LINE, capturing)) {
         int rc = record_start(st);
         if (rc) return rc;
         k_plain_lines<R, F, FJ, G><<<per_line_grid(n_hint, 256, ds), 256, lds, st>>>(f, P, s, n, o, ds, ncross, fj, g);
@@ -1857,14 +1864,10 @@ static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsign
     TangentLines tl{nullptr, nullptr, q + 2};
     char* ws = nullptr;
     const unsigned long long listed = plain_listed_lines(P.method == kRKF45, n_hint, !ds.N);
-    if (listed) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        HIP_TRY(hipStreamIsCapturing(st, &cap));
-        if (cap == hipStreamCaptureStatusNone) {
-            HIP_TRY(hipMallocAsync((void**)&ws, 5 * (size_t)listed, st));
-            tl.list = (unsigned*)ws;
-            tl.marked = (unsigned char*)ws + 4 * (size_t)listed;
-        }
+    if (listed && !capturing) {
+        HIP_TRY(hipMallocAsync((void**)&ws, 5 * (size_t)listed, st));
+        tl.list = (unsigned*)ws;
+        tl.marked = (unsigned char*)ws + 4 * (size_t)listed;
     }
     int grid = 0;
     rc = tl.list ? persistent_grid(k_plain_sides<R, F, FJ, G>, &grid, lds)

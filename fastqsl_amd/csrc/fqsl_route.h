@@ -37,6 +37,14 @@ inline bool plain_in_place(const void* const* seeds, int nseeds, const void* con
     return false;
 }
 
+// Whether a plain trace runs one thread per line.  The other kernels draw their
+// work from a counter in a ring that later launches share; a captured launch
+// keeps its counter, and a replay may meet a launch that the ring has come round
+// to.  The per-line schedule has no such counter to be captured.
+inline bool plain_by_lines(bool in_place, bool per_line, bool capturing) {
+    return in_place || (per_line && capturing);
+}
+
 // Consecutive requests of a batch and their lines: those of one layout, which a
 // launch by quads takes together, or of one field and method, which a launch by
 // lanes takes.  `counter` is the work counter of that launch.  Layouts of one

@@ -51,7 +51,9 @@ extern "C" {
                              stage points, stage positions, increments, error norm), controller and Q */
 
 /* how lines are mapped to lanes */
-/* The Scott tracer's schedules; the plain tracers take either and run the same kernels. */
+/* The Scott tracer's schedules; the plain tracers take either and run the same kernels
+ * (on a capturing stream FQSL_SCHED_PER_LINE runs one thread per line, whose graph needs
+ * no work counter of the library; a persistent launch keeps the one it was captured with). */
 #define FQSL_SCHED_PERSISTENT 0 /* persistent grid, each lane refills from a device queue */
 #define FQSL_SCHED_PER_LINE 1   /* one thread per line, one launch */
 

@@ -35,3 +35,7 @@ extern "C" int rt_batch_groups(int nreq, const int* kind, const char* other, con
 extern "C" int rt_plain_in_place(const void* const* seeds, int nseeds, const void* const* out, int nout) {
     return fqsl::plain_in_place(seeds, nseeds, out, nout) ? 1 : 0;
 }
+
+extern "C" int rt_plain_by_lines(int in_place, int per_line, int capturing) {
+    return fqsl::plain_by_lines(in_place != 0, per_line != 0, capturing != 0) ? 1 : 0;
+}

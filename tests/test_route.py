@@ -63,3 +63,11 @@ def test_results_over_the_seeds_are_seen(route, out, expected):
     seeds = (ctypes.c_void_p * 3)(10, 20, 30)
     arr = (ctypes.c_void_p * max(1, len(out)))(*out)
     assert route.rt_plain_in_place(seeds, 3, arr, len(out)) == expected
+
+
+def test_captured_per_line_launches_hold_no_work_counter(route):
+    for in_place in (0, 1):
+        for per_line in (0, 1):
+            for capturing in (0, 1):
+                got = route.rt_plain_by_lines(in_place, per_line, capturing)
+                assert got == (1 if in_place or (per_line and capturing) else 0)
