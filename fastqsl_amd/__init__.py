@@ -10,13 +10,13 @@ host side that keeps the ``fastqslpy`` entry points:
 * ``Field``, ``trace_scott``, ``trace_plain`` -- the direct API
 """
 from ._lib import FqslError, lib, last_kernel_ms
-from .field import Field
+from .field import Field, release_field_memory
 from .trace import trace_plain, trace_scott
 from . import synth
 
 __version__ = "0.1.0"
 
-__all__ = ["Field", "trace_scott", "trace_plain", "FqslError", "lib", "last_kernel_ms", "synth",
+__all__ = ["Field", "trace_scott", "trace_plain", "FqslError", "lib", "last_kernel_ms", "release_field_memory", "synth",
            "kernels", "FastQSL"]
 
 

@@ -80,6 +80,7 @@ PROTOTYPES = {
     "fqsl_version": (ctypes.c_char_p, []),
     "fqsl_field_create": (i32, [vp, vp, vp, i32, i32, i32, i32, i32, i32, ctypes.POINTER(vp)]),
     "fqsl_field_destroy": (i32, [vp]),
+    "fqsl_field_memory_trim": (i32, [ctypes.c_size_t, ctypes.POINTER(ctypes.c_size_t)]),
     "fqsl_field_bytes": (ctypes.c_size_t, [vp]),
     "fqsl_field_shape": (i32, [vp, ctypes.POINTER(i32), ctypes.POINTER(i32), ctypes.POINTER(i32)]),
     "fqsl_field_set_current": (i32, [vp, vp, vp, vp, i32, i32]),

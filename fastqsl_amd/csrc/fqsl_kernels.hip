@@ -174,10 +174,12 @@ static int grid_for(long n, int block) {
 // Device memory of fields.  A series of snapshots creates and destroys fields
 // of one size, and allocating gigabytes costs far more than filling them: the
 // driver clears memory that was in use before (a 320 x 320 x 256 field created,
-// mapped at 256^2 and destroyed over and over: 119.9 ms, 6.0 with the blocks kept).  Blocks of destroyed fields are therefore kept for the next ones:
-// at most kFieldCacheBytes per device, the oldest given back first, all of them
-// when an allocation fails, and only blocks of 1 MiB and more.  A block is
-// reused for requests it exceeds by less than an eighth.
+// mapped at 256^2 and destroyed over and over: 119.9 ms, 6.0 with the blocks
+// kept).  Blocks of destroyed fields are therefore kept for the next ones: at most
+// kFieldCacheBytes per device, the oldest given back first, all of them when an
+// allocation of this library finds no memory or fqsl_field_memory_trim asks for
+// them, and only blocks of 1 MiB and more.  A block is reused for requests it
+// exceeds by less than an eighth.
 constexpr size_t kFieldCacheBytes = 8ull << 30;
 constexpr size_t kFieldCacheMin = 1u << 20;
 struct FieldBlock {
@@ -195,7 +197,8 @@ static std::unordered_map<void*, size_t>& field_sizes() {  // blocks in use that
     return *m;
 }
 
-static void field_cache_drop(int device, size_t keep) {  // the lock is held
+// Frees what exceeds `keep` bytes; returns the bytes still held.  The lock is held.
+static size_t field_cache_drop(int device, size_t keep, bool* freed = nullptr) {
     size_t held = 0;
     std::vector<FieldBlock>& c = field_cache();
     for (size_t i = c.size(); i-- > 0;) {
@@ -205,14 +208,46 @@ static void field_cache_drop(int device, size_t keep) {  // the lock is held
             held -= c[i].bytes;
             (void)hipFree(c[i].ptr);
             c.erase(c.begin() + i);
+            if (freed) *freed = true;
         }
     }
+    return held;
+}
+
+extern "C" int fqsl_field_memory_trim(size_t keep_bytes, size_t* held_bytes) {
+    int dev = 0;
+    HIP_TRY(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(g_field_mu);
+    const size_t held = field_cache_drop(dev, keep_bytes);
+    if (held_bytes) *held_bytes = held;
+    return FQSL_OK;
+}
+
+// Every allocation of this library but a field's own: one that finds no memory is
+// tried again with the kept blocks given back.  (hipFree waits for the device.)
+static bool field_cache_give_back() {
+    (void)hipGetLastError();
+    int dev = 0;
+    bool freed = false;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lk(g_field_mu);
+    field_cache_drop(dev, 0, &freed);
+    return freed;
+}
+template <typename T>
+static hipError_t dev_malloc(T** out, size_t bytes) {
+    return alloc_or_give_back(hipErrorOutOfMemory, [&] { return hipMalloc((void**)out, bytes); }, field_cache_give_back);
+}
+template <typename T>
+static hipError_t dev_malloc_async(T** out, size_t bytes, hipStream_t st) {
+    return alloc_or_give_back(hipErrorOutOfMemory, [&] { return hipMallocAsync((void**)out, bytes, st); },
+                              field_cache_give_back);
 }
 
 template <typename T>
 static hipError_t field_malloc(int device, T** out, size_t bytes) {
     *out = nullptr;
-    if (bytes < kFieldCacheMin) return hipMalloc((void**)out, bytes);
+    if (bytes < kFieldCacheMin) return dev_malloc(out, bytes);
     std::lock_guard<std::mutex> lk(g_field_mu);
     std::vector<FieldBlock>& c = field_cache();
     int best = -1;
@@ -227,13 +262,15 @@ static hipError_t field_malloc(int device, T** out, size_t bytes) {
         got = c[best].bytes;
         c.erase(c.begin() + best);
     } else {
-        hipError_t e = hipMalloc(&p, bytes);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            field_cache_drop(device, 0);
-            e = hipMalloc(&p, bytes);
-            if (e != hipSuccess) return e;
-        }
+        bool freed = false;
+        const hipError_t e = alloc_or_give_back(
+            hipErrorOutOfMemory, [&] { return hipMalloc(&p, bytes); },
+            [&] {
+                (void)hipGetLastError();
+                field_cache_drop(device, 0, &freed);
+                return freed;
+            });
+        if (e != hipSuccess) return e;
     }
     field_sizes()[p] = got;
     *out = (T*)p;
@@ -477,7 +514,7 @@ static int build_stretch(const std::vector<double> (&a)[3], const int* n, int ru
     }
     memcpy(host.data() + offc, compact.data(), compact.size() * sizeof(uint2));
     char* d = nullptr;
-    HIP_TRY(hipMalloc(&d, total));
+    HIP_TRY(dev_malloc(&d, total));
     const void* rec64[3] = {d + off64[0], d + off64[1], d + off64[2]};
     const void* rec32[3] = {d + off32[0], d + off32[1], d + off32[2]};
     const int* ref[3] = {(const int*)(d + offr[0]), (const int*)(d + offr[1]), (const int*)(d + offr[2])};
@@ -605,7 +642,7 @@ static int queue_slot(unsigned long long** slot) {
     if ((int)g_queues.size() <= dev) g_queues.resize(dev + 1);
     DeviceQueues& d = g_queues[dev];
     if (!d.slots) {
-        HIP_TRY(hipMalloc(&d.slots, (size_t)kQueueSlots * kQueueSlotWidth * sizeof(unsigned long long)));
+        HIP_TRY(dev_malloc(&d.slots, (size_t)kQueueSlots * kQueueSlotWidth * sizeof(unsigned long long)));
         HIP_TRY(hipMemset(d.slots, 0, (size_t)kQueueSlots * kQueueSlotWidth * sizeof(unsigned long long)));
     }
     *slot = d.slots + (size_t)kQueueSlotWidth * (d.next++ % kQueueSlots);
@@ -1805,7 +1842,7 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
         rc = queue_slot(&q);
         if (rc) return rc;
         void* ws = nullptr;
-        HIP_TRY(hipMallocAsync(&ws, w.bytes, st));
+        HIP_TRY(dev_malloc_async(&ws, w.bytes, st));
         const hipError_t e = scott_persistent_launches<R, F, FJ, X>(f, P, s, n, o, ds, st, n_hint, fj, (char*)ws,
                                                                     w, ordered, q, step, true, pairs);
         const hipError_t ef = hipFreeAsync(ws, st);
@@ -1865,9 +1902,13 @@ static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsign
     char* ws = nullptr;
     const unsigned long long listed = plain_listed_lines(P.method == kRKF45, n_hint, !ds.N);
     if (listed && !capturing) {
-        HIP_TRY(hipMallocAsync((void**)&ws, 5 * (size_t)listed, st));
-        tl.list = (unsigned*)ws;
-        tl.marked = (unsigned char*)ws + 4 * (size_t)listed;
+        if (dev_malloc_async(&ws, 5 * (size_t)listed, st) == hipSuccess) {
+            tl.list = (unsigned*)ws;
+            tl.marked = (unsigned char*)ws + 4 * (size_t)listed;
+        } else {  // no room: by quads too
+            (void)hipGetLastError();
+            ws = nullptr;
+        }
     }
     int grid = 0;
     rc = tl.list ? persistent_grid(k_plain_sides<R, F, FJ, G>, &grid, lds)
@@ -2790,7 +2831,7 @@ extern "C" int fqsl_qmap_plane(const fqsl_field* field, const fqsl_plane* plane,
     if (n == 0) return FQSL_OK;
     hipStream_t st = (hipStream_t)stream;
     float* seeds = nullptr;
-    HIP_TRY(hipMallocAsync((void**)&seeds, 3 * sizeof(float) * n, st));
+    HIP_TRY(dev_malloc_async(&seeds, 3 * sizeof(float) * n, st));
     k_plane_seeds<<<grid_for((long)n, 256), 256, 0, st>>>(*plane, seeds, seeds + n, seeds + 2 * n);
     hipError_t e = hipGetLastError();
     int rc = e == hipSuccess ? fqsl_trace_scott(field, params, n, seeds, seeds + n, seeds + 2 * n, out, stream)
@@ -2830,7 +2871,7 @@ extern "C" int fqsl_qmap_plane_neighbour(const fqsl_field* field, const fqsl_pla
     const size_t o_pout = take(32 * sizeof(float) * n);
     hipStream_t st = (hipStream_t)stream;
     char* ws = nullptr;
-    HIP_TRY(hipMallocAsync((void**)&ws, off, st));
+    HIP_TRY(dev_malloc_async(&ws, off, st));
     float* sd = (float*)(ws + o_seed);
     float* m = (float*)(ws + o_main);  // 18 arrays of n: start xyz, end xyz, flags, b_this xyz, b_flag, b_start xyz, b_end xyz
     float *sx = m, *sy = m + n, *sz = m + 2 * n, *ex = m + 3 * n, *ey = m + 4 * n, *ez = m + 5 * n;
@@ -2937,7 +2978,7 @@ static int server_trace(fqsl_server* S, const std::vector<ServerReq>& take) {
         if (S->ws) HIP_TRY(hipFree(S->ws));
         S->ws = nullptr;
         S->ws_bytes = 0;
-        HIP_TRY(hipMalloc(&S->ws, need));
+        HIP_TRY(dev_malloc(&S->ws, need));
         S->ws_bytes = need;
     }
     fqsl_scott_batch* b = nullptr;
@@ -3689,7 +3730,7 @@ extern "C" int fqsl_pseudo_seeds(uint64_t n, const int32_t* b_flag, const float*
     hipStream_t st = (hipStream_t)stream;
     const size_t wsb = pseudo_ws_bytes(n);
     void* ws = nullptr;
-    HIP_TRY(hipMallocAsync(&ws, wsb + 2 * sizeof(unsigned long long), st));
+    HIP_TRY(dev_malloc_async(&ws, wsb + 2 * sizeof(unsigned long long), st));
     unsigned long long* total = (unsigned long long*)((char*)ws + wsb);
     rc = pseudo_launch(n, b_flag, x_start, y_start, z_start, flag_start, bz_start, bz_end, stride, capacity, seed_x,
                        seed_y, seed_z, bz0_start, bz0_end, pixel, total, ws, st);
@@ -3861,7 +3902,7 @@ extern "C" int fqsl_bad_pixels(uint64_t n, const int32_t* b_flag, const float* q
     // block counts and the total in one stream-ordered allocation
     const size_t counts_bytes = align256((size_t)nblocks * sizeof(unsigned) + 16);
     unsigned* counts = nullptr;
-    HIP_TRY(hipMallocAsync((void**)&counts, counts_bytes + sizeof(unsigned long long), st));
+    HIP_TRY(dev_malloc_async(&counts, counts_bytes + sizeof(unsigned long long), st));
     unsigned long long* total = (unsigned long long*)((char*)counts + counts_bytes);
     k_bad_count<<<nblocks, kCompactBlock, 0, st>>>(n, b_flag, q, counts);
     k_pseudo_scan<<<1, 1024, 0, st>>>(nblocks, counts, total);

@@ -74,4 +74,13 @@ inline void batch_spans(int nreq, const int* kind, const char* other, const unsi
     }
 }
 
+// An allocation that may find the memory in what the library keeps: `alloc` is
+// tried again when it fails for want of memory (`full`) and `give_back` has freed
+// some.
+template <typename E, class Alloc, class GiveBack>
+E alloc_or_give_back(E full, Alloc alloc, GiveBack give_back) {
+    const E e = alloc();
+    return e == full && give_back() ? alloc() : e;
+}
+
 }  // namespace fqsl

@@ -148,6 +148,16 @@ class Field:
         self.close()
 
 
+def release_field_memory(keep: int = 0) -> int:
+    """Free what the library keeps of closed fields' memory on the current
+    device (up to 8 GiB, for the next fields) beyond ``keep`` bytes; returns the
+    bytes still kept.  Its own allocations find that memory by themselves, torch's
+    cannot."""
+    held = ctypes.c_size_t()
+    _lib.check(_lib.lib().fqsl_field_memory_trim(int(keep), ctypes.byref(held)))
+    return int(held.value)
+
+
 def _maybe_torch(x):
     try:
         import torch

@@ -78,8 +78,14 @@ int fqsl_field_create(const void *bx, const void *by, const void *bz, int nx, in
 /* Waits for the device.  Up to 8 GiB per device of the layouts' memory is kept
  * for the next fields (fields of a time series have one size, and allocating
  * gigabytes anew costs far more than filling them); it is given back when an
- * allocation for a field fails or other fields' memory takes its place. */
+ * allocation of this library finds no memory, when other fields' memory takes its
+ * place, or by fqsl_field_memory_trim. */
 int fqsl_field_destroy(fqsl_field *field);
+/* Frees what is kept of destroyed fields' memory on the current device beyond
+ * keep_bytes (0: all), for other allocators of the process, which cannot ask for
+ * it; *held_bytes (may be NULL) receives the bytes still kept.  Waits for the
+ * device if it frees any. */
+int fqsl_field_memory_trim(size_t keep_bytes, size_t *held_bytes);
 /* Device bytes held by the field's layouts. */
 size_t fqsl_field_bytes(const fqsl_field *field);
 int fqsl_field_shape(const fqsl_field *field, int *nx, int *ny, int *nz);

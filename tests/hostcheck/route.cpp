@@ -39,3 +39,11 @@ extern "C" int rt_plain_in_place(const void* const* seeds, int nseeds, const voi
 extern "C" int rt_plain_by_lines(int in_place, int per_line, int capturing) {
     return fqsl::plain_by_lines(in_place != 0, per_line != 0, capturing != 0) ? 1 : 0;
 }
+
+// An allocator that fails with `code` until its `ok_at`-th call, with blocks to give back or
+// none; returns the code of the last call and how often it was called.
+extern "C" int rt_alloc_or_give_back(int full, int code, int ok_at, int has_blocks, int* calls) {
+    *calls = 0;
+    return fqsl::alloc_or_give_back(
+        full, [&] { return ++*calls >= ok_at ? 0 : code; }, [&] { return has_blocks != 0; });
+}

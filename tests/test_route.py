@@ -1,6 +1,7 @@
 """The rules by which a call picks its kernels and sizes its memory (host code)."""
 import ctypes
 import os
+import re
 import subprocess
 
 import numpy as np
@@ -71,3 +72,24 @@ def test_captured_per_line_launches_hold_no_work_counter(route):
             for capturing in (0, 1):
                 got = route.rt_plain_by_lines(in_place, per_line, capturing)
                 assert got == (1 if in_place or (per_line and capturing) else 0)
+
+
+@pytest.mark.parametrize("code,ok_at,has_blocks,expected,calls", [
+    (2, 1, 1, 0, 1),    # there is room
+    (2, 2, 1, 0, 2),    # room once the kept blocks are given back
+    (2, 3, 1, 2, 2),    # not even then
+    (2, 2, 0, 2, 1),    # nothing to give back
+    (7, 2, 1, 7, 1),    # another error
+])
+def test_allocations_find_kept_memory(route, code, ok_at, has_blocks, expected, calls):
+    n = ctypes.c_int()
+    assert route.rt_alloc_or_give_back(2, code, ok_at, has_blocks, ctypes.byref(n)) == expected
+    assert n.value == calls
+
+
+def test_every_device_allocation_may_find_kept_memory():
+    src = open(os.path.join(ROOT, "fastqsl_amd", "csrc", "fqsl_kernels.hip")).read()
+    src = re.sub(r"//[^\n]*|\"[^\"\n]*\"", "", src)
+    bare = re.findall(r"[^\n]*\bhipMalloc(?:Async|Managed|FromPoolAsync)?\([^\n]*", src)
+    inside = [l for l in bare if "return hipMalloc" in l and "[&] {" in l]
+    assert len(inside) == 3 and bare == inside, bare
