@@ -186,6 +186,7 @@ struct FieldBlock {
     int device;
     void* ptr;
     size_t bytes;
+    hipEvent_t ready;  // recorded behind the work that still uses the block; NULL: none does
 };
 static std::mutex g_field_mu;
 static std::vector<FieldBlock>& field_cache() {  // oldest first; not destroyed at exit, when HIP may be gone
@@ -206,6 +207,10 @@ static size_t field_cache_drop(int device, size_t keep, bool* freed = nullptr) {
         held += c[i].bytes;
         if (held > keep) {
             held -= c[i].bytes;
+            if (c[i].ready) {
+                (void)hipEventSynchronize(c[i].ready);
+                (void)hipEventDestroy(c[i].ready);
+            }
             (void)hipFree(c[i].ptr);
             c.erase(c.begin() + i);
             if (freed) *freed = true;
@@ -251,15 +256,22 @@ static hipError_t field_malloc(int device, T** out, size_t bytes) {
     std::lock_guard<std::mutex> lk(g_field_mu);
     std::vector<FieldBlock>& c = field_cache();
     int best = -1;
-    for (int i = 0; i < (int)c.size(); ++i)
-        if (c[i].device == device && c[i].bytes >= bytes && c[i].bytes - bytes <= bytes / 8 &&
-            (best < 0 || c[i].bytes < c[best].bytes))
-            best = i;
+    for (int i = 0; i < (int)c.size(); ++i) {
+        if (c[i].device != device || c[i].bytes < bytes || c[i].bytes - bytes > bytes / 8 ||
+            (best >= 0 && c[i].bytes >= c[best].bytes))
+            continue;
+        if (c[i].ready && hipEventQuery(c[i].ready) != hipSuccess) {
+            (void)hipGetLastError();  // still in use: not an error of this call
+            continue;
+        }
+        best = i;
+    }
     void* p = nullptr;
     size_t got = bytes;
     if (best >= 0) {
         p = c[best].ptr;
         got = c[best].bytes;
+        if (c[best].ready) (void)hipEventDestroy(c[best].ready);
         c.erase(c.begin() + best);
     } else {
         bool freed = false;
@@ -277,34 +289,49 @@ static hipError_t field_malloc(int device, T** out, size_t bytes) {
     return hipSuccess;
 }
 
-// As hipFree, which waits for the device before the memory can be used again;
-// `done`: the work that used it is known to have ended.
-static void field_release(int device, void* p, bool done = false) {
-    if (!p) return;
-    size_t bytes = 0;
-    {
-        std::lock_guard<std::mutex> lk(g_field_mu);
-        auto it = field_sizes().find(p);
-        if (it != field_sizes().end()) {
-            bytes = it->second;
-            field_sizes().erase(it);
-        }
-    }
-    int cur = -1;
-    if (bytes == 0 || bytes > kFieldCacheBytes || hipGetDevice(&cur) != hipSuccess ||
-        (cur != device && hipSetDevice(device) != hipSuccess)) {
-        (void)hipFree(p);
-        return;
-    }
-    const hipError_t e = done ? hipSuccess : hipDeviceSynchronize();
-    if (cur != device) (void)hipSetDevice(cur);
-    if (e != hipSuccess) {
-        (void)hipFree(p);
-        return;
-    }
+// The size of a block that may be kept, which is then no longer in use; 0: of another.
+static size_t field_block_bytes(void* p) {
     std::lock_guard<std::mutex> lk(g_field_mu);
-    field_cache().push_back(FieldBlock{device, p, bytes});
+    auto it = field_sizes().find(p);
+    if (it == field_sizes().end()) return 0;
+    const size_t bytes = it->second;
+    field_sizes().erase(it);
+    return bytes <= kFieldCacheBytes ? bytes : 0;
+}
+static void field_keep(int device, void* p, size_t bytes, hipEvent_t ready) {
+    std::lock_guard<std::mutex> lk(g_field_mu);
+    field_cache().push_back(FieldBlock{device, p, bytes, ready});
     field_cache_drop(device, kFieldCacheBytes);
+}
+
+// As hipFree, which waits for the device before the memory can be used again.
+static void field_release(int device, void* p) {
+    if (!p) return;
+    const size_t bytes = field_block_bytes(p);
+    int cur = -1;
+    if (bytes == 0 || hipGetDevice(&cur) != hipSuccess || (cur != device && hipSetDevice(device) != hipSuccess)) {
+        (void)hipFree(p);
+        return;
+    }
+    const hipError_t e = hipDeviceSynchronize();
+    if (cur != device) (void)hipSetDevice(cur);
+    if (e == hipSuccess) field_keep(device, p, bytes, nullptr);
+    else (void)hipFree(p);
+}
+
+// The same for memory of the current device that only the work enqueued on `st`
+// uses, without a wait: the next owner is found once that work has ended.
+static void field_release_after(int device, void* p, hipStream_t st) {
+    const size_t bytes = field_block_bytes(p);
+    hipEvent_t ready = nullptr;
+    if (bytes && hipEventCreateWithFlags(&ready, hipEventDisableTiming) == hipSuccess) {
+        if (hipEventRecord(ready, st) == hipSuccess) {
+            field_keep(device, p, bytes, ready);
+            return;
+        }
+        (void)hipEventDestroy(ready);
+    }
+    (void)hipFree(p);
 }
 
 static void build_cells(const void* const* b, int dtype, const int* n, float4* cells) {
@@ -3315,11 +3342,7 @@ extern "C" int fqsl_TraceAllBlineScott(float* Bx, float* By, float* Bz, int* Bsh
                  ? launch_scott<float, FieldSoA<float>, NoCurrent, double>(f, P, s, n, o, ds, schedule, st, n_hint, nullptr)
                  : launch_scott<float>(f, P, s, n, o, ds, schedule, st, n_hint, nullptr, NoCurrent{}, pairs);
     }
-    if (pairs) {  // other streams may take the block once this one is done with it
-        const hipError_t e = hipStreamSynchronize(st);
-        field_release(dev, pairs, e == hipSuccess);
-        if (rc == FQSL_OK && e != hipSuccess) return set_err(FQSL_ERR_HIP, "Scott trace: %s", hipGetErrorString(e));
-    }
+    if (pairs) field_release_after(dev, pairs, st);
     return rc;
 }
 
