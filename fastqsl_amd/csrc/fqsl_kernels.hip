@@ -653,7 +653,8 @@ extern "C" int fqsl_tune_get(int knob, int* value) {
 // clears it with a fill kernel on its stream before the persistent launch.
 // Calls that are more than kQueueSlots launches apart never share a slot.
 static constexpr int kQueueSlots = 4096;
-static constexpr int kQueueSlotWidth = 8;  // counters per slot (one per XCD queue)
+static constexpr int kQueueSlotWidth = 16;  // words per slot: a counter per XCD queue, then the votes
+static constexpr int kSlotVotes = 8;
 struct DeviceQueues {
     unsigned long long* slots = nullptr;
     unsigned next = 0;
@@ -915,11 +916,34 @@ __global__ void __launch_bounds__(256) k_order_predict(F f, Seeds s, unsigned lo
         if (hist[t]) atomicAdd(&counts[t], hist[t]);
 }
 
-// Exclusive scan of the bucket counts (one block).
-__global__ void __launch_bounds__(kOrderBuckets) k_order_scan(unsigned* counts) {
+// Where the launch's own lines tell which of two kernels traces them faster, both
+// are launched and one returns at once (2-3 us): the second where `votes` is
+// positive, the first elsewhere.  votes == NULL: only one was launched.
+struct Pick {
+    const unsigned long long* votes;
+};
+__device__ __forceinline__ bool picked(const Pick& p, bool second) {
+    return !p.votes || ((long long)p.votes[0] > 0) == second;
+}
+
+// Exclusive scan of the bucket counts (one block).  With `votes`, whether the
+// estimated lengths add up to more than `work` times the longest one.
+__global__ void __launch_bounds__(kOrderBuckets) k_order_scan(unsigned* counts, int nbuckets, unsigned long long* votes,
+                                                              unsigned long long work) {
     __shared__ unsigned v[kOrderBuckets];
     v[threadIdx.x] = counts[threadIdx.x];
     __syncthreads();
+    if (threadIdx.x == 0 && votes) {
+        unsigned long long sum = 0, longest = 0;
+        for (int t = 0; t < nbuckets; ++t) {
+            // in half buckets, without the estimate's two steps that leave the box
+            const int half = 2 * (nbuckets - 1 - t) + 1 - 2 * nbuckets / kPredSteps;
+            const unsigned long long len = half < 1 ? 1ull : (unsigned long long)half;
+            if (v[t] && !longest) longest = len;
+            sum += v[t] * len;
+        }
+        votes[0] = sum > work * longest ? 1ull : 0ull;
+    }
     if (threadIdx.x == 0) {
         unsigned acc = 0;
         for (int t = 0; t < kOrderBuckets; ++t) {
@@ -1039,7 +1063,8 @@ template <typename R, class F, class FJ, typename X>
 __global__ void __launch_bounds__(256) k_scott_persistent(F f, ScottParams P, Seeds s, unsigned long long n,
                                                           const R* frames, ScottRec<R>* recs, DevScalars ds,
                                                           unsigned long long* queues, int nq, int refill_min,
-                                                          const unsigned* order, FJ fj) {
+                                                          const unsigned* order, FJ fj, Pick pick) {
+    if (!picked(pick, true)) return;
     scott_persistent_body<R, F, FJ, X>(f, P, s, n, frames, recs, ds, queues, nq, refill_min, order, fj);
 }
 // The mixed variant, at two waves per SIMD.
@@ -1047,7 +1072,8 @@ template <typename R, class F, class FJ, typename X>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_scott_persistent_w2(F f, ScottParams P, Seeds s, unsigned long long n, const R* frames, ScottRec<R>* recs,
                       DevScalars ds, unsigned long long* queues, int nq, int refill_min, const unsigned* order,
-                      FJ fj) {
+                      FJ fj, Pick pick) {
+    if (!picked(pick, true)) return;
     scott_persistent_body<R, F, FJ, X>(f, P, s, n, frames, recs, ds, queues, nq, refill_min, order, fj);
 }
 
@@ -1215,7 +1241,8 @@ struct ScottLines {
 template <typename R, class F, class FJ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1)))
 k_scott_quads(F f, ScottParams P, Seeds s, unsigned long long n, const R* frames, ScottRec<R>* recs, DevScalars ds,
-              unsigned long long* queue, int spread, int refill_min, const unsigned* order, FJ fj) {
+              unsigned long long* queue, int spread, int refill_min, const unsigned* order, FJ fj, Pick pick) {
+    if (!picked(pick, false)) return;
     apply_scalars(f, P, n, ds);
     fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];  // J lives on B's grid
     P.ctl = scott_ctl(P.tol);  // on the device, so every path forms the same bits
@@ -1684,21 +1711,22 @@ static int scott_waves(unsigned long long n) {
     return (w == 3 && n <= small_launch_lines()) ? 2 : w;
 }
 
-// Stepping kernel and grid of the persistent Scott schedule; kern == nullptr: by
-// quads.  `lines`: how many are traced at a time.
+// Stepping kernels and grids of the persistent Scott schedule: by quads (quads > 0),
+// by lanes (kern), or both, of which one runs (`work`: k_order_scan's).  `lines`:
+// how many are traced at a time.
 template <typename R, class F, class FJ, typename X>
 struct ScottStepping {
     decltype(&k_scott_persistent<R, F, FJ, X>) kern = nullptr;
-    int grid = 0;
-    unsigned long long lines = 0;
+    int grid = 0, quads = 0;
+    unsigned long long lines = 0, work = 0;
 };
 
-// FP64 lines up to which a launch goes by quads, four a resident quad: above it
-// the quads' extra instructions cost more than their shorter chain gives, first
-// where seeds lie anywhere in the box and share no cells (ms by quads / by lanes,
-// RK4 on 108 x 66 x 51: 16 k lines 2.05 / 3.66, 33 k 3.2 / 3.7, 66 k 4.8 / 3.7, 131 k
-// 8.3 / 5.3; RKF45 66 k 10.5 / 11.7, 131 k 18.0 / 14.9), last on maps (128^3: 147 k
-// 7.0 / 7.5, 200 k 8.4 / 7.4).
+// FP64 lines up to which a launch may go by quads, four a resident quad: above it
+// the quads' extra instructions cost more than their shorter chain gives where
+// seeds lie anywhere in the box (ms by quads / by lanes, 108 x 66 x 51: RK4 131 k
+// lines 8.3 / 5.3; RKF45 66 k 9.7 / 9.2, 131 k 18.0 / 14.9), and from 200 k on on maps
+// (128^3: 147 k 7.0 / 7.5, 200 k 8.4 / 7.4).  Below it RK4 launches of few short lines
+// and many long ones part ways (scott_fp64_quad_work).
 constexpr unsigned long long kScottQuadLinesFp64 = 65536;
 // Lines (or sides) a wavefront takes at the least.  With one or two quads of a
 // wavefront traced, few lines wait longer than in one wavefront: spread over every
@@ -1733,23 +1761,35 @@ constexpr int kScottSpread = 2;
 constexpr int kScottQuadRefillFp32 = 1, kScottQuadRefillFp64 = 2;
 
 template <typename R, class F, class FJ, typename X>
-static int scott_stepping(ScottStepping<R, F, FJ, X>* st, unsigned long long n) {
-    unsigned long long per_block = 64;  // quads
-    int rc = FQSL_OK;
+static int scott_stepping(ScottStepping<R, F, FJ, X>* st, const F& f, int method, unsigned long long n) {
+    const int pct = g_tune[FQSL_TUNE_GRID_PCT];
+    bool lanes = !std::is_same<R, X>::value, quads = !lanes;
+    st->work = 0;
+    if (sizeof(R) == 8 && method == kRK4) {
+        const unsigned long long nodes = (unsigned long long)f.n[0] * f.n[1] * f.n[2];
+        const unsigned long long work = scott_fp64_quad_work(3ull * sizeof(R) * nodes);
+        if (n > work) {
+            lanes = true;
+            st->work = work;
+        }
+    }
+    if (sizeof(R) == 8 && n > kScottQuadLinesFp64) {
+        lanes = true;
+        quads = false;
+        st->work = 0;
+    }
     st->kern = nullptr;
+    st->grid = st->quads = 0;
     if constexpr (!std::is_same<R, X>::value) st->kern = k_scott_persistent_w2<R, F, FJ, X>;
     else if constexpr (sizeof(R) == 8)
-        if (n > kScottQuadLinesFp64) st->kern = k_scott_persistent<R, F, FJ, X>;
-    if (st->kern) {
-        per_block = 256;
-        rc = persistent_grid(st->kern, &st->grid);
-    } else if constexpr (std::is_same<R, X>::value) {
-        rc = persistent_grid(k_scott_quads<R, F, FJ>, &st->grid);
-    }
+        if (lanes) st->kern = k_scott_persistent<R, F, FJ, X>;
+    int rc = st->kern ? persistent_grid(st->kern, &st->grid) : FQSL_OK;
+    if constexpr (std::is_same<R, X>::value)
+        if (quads && rc == FQSL_OK) rc = persistent_grid(k_scott_quads<R, F, FJ>, &st->quads);
     if (rc) return rc;
-    st->grid = (int)((long)st->grid * g_tune[FQSL_TUNE_GRID_PCT] / 100);
-    if (st->grid < 1) st->grid = 1;
-    st->lines = per_block * (unsigned long long)st->grid;
+    for (int* g : {&st->grid, &st->quads})
+        if (*g) *g = std::max(1, (int)((long)*g * pct / 100));
+    st->lines = st->quads ? 64ull * st->quads : 256ull * st->grid;
     return FQSL_OK;
 }
 
@@ -1762,8 +1802,8 @@ template <typename R, class F, class FJ, typename X>
 static bool scott_ordered(const DevScalars& ds, const F& f, unsigned long long n_hint, const ScottStepping<R, F, FJ, X>& st) {
     const int om = g_tune[FQSL_TUNE_ORDER];
     return (!ds.shape || f.n[0] > 0) && n_hint < (1ull << 32) &&
-           (om == 2 || (om == 1 && (st.kern ? n_hint <= 64ull * st.lines
-                                            : n_hint > st.lines && n_hint <= 16ull * st.lines)));
+           (om == 2 || (om == 1 && (!st.quads ? n_hint <= 64ull * st.lines
+                                              : n_hint > st.lines && n_hint <= 16ull * st.lines)));
 }
 
 // The persistent schedule's launches on `st` over a workspace `ws` laid out
@@ -1792,30 +1832,36 @@ static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, co
         k_zero_u32<<<1, 256, 0, st>>>(counts, kOrderBuckets);
         k_order_predict<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(
             f, s, n, g_tune[FQSL_TUNE_ORDER_BUCKETS], key, counts);
-        k_order_scan<<<1, kOrderBuckets, 0, st>>>(counts);
+        k_order_scan<<<1, kOrderBuckets, 0, st>>>(counts, g_tune[FQSL_TUNE_ORDER_BUCKETS],
+                                                  step.work ? q + kSlotVotes : nullptr, step.work);
         const int sg = grid_for((long)n_hint, 256) < 4096 ? grid_for((long)n_hint, 256) : 4096;
         k_order_scatter<<<sg, 256, 0, st>>>(key, n, counts, order);
     }
     k_scott_prep<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(f, P, s, n, frames, o, ds);
     if (timed) e = hipEventRecord(g_evs0, st);
+    // without the estimated lengths nothing tells which of two kernels is the faster one
+    const Pick pick{step.work && ordered ? q + kSlotVotes : nullptr};
     if constexpr (std::is_same<R, X>::value) {
-        if (!step.kern) {
-            const QuadGrid g = quad_grid(n_hint, step.grid, kScottSpread, quad_min<R>());
+        if (step.quads) {
+            const QuadGrid g = quad_grid(n_hint, step.quads, kScottSpread, quad_min<R>());
             const int grid = g.blocks, waves = g.waves;
             const int refill = sizeof(R) == 4 ? kScottQuadRefillFp32 : kScottQuadRefillFp64;
             bool done = false;
             if constexpr (std::is_same<F, FieldSoA<float>>::value) {
                 if (pairs) {
                     k_scott_quads<R, FieldPairs, FJ><<<grid, 256, 0, st>>>(
-                        FieldPairs{pairs, {f.n[0], f.n[1], f.n[2]}}, P, s, n, frames, recs, ds, q, waves, refill, order, fj);
+                        FieldPairs{pairs, {f.n[0], f.n[1], f.n[2]}}, P, s, n, frames, recs, ds, q, waves, refill, order, fj,
+                        pick);
                     done = true;
                 }
             }
             if (!done)
-                k_scott_quads<R, F, FJ><<<grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, waves, refill, order, fj);
+                k_scott_quads<R, F, FJ><<<grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, waves, refill, order, fj,
+                                                              pick);
         }
     }
-    if (step.kern) step.kern<<<step.grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, nq, refill_min, order, fj);
+    if (step.kern && (pick.votes || !step.quads))
+        step.kern<<<step.grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, nq, refill_min, order, fj, pick);
     if (timed && e == hipSuccess) e = hipEventRecord(g_evs1, st);
     if (timed && e == hipSuccess) g_evs_valid = true;
     k_scott_finish<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(f, P, n, frames, recs, o, ds);
@@ -1849,7 +1895,7 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
         // n_hint: number of lines, known on the host (sizes the workspace)
         if (n_hint == 0) return FQSL_OK;
         ScottStepping<R, F, FJ, X> step;
-        int rc = scott_stepping<R, F, FJ, X>(&step, n_hint);
+        int rc = scott_stepping<R, F, FJ, X>(&step, f, P.method, n_hint);
         if (rc) return rc;
         const bool ordered = scott_ordered<R, F, FJ, X>(ds, f, n_hint, step);
         const ScottWs w = scott_ws_layout<R>(n_hint, ordered);

@@ -45,6 +45,20 @@ inline bool plain_by_lines(bool in_place, bool per_line, bool capturing) {
     return in_place || (per_line && capturing);
 }
 
+// Most FP64 RK4 Scott lines' worth of work, counted in longest lines of the launch
+// by the queue order's estimate, that go by quads of lanes.  By lanes a launch that
+// fits the chip takes as long as its longest line (3.3 us an evaluation on a field
+// that the L2 caches hold, 5.0 on a larger one); by quads the chip does an
+// evaluation every 0.12-0.15 ns, so the two meet where the work is that many longest
+// lines.  ms by quads / by lanes: 64^3 seeds anywhere, 24,576 lines (14,500 longest)
+// 3.8 / 4.3, 32,768 (19,400) 4.5 / 4.4, 65,536 (38,600) 6.6 / 4.4, a 256^2 map (13,300)
+// 2.7 / 3.5; 128^3 49,152 lines (31,900) 11.7 / 13.1, 57,344 (36,900) 13.3 / 13.0, a
+// 256^2 map (18,400) 4.8 / 7.7.  RKF45 lines go by quads up to the full count: 15 of 16
+// such launches gain 1.03-1.5, one takes 1.05 times as long.
+inline unsigned long long scott_fp64_quad_work(unsigned long long field_bytes) {
+    return field_bytes <= (32ull << 20) ? 19000ull : 34000ull;
+}
+
 // Consecutive requests of a batch and their lines: those of one layout, which a
 // launch by quads takes together, or of one field and method, which a launch by
 // lanes takes.  `counter` is the work counter of that launch.  Layouts of one

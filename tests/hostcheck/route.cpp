@@ -47,3 +47,5 @@ extern "C" int rt_alloc_or_give_back(int full, int code, int ok_at, int has_bloc
     return fqsl::alloc_or_give_back(
         full, [&] { return ++*calls >= ok_at ? 0 : code; }, [&] { return has_blocks != 0; });
 }
+
+extern "C" unsigned long long rt_scott_fp64_quad_work(unsigned long long bytes) { return fqsl::scott_fp64_quad_work(bytes); }

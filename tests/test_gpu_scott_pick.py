@@ -1,0 +1,41 @@
+"""FP64 RK4 launches of which the lines' estimated lengths pick the kernel.
+
+Seeds anywhere in the box (many long lines: one line per lane) and seeds on a
+plane with few long lines (by quads of lanes), at the counts where the choice
+begins and ends: the bits are those of one thread per line.
+"""
+import numpy as np
+import pytest
+
+from fastqsl_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+SHAPE = (24, 22, 18)
+
+
+@pytest.mark.parametrize("kind", ["volume", "plane"])
+@pytest.mark.parametrize("twist", [False, True])
+@pytest.mark.parametrize("n", [19000, 19001, 40000, 65536, 65537])
+def test_picked_kernel_gives_the_bits_of_one_thread_per_line(n, kind, twist):
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import fastqsl_amd as fq
+    b = synth.multipole(SHAPE, seed=3, count=12, device="cpu")
+    rng = np.random.default_rng(n)
+    p = rng.uniform(0.0, 1.0, (n, 3)) * (np.array(SHAPE) - 1)
+    if kind == "plane":
+        p[:, 2] = 0.0
+        p[: n - 50, :2] = p[: n - 50, :2] * 0.05       # nearly all lines start in one corner
+    p[3], p[5, 2] = np.nan, -0.5
+    x, y, z = (torch.as_tensor(np.ascontiguousarray(p[:, i], dtype=np.float32)).cuda() for i in range(3))
+    names = fq.trace.SCOTT_OUTPUTS + (("twist",) if twist else ())
+    kw = dict(method="rk4", step=0.25, precision="fp64", outputs=names)
+    with fq.Field(*b, layouts=("soa64",), current=(b[1], b[2], b[0]) if twist else None) as f:
+        ref = fq.trace_scott(f, x, y, z, schedule="per_line", **kw)
+        for _ in range(2):
+            got = fq.trace_scott(f, x, y, z, schedule="persistent", **kw)
+            torch.cuda.synchronize()
+            for k in names:
+                np.testing.assert_array_equal(got[k].cpu().numpy(), ref[k].cpu().numpy(), err_msg=k)
