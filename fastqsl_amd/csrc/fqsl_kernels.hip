@@ -926,6 +926,29 @@ __device__ __forceinline__ bool picked(const Pick& p, bool second) {
     return !p.votes || ((long long)p.votes[0] > 0) == second;
 }
 
+// Workgroups that trace where the lines lie far apart (0: all); the rest return.
+struct FarGrid {
+    const unsigned long long* votes;
+    int blocks;
+};
+
+// Whether the lines of neighbouring lanes begin near each other, within `reach`
+// cells: every pair votes, one for and one against.  All lanes of the wavefront call.
+__device__ __forceinline__ void vote_near(unsigned long long* votes, const float p0[3], bool in, float reach) {
+    const int lane = __lane_id();
+    const bool pair = lane < 63 && in && __shfl_down(in ? 1 : 0, 1) != 0;
+    bool near = pair;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) near = near && fabsf(__shfl_down(p0[a], 1) - p0[a]) <= reach;
+    const int sum = 2 * __popcll(__ballot(near)) - __popcll(__ballot(pair));
+    if (lane == 0 && sum != 0) atomicAdd(votes, (unsigned long long)(long long)sum);
+}
+// A map of few pixels on a large box has them up to two cells apart; of lines anywhere
+// in a box one pair in a thousand is that near.
+constexpr float kNearCells = 4.f;
+// One workgroup in so many votes: a vote is an atomic on one word, ~8 ns each.
+constexpr unsigned kVoteBlocks = 64;
+
 // Exclusive scan of the bucket counts (one block).  With `votes`, whether the
 // estimated lengths add up to more than `work` times the longest one.
 __global__ void __launch_bounds__(kOrderBuckets) k_order_scan(unsigned* counts, int nbuckets, unsigned long long* votes,
@@ -1389,7 +1412,8 @@ struct TangentLines {
 // list of the tangent lines.
 template <typename R, class F, class G>
 __global__ void __launch_bounds__(256) k_plain_prep(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o,
-                                                    DevScalars ds, const float* ncross, TangentLines tl, G g) {
+                                                    DevScalars ds, const float* ncross, TangentLines tl, G g,
+                                                    unsigned long long* votes) {
 #if defined(__HIP_DEVICE_COMPILE__)
     apply_plain_scalars(f, P, n, ds, ncross);
     grid_prologue(g);
@@ -1414,6 +1438,11 @@ __global__ void __launch_bounds__(256) k_plain_prep(F f, PlainParams P, Seeds s,
                 if (o.btx) { o.btx[i] = b[0]; o.bty[i] = b[1]; o.btz[i] = b[2]; }
                 if (o.bflag) o.bflag[i] = b_flag(b, P);
             }
+        }
+        if (votes && blockIdx.x % kVoteBlocks == 0) {
+            float p0[3] = {0.f, 0.f, 0.f};
+            if (in) { p0[0] = s.x[i]; p0[1] = s.y[i]; p0[2] = s.z[i]; }
+            vote_near(votes, p0, in, kNearCells);
         }
         const unsigned long long m = __ballot(tangent);
         if (m != 0ull) {
@@ -1535,7 +1564,9 @@ constexpr int kPlainQuadMin = 4;
 template <typename R, class F, class FJ, class G>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 2)))
 k_plain_quads(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, DevScalars ds, const float* ncross,
-              unsigned long long* queue, int spread, FJ fj, G g) {
+              unsigned long long* queue, int spread, FJ fj, G g, Pick pick, FarGrid far) {
+    if (!picked(pick, false)) return;
+    if (far.blocks && (int)blockIdx.x >= far.blocks && (long long)far.votes[0] <= 0) return;
     apply_plain_scalars(f, P, n, ds, ncross);
     fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];  // J lives on B's grid
     grid_prologue(g);
@@ -1556,7 +1587,8 @@ k_plain_quads(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, Dev
 template <typename R, class F, class FJ, class G>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 2)))
 k_plain_sides(F f, PlainParams P, Seeds s, unsigned long long n, PlainOut o, DevScalars ds, const float* ncross,
-              unsigned long long* queue, int refill_min, int tangent_blocks, TangentLines tl, FJ fj, G g) {
+              unsigned long long* queue, int refill_min, int tangent_blocks, TangentLines tl, FJ fj, G g, Pick pick) {
+    if (!picked(pick, true)) return;
     apply_plain_scalars(f, P, n, ds, ncross);
     fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];
     grid_prologue(g);
@@ -1983,24 +2015,35 @@ static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsign
             ws = nullptr;
         }
     }
-    int grid = 0;
-    rc = tl.list ? persistent_grid(k_plain_sides<R, F, FJ, G>, &grid, lds)
-                 : persistent_grid(k_plain_quads<R, F, FJ, G>, &grid, lds);
-    const unsigned long long blocks = (2ull * n_hint + 3) / 4;  // one side per wavefront at the least
-    if (blocks < (unsigned long long)grid) grid = (int)(blocks < 1 ? 1 : blocks);
+    // FP64 RK4: where the lines lie far apart fewer quads at a time, and where they
+    // lie close together lanes (fqsl_route.h)
+    const bool rk4_fp64 = sizeof(R) == 8 && P.method == kRK4;
+    const bool vote = rk4_fp64 && n_hint >= kPlainRk4Fp64VoteLines, both = rk4_fp64 && n_hint >= kPlainRk4Fp64PickLines;
+    unsigned long long* const votes = vote ? q + kSlotVotes : nullptr;
+    int sides = 0, quads = 0;
+    if (tl.list || both) rc = persistent_grid(k_plain_sides<R, F, FJ, G>, &sides, lds);
+    if (!tl.list && rc == FQSL_OK) rc = persistent_grid(k_plain_quads<R, F, FJ, G>, &quads, lds);
+    if (both && n_hint >= 192ull * sides) sides = std::max(1, sides / 2);  // three sides a lane of the half
+    const FarGrid far{votes, vote ? std::max(1, quads / 2) : 0};
+    const Pick pick{both ? votes : nullptr};
+    const unsigned long long blocks = std::max(1ull, (2ull * n_hint + 3) / 4);  // one side per wavefront at the least
+    for (int* g2 : {&sides, &quads})
+        if (blocks < (unsigned long long)*g2) *g2 = (int)blocks;
     if (rc == FQSL_OK) {
         k_zero_u64<<<1, 64, 0, st>>>(q, kQueueSlotWidth);
         rc = record_start(st);
     }
-    if (rc == FQSL_OK && (tl.list || o.len || o.evals || o.tw || o.btx || o.bflag))
-        k_plain_prep<R, F, G><<<per_line_grid(n_hint, 256, ds), 256, lds, st>>>(f, P, s, n, o, ds, ncross, tl, g);
+    if (rc == FQSL_OK && (tl.list || vote || o.len || o.evals || o.tw || o.btx || o.bflag))
+        k_plain_prep<R, F, G><<<per_line_grid(n_hint, 256, ds), 256, lds, st>>>(f, P, s, n, o, ds, ncross, tl, g,
+                                                                                votes);
     if (rc == FQSL_OK) {
-        if (tl.list)
-            k_plain_sides<R, F, FJ, G><<<grid, 256, lds, st>>>(f, P, s, n, o, ds, ncross, q,
-                                                               g_tune[FQSL_TUNE_PLAIN_REFILL], cu_count(), tl, fj, g);
-        else
-            k_plain_quads<R, F, FJ, G><<<grid, 256, lds, st>>>(f, P, s, n, o, ds, ncross, q,
-                                                               cu_count() * 4 * kPlainSpread, fj, g);
+        if (sides)
+            k_plain_sides<R, F, FJ, G><<<sides, 256, lds, st>>>(f, P, s, n, o, ds, ncross, q,
+                                                                g_tune[FQSL_TUNE_PLAIN_REFILL], cu_count(), tl, fj, g,
+                                                                pick);
+        if (quads)
+            k_plain_quads<R, F, FJ, G><<<quads, 256, lds, st>>>(f, P, s, n, o, ds, ncross, q,
+                                                                cu_count() * 4 * kPlainSpread, fj, g, pick, far);
         rc = record_end(st);
     }
     const hipError_t e = hipGetLastError();
