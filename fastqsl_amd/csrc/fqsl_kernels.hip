@@ -894,10 +894,21 @@ __global__ void k_zero_u32(unsigned* p, int count) {
     for (int t = threadIdx.x; t < count; t += blockDim.x) p[t] = 0u;
 }
 
+// Where the launch's own lines tell which of two kernels traces them faster, both
+// are launched and one returns at once (2-3 us): the second where `votes` is
+// positive, the first elsewhere.  votes == NULL: only one was launched.
+struct Pick {
+    const unsigned long long* votes;
+};
+__device__ __forceinline__ bool picked(const Pick& p, bool second) {
+    return !p.votes || ((long long)p.votes[0] > 0) == second;
+}
+
 // Bucket key per line (0 = longest) and the bucket counts.
 template <typename R, class F>
 __global__ void __launch_bounds__(256) k_order_predict(F f, Seeds s, unsigned long long n, int nbuckets,
-                                                       unsigned char* __restrict__ key, unsigned* counts) {
+                                                       unsigned char* __restrict__ key, unsigned* counts, Pick pick) {
+    if (!picked(pick, true)) return;
     __shared__ unsigned hist[kOrderBuckets];
     for (int t = threadIdx.x; t < kOrderBuckets; t += blockDim.x) hist[t] = 0u;
     __syncthreads();
@@ -914,16 +925,6 @@ __global__ void __launch_bounds__(256) k_order_predict(F f, Seeds s, unsigned lo
     __syncthreads();
     for (int t = threadIdx.x; t < kOrderBuckets; t += blockDim.x)
         if (hist[t]) atomicAdd(&counts[t], hist[t]);
-}
-
-// Where the launch's own lines tell which of two kernels traces them faster, both
-// are launched and one returns at once (2-3 us): the second where `votes` is
-// positive, the first elsewhere.  votes == NULL: only one was launched.
-struct Pick {
-    const unsigned long long* votes;
-};
-__device__ __forceinline__ bool picked(const Pick& p, bool second) {
-    return !p.votes || ((long long)p.votes[0] > 0) == second;
 }
 
 // Workgroups that trace where the lines lie far apart (0: all); the rest return.
@@ -946,6 +947,7 @@ __device__ __forceinline__ void vote_near(unsigned long long* votes, const float
 // A map of few pixels on a large box has them up to two cells apart; of lines anywhere
 // in a box one pair in a thousand is that near.
 constexpr float kNearCells = 4.f;
+constexpr float kDenseCells = 0.24f;  // of a Scott map's pixels: see kScottDenseLines
 // One workgroup in so many votes: a vote is an atomic on one word, ~8 ns each.
 constexpr unsigned kVoteBlocks = 64;
 
@@ -982,7 +984,8 @@ __global__ void __launch_bounds__(kOrderBuckets) k_order_scan(unsigned* counts, 
 // order[offset(bucket) + rank] = line, 256 lines per block step: one global
 // atomic per (block step, bucket) reserves the block's range in a bucket.
 __global__ void __launch_bounds__(256) k_order_scatter(const unsigned char* __restrict__ key, unsigned long long n,
-                                                       unsigned* offs, unsigned* __restrict__ order) {
+                                                       unsigned* offs, unsigned* __restrict__ order, Pick pick) {
+    if (!picked(pick, true)) return;
     __shared__ unsigned hist[kOrderBuckets], base[kOrderBuckets];
     for (unsigned long long c0 = blockIdx.x * 256ull; c0 < n; c0 += gridDim.x * 256ull) {
         hist[threadIdx.x] = 0u;
@@ -1003,11 +1006,17 @@ __global__ void __launch_bounds__(256) k_order_scatter(const unsigned char* __re
 // stepping kernel and B at the seed (Interp3d rule) straight to the output.
 template <typename R, class F>
 __global__ void __launch_bounds__(256) k_scott_prep(F f, ScottParams P, Seeds s, unsigned long long n,
-                                                    R* __restrict__ frames, ScottOut o, DevScalars ds) {
+                                                    R* __restrict__ frames, ScottOut o, DevScalars ds,
+                                                    unsigned long long* votes) {
     apply_scalars(f, P, n, ds);
-    for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < n;
-         i += (unsigned long long)gridDim.x * blockDim.x) {
-        const float p0[3] = {s.x[i], s.y[i], s.z[i]};
+    for (unsigned long long i0 = blockIdx.x * (unsigned long long)blockDim.x; i0 < n;
+         i0 += (unsigned long long)gridDim.x * blockDim.x) {
+        const unsigned long long i = i0 + threadIdx.x;
+        const bool in = i < n;
+        float p0[3] = {0.f, 0.f, 0.f};
+        if (in) { p0[0] = s.x[i]; p0[1] = s.y[i]; p0[2] = s.z[i]; }
+        if (votes && blockIdx.x % kVoteBlocks == 0) vote_near(votes, p0, in, kDenseCells);
+        if (!in) continue;
         R u0[3], v0[3], b0z;
         double nb0;
         seed_frame<R>(f, p0, u0, v0, &b0z, &nb0);
@@ -1028,7 +1037,7 @@ __global__ void __launch_bounds__(256) k_scott_prep(F f, ScottParams P, Seeds s,
 // queue entries once at least `refill_min` lanes of the wavefront are idle (or
 // all are), so the setup of refilled lines runs once for the group.  A wave
 // exits once every queue is empty and all its lanes are idle.
-template <typename R, class F, class FJ, typename X>
+template <typename R, class F, class FJ, typename X, bool kRoll = false>
 __device__ __forceinline__ void scott_persistent_body(F f, ScottParams P, Seeds s, unsigned long long n,
                                                       const R* __restrict__ frames, ScottRec<R>* __restrict__ recs,
                                                       DevScalars ds, unsigned long long* queues, int nq,
@@ -1073,7 +1082,7 @@ __device__ __forceinline__ void scott_persistent_body(F f, ScottParams P, Seeds 
         }
         if (active) {
             ScottEnd<R> e;
-            const int st = scott_attempt<R, F, FJ, X>(L, f, P, e, fj);
+            const int st = scott_attempt<R, F, FJ, X, kRoll>(L, f, P, e, fj);
             if (st != kTracing) {
                 recs[idx] = ScottRec<R>{L.st, e, L.len, st, L.evals, L.tw};
                 active = false;
@@ -1098,6 +1107,16 @@ k_scott_persistent_w2(F f, ScottParams P, Seeds s, unsigned long long n, const R
                       FJ fj, Pick pick) {
     if (!picked(pick, true)) return;
     scott_persistent_body<R, F, FJ, X>(f, P, s, n, frames, recs, ds, queues, nq, refill_min, order, fj);
+}
+
+// FP32c lines, the stages rolled into one loop, at three waves per SIMD.
+template <typename R, class F, class FJ, typename X>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
+k_scott_persistent_w3(F f, ScottParams P, Seeds s, unsigned long long n, const R* frames, ScottRec<R>* recs,
+                      DevScalars ds, unsigned long long* queues, int nq, int refill_min, const unsigned* order,
+                      FJ fj, Pick pick) {
+    if (!picked(pick, true)) return;
+    scott_persistent_body<R, F, FJ, X, true>(f, P, s, n, frames, recs, ds, queues, nq, refill_min, order, fj);
 }
 
 // Persistent stepping with one line per quad of lanes (fqsl_quad_scott.h), the
@@ -1744,14 +1763,25 @@ static int scott_waves(unsigned long long n) {
 }
 
 // Stepping kernels and grids of the persistent Scott schedule: by quads (quads > 0),
-// by lanes (kern), or both, of which one runs (`work`: k_order_scan's).  `lines`:
-// how many are traced at a time.
+// by lanes (kern), or both, of which one runs: by the work (`work`: k_order_scan's) or
+// by how dense the seeds lie.  `lines`: how many are traced at a time; `ordered_up_to`:
+// how many are ordered by default.
 template <typename R, class F, class FJ, typename X>
 struct ScottStepping {
     decltype(&k_scott_persistent<R, F, FJ, X>) kern = nullptr;
     int grid = 0, quads = 0;
-    unsigned long long lines = 0, work = 0;
+    unsigned long long lines = 0, ordered_up_to = 0, work = 0;
+    bool dense = false;
 };
+
+// FP32c RK4 lines from which dense seeds go by lanes, three wavefronts a SIMD, as the
+// pixels of a fine map do: they share their cells then, and a quad's landing and refill
+// weigh on short lines (ms by quads / by lanes: maps of 1.2 M pixels on 256^3 20.2 / 16.8,
+// a quarter of its side 8.2 / 6.6, 2.5 M 38.1 / 34.0, 4.2 M 61.0 / 53.4, on 64^3 16.7 / 14.0;
+// 1 M pixels 16.5 / 15.6 on 256^3, 9.1 / 9.4 on 160 x 128 x 128, 4.5 / 4.6 on 64^3).  Cubes of
+// samples a quarter of a cell apart take 37.7 / 39.3, half a cell 65 / 71, lines anywhere
+// 84 / 95; RKF45 maps 0.99-1.05.
+constexpr unsigned long long kScottDenseLines = 1ull << 20;
 
 // FP64 lines up to which a launch may go by quads, four a resident quad: above it
 // the quads' extra instructions cost more than their shorter chain gives where
@@ -1812,9 +1842,14 @@ static int scott_stepping(ScottStepping<R, F, FJ, X>* st, const F& f, int method
     }
     st->kern = nullptr;
     st->grid = st->quads = 0;
+    st->dense = false;
     if constexpr (!std::is_same<R, X>::value) st->kern = k_scott_persistent_w2<R, F, FJ, X>;
-    else if constexpr (sizeof(R) == 8)
+    else if constexpr (sizeof(R) == 8) {
         if (lanes) st->kern = k_scott_persistent<R, F, FJ, X>;
+    } else if constexpr (std::is_same<F, FieldCell32>::value && !has_current<FJ>()) {
+        st->dense = method == kRK4 && n > kScottDenseLines;
+        if (st->dense) st->kern = k_scott_persistent_w3<R, F, FJ, X>;
+    }
     int rc = st->kern ? persistent_grid(st->kern, &st->grid) : FQSL_OK;
     if constexpr (std::is_same<R, X>::value)
         if (quads && rc == FQSL_OK) rc = persistent_grid(k_scott_quads<R, F, FJ>, &st->quads);
@@ -1822,6 +1857,7 @@ static int scott_stepping(ScottStepping<R, F, FJ, X>* st, const F& f, int method
     for (int* g : {&st->grid, &st->quads})
         if (*g) *g = std::max(1, (int)((long)*g * pct / 100));
     st->lines = st->quads ? 64ull * st->quads : 256ull * st->grid;
+    st->ordered_up_to = st->quads && !st->dense ? 16ull * st->lines : 64ull * 256ull * st->grid;
     return FQSL_OK;
 }
 
@@ -1834,8 +1870,7 @@ template <typename R, class F, class FJ, typename X>
 static bool scott_ordered(const DevScalars& ds, const F& f, unsigned long long n_hint, const ScottStepping<R, F, FJ, X>& st) {
     const int om = g_tune[FQSL_TUNE_ORDER];
     return (!ds.shape || f.n[0] > 0) && n_hint < (1ull << 32) &&
-           (om == 2 || (om == 1 && (!st.quads ? n_hint <= 64ull * st.lines
-                                              : n_hint > st.lines && n_hint <= 16ull * st.lines)));
+           (om == 2 || (om == 1 && n_hint <= st.ordered_up_to && (!st.quads || n_hint > st.lines)));
 }
 
 // The persistent schedule's launches on `st` over a workspace `ws` laid out
@@ -1860,19 +1895,22 @@ static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, co
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (timed && record_start(st)) return hipErrorUnknown;
+    k_scott_prep<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(f, P, s, n, frames, o, ds,
+                                                                    step.dense ? q + kSlotVotes : nullptr);
+    // dense lines go by lanes, ordered; by quads such a launch is not
+    const Pick dense{step.dense ? q + kSlotVotes : nullptr};
     if (ordered) {
         k_zero_u32<<<1, 256, 0, st>>>(counts, kOrderBuckets);
         k_order_predict<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(
-            f, s, n, g_tune[FQSL_TUNE_ORDER_BUCKETS], key, counts);
+            f, s, n, g_tune[FQSL_TUNE_ORDER_BUCKETS], key, counts, dense);
         k_order_scan<<<1, kOrderBuckets, 0, st>>>(counts, g_tune[FQSL_TUNE_ORDER_BUCKETS],
                                                   step.work ? q + kSlotVotes : nullptr, step.work);
         const int sg = grid_for((long)n_hint, 256) < 4096 ? grid_for((long)n_hint, 256) : 4096;
-        k_order_scatter<<<sg, 256, 0, st>>>(key, n, counts, order);
+        k_order_scatter<<<sg, 256, 0, st>>>(key, n, counts, order, dense);
     }
-    k_scott_prep<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(f, P, s, n, frames, o, ds);
     if (timed) e = hipEventRecord(g_evs0, st);
     // without the estimated lengths nothing tells which of two kernels is the faster one
-    const Pick pick{step.work && ordered ? q + kSlotVotes : nullptr};
+    const Pick pick{(step.work && ordered) || step.dense ? q + kSlotVotes : nullptr};
     if constexpr (std::is_same<R, X>::value) {
         if (step.quads) {
             const QuadGrid g = quad_grid(n_hint, step.quads, kScottSpread, quad_min<R>());
@@ -1888,8 +1926,8 @@ static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, co
                 }
             }
             if (!done)
-                k_scott_quads<R, F, FJ><<<grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, waves, refill, order, fj,
-                                                              pick);
+                k_scott_quads<R, F, FJ><<<grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, waves, refill,
+                                                              step.dense ? nullptr : order, fj, pick);
         }
     }
     if (step.kern && (pick.votes || !step.quads))

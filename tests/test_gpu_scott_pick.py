@@ -39,3 +39,32 @@ def test_picked_kernel_gives_the_bits_of_one_thread_per_line(n, kind, twist):
             torch.cuda.synchronize()
             for k in names:
                 np.testing.assert_array_equal(got[k].cpu().numpy(), ref[k].cpu().numpy(), err_msg=k)
+
+
+@pytest.mark.parametrize("kind", ["volume", "map"])
+@pytest.mark.parametrize("n", [2 ** 20, 2 ** 20 + 1, 2 ** 20 + 300001])
+def test_large_fp32c_rk4_launches(n, kind):
+    """FP32c RK4 lines on cells: dense seeds by lanes, others by quads."""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import fastqsl_amd as fq
+    b = synth.multipole(SHAPE, seed=3, count=12, device="cpu")
+    hi = np.array(SHAPE, float) - 1
+    if kind == "volume":
+        p = np.random.default_rng(1).uniform(-0.02, 1.02, (n, 3)) * hi
+    else:
+        t = np.arange(n)
+        p = np.column_stack([(t % 1100) / 1100 * hi[0], (t // 1100) / (n // 1100 + 1) * hi[1], np.zeros(n)])
+    p[7], p[9, 1], p[11], p[13, 2] = np.nan, np.nan, hi + 50.0, -0.5
+    x, y, z = (torch.as_tensor(np.ascontiguousarray(p[:, i], dtype=np.float32)).cuda() for i in range(3))
+    names = fq.trace.SCOTT_OUTPUTS
+    kw = dict(method="rk4", step=0.5, precision="fp32c", outputs=names)
+    with fq.Field(*b, layouts=("cell32",)) as f:
+        got = fq.trace_scott(f, x, y, z, schedule="persistent", **kw)
+        ref = fq.trace_scott(f, x, y, z, schedule="per_line", **kw)
+        torch.cuda.synchronize()
+        for k in names:
+            assert torch.equal(got[k].view(torch.int32 if got[k].element_size() == 4 else torch.int64),
+                               ref[k].view(torch.int32 if ref[k].element_size() == 4 else torch.int64)) or \
+                np.array_equal(got[k].cpu().numpy(), ref[k].cpu().numpy(), equal_nan=True), k
