@@ -2765,14 +2765,8 @@ int batch_step_groups(const fqsl_scott_batch* b, const BatchGroup& S, hipStream_
     return FQSL_OK;
 }
 
-// FP32c lines of a layout up to which a batch goes by quads: 1.4 M lines over three
-// fields 41.1 ms against 48.9 by lanes, but 50.5 M lines in 256 requests 1.55 s
-// against 1.46: with hundreds of lines a quad no tail is left to shorten, and a
-// launch per (field, method) keeps to one field at a time.
-constexpr unsigned long long kBatchQuadLinesFp32 = 1ull << 24;
-
-// The requests of one layout: by quads, in one launch, up to the line counts above
-// (FP64: as a single trace, scott_stepping).
+// The requests of one layout: by quads, in one launch, or by lanes, one for each field
+// and method (batch_fp32_by_quads, batch_fp64_by_quads).
 template <typename R, class F, typename X = R>
 int batch_launch(const fqsl_scott_batch* b, const BatchGroup& S, hipStream_t st) {
     const BatchGroupArgs g{b->reqs, b->offs, S.r0, S.r1, S.base, S.n};
@@ -2782,7 +2776,14 @@ int batch_launch(const fqsl_scott_batch* b, const BatchGroup& S, hipStream_t st)
     int rc = FQSL_OK;
     bool quads = false;
     if constexpr (std::is_same<R, X>::value) {
-        quads = S.n <= (sizeof(R) == 4 ? kBatchQuadLinesFp32 : kScottQuadLinesFp64);
+        unsigned long long rk4 = 0;
+        int groups = 0;
+        for (const BatchGroup& G : b->groups) {
+            if (G.n == 0 || G.r0 < S.r0 || G.r0 >= S.r1) continue;
+            ++groups;
+            if (G.method == kRK4) rk4 += G.n;
+        }
+        quads = sizeof(R) == 4 ? batch_fp32_by_quads(S.n - rk4, rk4) : batch_fp64_by_quads(S.n, groups, rk4 != 0);
         if (quads) {
             int full = 0;
             rc = persistent_grid(k_batch_quads<R, F>, &full);

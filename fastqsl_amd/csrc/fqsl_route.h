@@ -103,6 +103,24 @@ inline void batch_spans(int nreq, const int* kind, const char* other, const unsi
     }
 }
 
+// Whether one launch by quads takes all requests of a batch's layout.  By lanes each
+// (field, method) group is a launch of its own.
+// FP32c: lines of which a quad has hundreds leave no tail to shorten, and a launch per
+// group keeps to one field at a time; fixed-step lines hold on longer (three fields, ms by
+// quads / by lanes: 1.9 M lines RKF45 23.7 / 28.7, 7.7 M 87 / 89 and seeds anywhere 138 /
+// 136, 15.4 M 171 / 167 and 275 / 265; RK4 1.9 M 23.9 / 28.5, 15.4 M 167 / 168 and 325 /
+// 348; both 16.6 M 183 / 186; 50.5 M in 256 requests 1.55 s / 1.46).
+inline bool batch_fp32_by_quads(unsigned long long rkf45_lines, unsigned long long rk4_lines) {
+    return rkf45_lines + rk4_lines / 2 <= (1ull << 23);
+}
+// FP64: of several groups each would wait for its longest line in turn; one alone does
+// so once, and its lines are not ordered (ms by quads / by lanes: one RK4 request on 96^3
+// of 16,384 map pixels 2.9 / 5.0, 24,576 5.6 / 5.3, 65,536 7.8 / 5.1; RKF45 24,576 7.8 / 9.0,
+// 40,000 9.2 / 9.0; two of 32,000 RK4 10.8 / 12.9, RKF45 11.0 / 20.4; twelve of 5,000 9.2 / 24.8).
+inline bool batch_fp64_by_quads(unsigned long long lines, int groups, bool rk4) {
+    return lines <= (groups > 1 ? 65536ull : rk4 ? 20000ull : 32768ull);
+}
+
 // An allocation that may find the memory in what the library keeps: `alloc` is
 // tried again when it fails for want of memory (`full`) and `give_back` has freed
 // some.

@@ -49,3 +49,10 @@ extern "C" int rt_alloc_or_give_back(int full, int code, int ok_at, int has_bloc
 }
 
 extern "C" unsigned long long rt_scott_fp64_quad_work(unsigned long long bytes) { return fqsl::scott_fp64_quad_work(bytes); }
+
+extern "C" int rt_batch_fp32_by_quads(unsigned long long rkf45, unsigned long long rk4) {
+    return fqsl::batch_fp32_by_quads(rkf45, rk4) ? 1 : 0;
+}
+extern "C" int rt_batch_fp64_by_quads(unsigned long long lines, int groups, int rk4) {
+    return fqsl::batch_fp64_by_quads(lines, groups, rk4 != 0) ? 1 : 0;
+}

@@ -51,3 +51,26 @@ def test_large_cell_layout_beside_a_small_one_without_cells():
                         np.testing.assert_array_equal(res[name][part].cpu().numpy(), ref[name].cpu().numpy(),
                                                       err_msg=f"{name} of request {k}")
                     assert int((ref["flag_end"] > 0).sum()) > 0
+
+
+@pytest.mark.parametrize("method,n", [("rk4", 20000), ("rk4", 20001), ("rkf45", 32768), ("rkf45", 32769)])
+def test_one_fp64_request_on_both_sides_of_its_rule(method, n):
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import fastqsl_amd as fq
+    from fastqsl_amd.batch import ScottBatch
+    shape = (20, 17, 15)
+    rng = np.random.default_rng(2)
+    p = torch.as_tensor((rng.uniform(-0.02, 1.02, (n, 3)) * (np.array(shape) - 1)).astype(np.float32)).cuda()
+    x, y, z = (p[:, i].contiguous() for i in range(3))
+    with fq.Field(*synth.multipole(shape, seed=3, count=8, device="cpu"), layouts=("soa64",)) as f:
+        rq = dict(field=f, x=x, y=y, z=z, method=method, step=0.25, tol=1e-5)
+        ref = fq.trace_scott(f, x, y, z, method=method, step=0.25, tol=1e-5, precision="fp64", schedule="per_line",
+                             outputs=NAMES)
+        with ScottBatch([rq], precision="fp64", outputs=NAMES) as batch:
+            for _ in range(2):
+                batch.run()
+            torch.cuda.synchronize()
+            for name in NAMES:
+                np.testing.assert_array_equal(batch.results[0][name].cpu().numpy(), ref[name].cpu().numpy(), err_msg=name)

@@ -100,3 +100,13 @@ def test_fp64_work_that_goes_by_quads(route):
     f.restype, f.argtypes = ctypes.c_ulonglong, [ctypes.c_ulonglong]
     assert f(24 * 64 ** 3) == f(32 << 20) == 19000      # fields that the eight 4 MiB L2 caches hold
     assert f((32 << 20) + 1) == f(24 * 256 ** 3) == 34000
+
+
+def test_batches_by_quads(route):
+    u = ctypes.c_ulonglong
+    for rkf45, rk4, quads in ((0, 0, 1), (2 ** 23, 0, 1), (2 ** 23 + 1, 0, 0), (0, 2 ** 24, 1), (0, 2 ** 24 + 2, 0),
+                              (2 ** 22, 2 ** 23, 1), (2 ** 22 + 1, 2 ** 23, 0)):
+        assert route.rt_batch_fp32_by_quads(u(rkf45), u(rk4)) == quads, (rkf45, rk4)
+    for lines, groups, rk4, quads in ((20000, 1, 1, 1), (20001, 1, 1, 0), (32768, 1, 0, 1), (32769, 1, 0, 0),
+                                      (65536, 2, 1, 1), (65537, 2, 0, 0), (65536, 12, 0, 1)):
+        assert route.rt_batch_fp64_by_quads(u(lines), groups, rk4) == quads, (lines, groups, rk4)
