@@ -4,12 +4,13 @@ The knobs (``_lib.TUNE_KNOBS``) change speed only -- a line's result does not
 depend on the lane, wave, queue or launch that traces it -- so they can be
 picked per workload by measurement:
 
-* ``scott_waves``  waves per SIMD the FP32c Scott kernels with one line per lane
-                   (per-line schedule, batches) are built for (3 = 168 VGPRs per
-                   lane, 2 = 256; 0 = the compiler's choice);
+* ``scott_waves``  waves per SIMD the FP32c Scott kernel of the per-line schedule is
+                   built for (3 = 168 VGPRs per lane, 2 = 256; 0 = the compiler's
+                   choice); no persistent launch reads it, so it is not searched;
 * ``refill_min``   idle lanes a wavefront of a persistent kernel with one line per
-                   lane (mixed, large FP64 launches, batches) gathers before it
-                   claims new lines (the queue chunk: one atomic per chunk);
+                   lane (mixed, FP64 launches and batches too large for quads,
+                   large RK4 maps, very large FP32c batches) gathers before it claims
+                   new lines (the queue chunk: one atomic per chunk);
 * ``queues``       one seed queue of such a kernel, or one per XCD (8), the
                    launch's blocks spread over them;
 * ``grid_pct``     persistent grid size in % of one full occupancy wave;
@@ -19,7 +20,8 @@ picked per workload by measurement:
                    lanes where lines are traced by quads;
 * ``order_buckets``length classes of that order (fewer keep more locality).
 
-``autotune`` runs coordinate descent over these on the actual request, or on
+``autotune`` runs coordinate descent over those that the request's launches read
+(where lines are traced by quads of lanes, the order and the grid) on the request, or on
 a contiguous slice of it when it is larger than ``sample`` lines (contiguous,
 because neighbouring seeds share cache lines of the field: a random subset
 has a different L2 behaviour and picks different knobs), keeps the fastest
@@ -47,6 +49,23 @@ SPACE = {
 }
 DEFAULTS = {"order": 1, "order_buckets": 64, "scott_waves": 3, "refill_min": 8, "queues": 1,
             "grid_pct": 100}
+
+
+# Line counts from which a request may be traced one line per lane (see fqsl_route.h):
+# single FP64 launches and batches, FP32c RK4 maps, FP32c batches.
+_LANES_FROM = {"fp64": 19000, "rk4": 1 << 20, "batch": 1 << 23}
+
+
+def searched(precision, method="rkf45", lines=0, batch=False):
+    """The knobs that a persistent Scott launch, or a batch, of ``lines`` lines reads."""
+    knobs = [] if batch else ["order", "order_buckets"]
+    lanes = (precision == "mixed" or (precision == "fp64" and lines > _LANES_FROM["fp64"])
+             or (precision == "fp32c" and lines > _LANES_FROM["batch" if batch else "rk4"] and (batch or method == "rk4")))
+    if lanes:
+        knobs.append("refill_min")
+        if not batch:
+            knobs.append("queues")
+    return knobs + ["grid_pct"]
 
 
 def cache_path() -> str:
@@ -153,7 +172,8 @@ def autotune(field, x, y, z, method="rkf45", step=0.25, tol=1e-6, precision="fp3
         return float(np.median(ms))
 
     try:
-        best, best_ms, seen = coordinate_descent(measure, log=log)
+        space = {k: SPACE[k] for k in searched(precision, method, int(xs.numel()))}
+        best, best_ms, seen = coordinate_descent(measure, space=space, log=log)
     except Exception:
         apply(before)
         raise
@@ -167,9 +187,6 @@ def autotune(field, x, y, z, method="rkf45", step=0.25, tol=1e-6, precision="fp3
 
 
 BATCH_SPACE = {
-    "order": (1, 2, 0),
-    "order_buckets": (64, 16, 256),
-    "scott_waves": (3, 2, 0),
     "refill_min": (8, 4, 16, 32),
     "grid_pct": (100, 75),
 }
@@ -177,9 +194,9 @@ BATCH_SPACE = {
 
 def autotune_batch(requests, precision="fp32c", outputs=("q_0", "flag_start", "flag_end"),
                    max_lines=1 << 23, log=None):
-    """Pick the knobs for a batch of requests (``batch.ScottBatch``): the
-    stepping kernel's waves per SIMD and refill chunk are fixed when a batch is
-    planned, the grid size when it runs.  Measures on the leading requests up
+    """Pick the knobs for a batch of requests (``batch.ScottBatch``): the refill
+    chunk, where lines are traced one per lane, is fixed when a batch is planned,
+    the grid size when it runs.  Measures on the leading requests up
     to `max_lines` lines (each point plans a fresh batch and times its second
     run), applies the best configuration and returns it."""
     from .batch import ScottBatch
@@ -201,7 +218,8 @@ def autotune_batch(requests, precision="fp32c", outputs=("q_0", "flag_start", "f
 
     before = current()
     try:
-        best, best_ms, _ = coordinate_descent(measure, space=BATCH_SPACE,
+        space = {k: BATCH_SPACE[k] for k in searched(precision, lines=lines, batch=True)}
+        best, best_ms, _ = coordinate_descent(measure, space=space,
                                               start={k: DEFAULTS[k] for k in BATCH_SPACE}, rounds=1,
                                               log=log)
     except Exception:

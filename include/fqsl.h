@@ -506,17 +506,16 @@ int fqsl_TraceAllBlineStretch(float *Bx, float *By, float *Bz, int *BshapeN, flo
 /* ---------------------------------------------------------- tuning knobs */
 /* Process-wide launch parameters (fastqsl_amd._lib.tune_set / tune_get).
  * They change speed only, never results. */
-#define FQSL_TUNE_SCOTT_WAVES 0 /* waves/SIMD of the FP32c Scott kernels that run one line per lane
-                                 (the per-line schedule, batches): 3 (default: the stages
-                                 rolled into one loop), 2 (unrolled) or 0 (compiler's
-                                 choice); a launch of at most one two-wave grid's lanes
-                                 (131,072 lines on 256 CUs) runs two; the mixed variant
-                                 and the twist tracer always run two */
+#define FQSL_TUNE_SCOTT_WAVES 0 /* waves/SIMD of the FP32c Scott kernel of the per-line schedule: 3
+                                 (default: the stages rolled into one loop), 2 (unrolled) or
+                                 0 (compiler's choice); a launch of at most one two-wave
+                                 grid's lanes (131,072 lines on 256 CUs) runs two; the mixed
+                                 variant and the twist tracer always run two */
 #define FQSL_TUNE_GRID_PCT 1    /* persistent grid size in % of one full occupancy wave (default 100) */
-#define FQSL_TUNE_QUEUES 2      /* seed queues of a persistent Scott kernel with one line per lane (mixed,
-                                   large FP64 launches): 1 (default) or 8 (one per XCD) */
-#define FQSL_TUNE_REFILL_MIN 3  /* idle lanes a wavefront of such a kernel gathers before it refills them
-                                   (1..64, default 8) */
+#define FQSL_TUNE_QUEUES 2      /* seed queues of a persistent Scott kernel with one line per lane (mixed, large
+                                   FP64 launches, large RK4 maps): 1 (default) or 8 (one per XCD) */
+#define FQSL_TUNE_REFILL_MIN 3  /* idle lanes a wavefront of such a kernel, or of a batch's, gathers before it
+                                   refills them (1..64, default 8) */
 #define FQSL_TUNE_ORDER 4       /* persistent Scott queue order: 0 = seed order, 2 = longest first by a
                                    coarse length estimate, 1 (default) = longest first up to 64 lines per
                                    persistent lane, or where lines are traced by quads of lanes from one
