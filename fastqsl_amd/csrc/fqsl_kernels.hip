@@ -2747,10 +2747,18 @@ std::vector<int> batch_order(const fqsl_scott_request* reqs, int nreq) {
     return ord;
 }
 
+// The stepping kernel of lines one per lane: FP64, FP32c (three waves, rolled stages)
+// or mixed; a type's other forms are not built.
+template <typename R, class F, typename X>
+constexpr auto batch_step_kernel() {
+    if constexpr (sizeof(R) == 8) return k_batch_step<R, F, X>;
+    else if constexpr (std::is_same<R, X>::value) return k_batch_step_w3<R, F, X>;
+    else return k_batch_step_w2<R, F, X>;
+}
+
 template <typename R, class F, typename X>
 int batch_step_groups(const fqsl_scott_batch* b, const BatchGroup& S, hipStream_t st) {
-    auto kern = sizeof(R) == 8 ? k_batch_step<R, F, X>
-              : std::is_same<R, X>::value ? k_batch_step_w3<R, F, X> : k_batch_step_w2<R, F, X>;
+    constexpr auto kern = batch_step_kernel<R, F, X>();
     int grid = 0;
     int rc = persistent_grid(kern, &grid);
     if (rc) return rc;
