@@ -11,7 +11,7 @@ ROOT = os.path.dirname(HERE)
 SOURCES = [os.path.join(HERE, "csrc", "fqsl_kernels.hip")]
 HEADERS = [os.path.join(HERE, "csrc", "fqsl_tracer.h"), os.path.join(HERE, "csrc", "fqsl_stretch.h"),
            os.path.join(HERE, "csrc", "fqsl_quad.h"), os.path.join(HERE, "csrc", "fqsl_quad_scott.h"),
-           os.path.join(HERE, "csrc", "fqsl_route.h"),
+           os.path.join(HERE, "csrc", "fqsl_route.h"), os.path.join(HERE, "csrc", "fqsl_step.h"),
            os.path.join(ROOT, "include", "fqsl.h")]
 
 HIPCC_FLAGS = [

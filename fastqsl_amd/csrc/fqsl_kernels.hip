@@ -2022,9 +2022,13 @@ static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsign
                         const DevScalars& ds, const float* ncross, int schedule, hipStream_t st,
                         unsigned long long n_hint, const FJ& fj = FJ{}, const G& g = G{}) {
     const int lds = grid_lds_bytes(g);
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    HIP_TRY(hipStreamIsCapturing(st, &cap));
-    const bool capturing = cap != hipStreamCaptureStatusNone;
+    const unsigned long long listed = plain_listed_lines(P.method == kRKF45, n_hint, !ds.N);
+    bool capturing = false;
+    if (listed || schedule == FQSL_SCHED_PER_LINE) {  // what else is launched does not depend on it
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(hipStreamIsCapturing(st, &cap));
+        capturing = cap != hipStreamCaptureStatusNone;
+    }
     const void* const seeds[] = {s.x, s.y, s.z};
     const void* const outs[] = {o.sx, o.sy, o.sz, o.ex, o.ey, o.ez, o.fs, o.fe, o.btx, o.bty, o.btz, o.bflag,
                                 o.bsx, o.bsy, o.bsz, o.bex, o.bey, o.bez, o.evals};
@@ -2043,7 +2047,6 @@ static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsign
     // 5 bytes a line; a capturing stream takes no allocation and traces by quads.
     TangentLines tl{nullptr, nullptr, q + 2};
     char* ws = nullptr;
-    const unsigned long long listed = plain_listed_lines(P.method == kRKF45, n_hint, !ds.N);
     if (listed && !capturing) {
         if (dev_malloc_async(&ws, 5 * (size_t)listed, st) == hipSuccess) {
             tl.list = (unsigned*)ws;

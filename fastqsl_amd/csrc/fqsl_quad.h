@@ -28,6 +28,7 @@
 
 #include "fqsl_stretch.h"
 #include "fqsl_tracer.h"
+#include "fqsl_step.h"
 
 namespace fqsl {
 
@@ -420,51 +421,21 @@ FQSL_COLD double plain_tol(double bn, double tol_coef) {
     return (bn <= 0.05 ? kTolBase / 8e3 : kTolBase * pow(bn, 1.5)) * tol_coef;
 }
 
-// tol / err / 11.09 with err = sqrt(e2), each rounded as the written expression
-// rounds it: square root and quotients from a refined v_rsq_f64 and a constant
-// reciprocal, with an exact remainder step each, ~20 instructions instead of
-// ~70.  (A step size is the product of all scales before it, and near the float
-// floor of the error norm one last bit leads to other steps.)
-__device__ __forceinline__ double scale_argument(double tol, double e2) {
-#pragma clang fp contract(off)  // a product and its remainder are not fused
-    double r = __builtin_amdgcn_rsq(e2);
-    double g = e2 * r, h = 0.5 * r;
-    const double d = fma(-h, g, 0.5);
-    g = fma(g, d, g);
-    h = fma(h, d, h);
-    g = fma(fma(-g, g, e2), h, g);
-    g = fma(fma(-g, g, e2), h, g);  // sqrt(e2)
-    r = 2.0 * h;
-    r = fma(fma(-g, r, 1.0), r, r);
-    double q = tol * r;
-    q = fma(fma(-g, q, tol), r, q);  // tol / sqrt(e2)
-    constexpr double kInv = 1.0 / 11.09;
-    const double w = q * kInv;
-    return fma(fma(-11.09, w, q), kInv, w);
-}
-FQSL_COLD double scale_argument_wide(double tol, double e2) { return tol / sqrt(e2) / 11.09; }
-
-FQSL_COLD double fifth_root(double q) { return pow(q, 0.2); }
-
-// Step control (TraceBlineAdaptive.cu:365-370): scales s, false when the step is
-// rejected.  The fifth root's library pow, most of the controller, runs only
-// where its value counts: not where a float estimate already tells that the
-// step is rejected or that the new one lies beyond its bounds.
+// Step control (TraceBlineAdaptive.cu:365-370) with the hardware's estimates: scales s,
+// false when the step is rejected.
 __device__ __forceinline__ bool next_step(double& s, double tol, double e2) {
-    const bool plain = e2 > 1e-60 && e2 < 1e60 && tol > 1e-60 && tol < 1e60;
-    const double q = plain ? scale_argument(tol, e2) : scale_argument_wide(tol, e2);
-    const float g = __builtin_amdgcn_exp2f(0.2f * __builtin_amdgcn_logf((float)q));  // within 1e-5 of the root
-    double scale = (double)g;
-    const double far = s * scale;
-    if (!(g < 0.617f || far > 100.1 || (g > 0.619f && far < 0.0999))) scale = fifth_root(q);
-    if (scale < 0.618) {
-        s = s * 0.618;
-        return false;
+    double q;
+    float g;
+    if (step_is_plain(s, tol, e2)) {
+        q = scale_argument(tol, e2, __builtin_amdgcn_rsq(e2));
+        g = __builtin_amdgcn_exp2f(0.2f * __builtin_amdgcn_logf((float)q));
+    } else {
+        q = scale_argument_wide(tol, e2);
+        g = NAN;
     }
-    s = s * scale;
-    if (s > 100.) s = 100.;
-    if (s < 1. / 10.) s = 1. / 10.;
-    return true;
+    const Step n = step_of_argument(s, q, g);
+    s = n.s;
+    return n.accepted;
 }
 
 template <int K, typename R, class F, class FJ, class G>
