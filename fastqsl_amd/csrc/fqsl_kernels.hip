@@ -2056,16 +2056,18 @@ static int launch_plain(const F& f, const PlainParams& P, const Seeds& s, unsign
             ws = nullptr;
         }
     }
-    // FP64 RK4: where the lines lie far apart fewer quads at a time, and where they
-    // lie close together lanes (fqsl_route.h)
-    const bool rk4_fp64 = sizeof(R) == 8 && P.method == kRK4;
-    const bool vote = rk4_fp64 && n_hint >= kPlainRk4Fp64VoteLines, both = rk4_fp64 && n_hint >= kPlainRk4Fp64PickLines;
+    // RK4 on component arrays: where the lines lie far apart fewer quads at a time, and
+    // where they lie close together lanes (fqsl_route.h)
+    constexpr bool kArrays = std::is_same<F, FieldSoA<R>>::value;
+    const bool counted = !ds.N && !ds.n_dev, rk4_arrays = kArrays && P.method == kRK4 && counted;
+    const bool vote = rk4_arrays && n_hint >= kPlainRk4VoteLines, both = rk4_arrays && n_hint >= kPlainRk4PickLines;
     unsigned long long* const votes = vote ? q + kSlotVotes : nullptr;
     int sides = 0, quads = 0;
     if (tl.list || both) rc = persistent_grid(k_plain_sides<R, F, FJ, G>, &sides, lds);
     if (!tl.list && rc == FQSL_OK) rc = persistent_grid(k_plain_quads<R, F, FJ, G>, &quads, lds);
-    if (both && n_hint >= 192ull * sides) sides = std::max(1, sides / 2);  // three sides a lane of the half
-    const FarGrid far{votes, vote ? std::max(1, quads / 2) : 0};
+    if ((both || (kArrays && sizeof(R) == 4)) && n_hint >= kPlainHalfSidesLines) sides = (sides + 1) / 2;
+    if (P.method == kRKF45 && n_hint <= kPlainQuadSides / 2) quads = std::min(quads, cu_count() * kPlainSpread);
+    const FarGrid far{votes, vote ? std::min(quads, cu_count()) : 0};
     const Pick pick{both ? votes : nullptr};
     const unsigned long long blocks = std::max(1ull, (2ull * n_hint + 3) / 4);  // one side per wavefront at the least
     for (int* g2 : {&sides, &quads})

@@ -25,20 +25,27 @@ inline unsigned long long plain_listed_lines(bool rkf45, unsigned long long line
     return list ? lines : 0ull;
 }
 
-// FP64 RK4 lines go by quads of lanes as the FP32 ones do, but a side's stage point
-// touches twelve cache lines of the three arrays and not one record.  Two resident
-// wavefronts a SIMD of 16 sides are 6.3 MB of lines for each 4 MiB L2 cache, and
-// sides that start anywhere in the box drive each other out of it.  From this count
-// on the seeds tell (vote_near: the lines of most neighbouring lanes begin within a
-// few cells or not); where they lie far apart, one wavefront a SIMD traces (ms two / one /
-// the kernels before quads, one lane a line: 160 x 128 x 128, 24,576 lines 6.5 / 4.3 / 8.9,
-// 65,536 19.9 / 9.0 / 16.9, 262,144 82 / 32.6 / 66; 64^3 262,144 13.0 / 11.9 / 12.9).
-constexpr unsigned long long kPlainRk4Fp64VoteLines = 16384;
+// RK4 lines go by quads of lanes on any layout, but on component arrays a side's stage
+// point touches twelve cache lines and not one record.  Two resident wavefronts a SIMD of
+// 16 sides are 6.3 MB of lines for each 4 MiB L2 cache (FP32 has four), and sides that
+// start anywhere in the box drive each other out of it.  From this count on the seeds
+// tell (vote_near: the lines of most neighbouring lanes begin within a few cells or not);
+// where they lie far apart, one wavefront a SIMD traces.  ms all / one / the kernels
+// before quads, one lane a line: FP64 160 x 128 x 128, 24,576 lines 6.5 / 4.3 / 8.9, 65,536
+// 19.9 / 9.0 / 16.9, 262,144 82 / 32.6 / 66; 64^3 262,144 13.0 / 11.9 / 12.9; FP32 160 x 128 x
+// 128, 16,384 lines 3.2 / 2.6 / 6.9, 65,536 14.8 / 7.4 / 12.8, 600,000 148 / 60 / 123; 64^3
+// 600,000 25.3 / 25.6 / 28.6.
+constexpr unsigned long long kPlainRk4VoteLines = 16384;
 // Close together no cache is short, and one side a lane takes fewer instructions: from
 // this count on near lines go by lanes (ms by quads / by lanes / before: maps on 160 x
-// 128 x 128, 65,536 lines 2.9 / 2.3 / 3.2, 131,072 4.4 / 3.3 / 3.9, 262,144 7.0 / 4.7 / 5.0,
-// 1 M 21 / 11.9 / 17; 32,768 lines 2.1 / 2.1 / 3.3).
-constexpr unsigned long long kPlainRk4Fp64PickLines = 65536;
+// 128 x 128, FP64 65,536 lines 2.9 / 2.3 / 3.2, 131,072 4.4 / 3.3 / 3.9, 1 M 21 / 11.9 / 17;
+// FP32 65,536 2.7 / 2.45 / 2.7, 262,144 6.7 / 4.3 / 4.9, 600,000 13.0 / 6.6 / 7.9; 32,768 lines
+// FP64 2.1 / 2.1 / 3.3, FP32 1.6 / 1.75 / 3.0).
+constexpr unsigned long long kPlainRk4PickLines = 65536;
+// One side a lane, from this count on half the resident grid, for the caches too (all /
+// half: RK4 maps FP64 131,072 lines on 160 x 128 x 128 3.8 / 3.3, FP32 600,000 on 200 x 160 x
+// 128 8.4 / 7.8, RKF45 maps 1.95 / 1.58, seeds anywhere 13.6 / 13.4; 65,536 FP64 2.3 / 2.9).
+constexpr unsigned long long kPlainHalfSidesLines = 98304;
 
 // Whether a plain trace writes a result where it reads its seeds.  The forward
 // and the backward side of a line are separate tasks, each of which reads the

@@ -1,4 +1,4 @@
-"""Large FP64 RK4 plain traces, of which the seeds pick the kernel.
+"""Large RK4 plain traces on component arrays, of which the seeds pick the kernel.
 
 Lines close together (one side a lane) and lines anywhere in the box (quads, one
 wavefront a SIMD), at the counts where each begins: the bits of the 4-byte
@@ -16,7 +16,8 @@ SHAPE = (26, 21, 17)
 
 @pytest.mark.parametrize("kind", ["volume", "map"])
 @pytest.mark.parametrize("n", [16383, 16384, 65535, 65536, 200001])
-def test_large_calls_equal_small_ones(n, kind):
+@pytest.mark.parametrize("layout,precision", [("soa64", "fp64"), ("soa32", "fp32c")])
+def test_large_calls_equal_small_ones(layout, precision, n, kind):
     import torch
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
@@ -31,8 +32,8 @@ def test_large_calls_equal_small_ones(n, kind):
     p[7], p[9, 1], p[11] = np.nan, np.nan, hi + 50.0
     x, y, z = (torch.as_tensor(np.ascontiguousarray(p[:, i], dtype=np.float32)).cuda() for i in range(3))
     names = tuple(k for k in fq.trace.PLAIN_OUTPUTS if k != "line_len")
-    kw = dict(method="rk4", step=0.25, precision="fp64", outputs=names)
-    with fq.Field(*b, layouts=("soa64",)) as f:
+    kw = dict(method="rk4", step=0.25, precision=precision, outputs=names)
+    with fq.Field(*b, layouts=(layout,)) as f:
         whole = fq.trace_plain(f, x, y, z, **kw)
         only = fq.trace_plain(f, x, y, z, **dict(kw, outputs=("end_x", "end_y", "end_z")))
         torch.cuda.synchronize()
