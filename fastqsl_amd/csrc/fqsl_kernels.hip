@@ -1007,7 +1007,7 @@ __global__ void __launch_bounds__(256) k_order_scatter(const unsigned char* __re
 template <typename R, class F>
 __global__ void __launch_bounds__(256) k_scott_prep(F f, ScottParams P, Seeds s, unsigned long long n,
                                                     R* __restrict__ frames, ScottOut o, DevScalars ds,
-                                                    unsigned long long* votes) {
+                                                    unsigned long long* votes, float reach) {
     apply_scalars(f, P, n, ds);
     for (unsigned long long i0 = blockIdx.x * (unsigned long long)blockDim.x; i0 < n;
          i0 += (unsigned long long)gridDim.x * blockDim.x) {
@@ -1015,7 +1015,7 @@ __global__ void __launch_bounds__(256) k_scott_prep(F f, ScottParams P, Seeds s,
         const bool in = i < n;
         float p0[3] = {0.f, 0.f, 0.f};
         if (in) { p0[0] = s.x[i]; p0[1] = s.y[i]; p0[2] = s.z[i]; }
-        if (votes && blockIdx.x % kVoteBlocks == 0) vote_near(votes, p0, in, kDenseCells);
+        if (votes && blockIdx.x % kVoteBlocks == 0) vote_near(votes, p0, in, reach);
         if (!in) continue;
         R u0[3], v0[3], b0z;
         double nb0;
@@ -1099,7 +1099,7 @@ __global__ void __launch_bounds__(256) k_scott_persistent(F f, ScottParams P, Se
     if (!picked(pick, true)) return;
     scott_persistent_body<R, F, FJ, X>(f, P, s, n, frames, recs, ds, queues, nq, refill_min, order, fj);
 }
-// The mixed variant, at two waves per SIMD.
+// The mixed variant, and FP32c lines with the twist, at two waves per SIMD.
 template <typename R, class F, class FJ, typename X>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_scott_persistent_w2(F f, ScottParams P, Seeds s, unsigned long long n, const R* frames, ScottRec<R>* recs,
@@ -1283,8 +1283,10 @@ struct ScottLines {
 template <typename R, class F, class FJ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1)))
 k_scott_quads(F f, ScottParams P, Seeds s, unsigned long long n, const R* frames, ScottRec<R>* recs, DevScalars ds,
-              unsigned long long* queue, int spread, int refill_min, const unsigned* order, FJ fj, Pick pick) {
+              unsigned long long* queue, int spread, int refill_min, const unsigned* order, FJ fj, Pick pick,
+              FarGrid far) {
     if (!picked(pick, false)) return;
+    if (far.blocks && (int)blockIdx.x >= far.blocks && (long long)far.votes[0] <= 0) return;
     apply_scalars(f, P, n, ds);
     fj.n[0] = f.n[0]; fj.n[1] = f.n[1]; fj.n[2] = f.n[2];  // J lives on B's grid
     P.ctl = scott_ctl(P.tol);  // on the device, so every path forms the same bits
@@ -1771,7 +1773,9 @@ struct ScottStepping {
     decltype(&k_scott_persistent<R, F, FJ, X>) kern = nullptr;
     int grid = 0, quads = 0;
     unsigned long long lines = 0, ordered_up_to = 0, work = 0;
-    bool dense = false;
+    float reach = 0.f;  // > 0: the seeds vote, within so many cells,
+    bool both = false;  // and near ones go by lanes,
+    int far = 0;        // or far ones in so many workgroups of quads
 };
 
 // FP32c RK4 lines from which dense seeds go by lanes, three wavefronts a SIMD, as the
@@ -1782,6 +1786,19 @@ struct ScottStepping {
 // samples a quarter of a cell apart take 37.7 / 39.3, half a cell 65 / 71, lines anywhere
 // 84 / 95; RKF45 maps 0.99-1.05.
 constexpr unsigned long long kScottDenseLines = 1ull << 20;
+// FP32c lines on component arrays, whose stage point touches twelve cache lines: the
+// quads take two wavefronts a SIMD and not four, and lines far apart one, so that these
+// lines stay in the L2 caches (4 / 2 / 1 a SIMD / by lanes, ms: maps on 256 x 200 x 160,
+// RKF45 262,144 lines 11.7 / 8.6 / 8.2 / 15.8; seeds anywhere 44 / 37 / 22.5 / 44, RK4 100 / 82 /
+// 41 / 92, 1 M 421 / 421 / 153 / 424).  Near RK4 lines by lanes from 300,000 on (160 x 128 x
+// 128 400,000 7.5 / 7.7 / 10.8 / 7.4, 1 M 19.8 / 20.3 / 26 / 13.5; 262,144 5.1 / 4.8 / 6.6 /
+// 6.5).  On a small field no line is far, and many go by lanes, RKF45 from 300,000 and RK4
+// from 180,000 on (64^3 RKF45 map 262,144 3.6 / 3.7 / 5.2 / 5.0, 400,000 5.3 / 5.7 / 8.1 / 5.5,
+// 1 M 13.5 / 13.7 / 20 / 11.4; RK4 anywhere 200,000 9.0 / 8.5 / 8.7 / 9.0, 400,000 17.4 / 16.8 /
+// 17.6 / 16.1; with the twist 200,000 13.1 / 11.8 by four a SIMD / by lanes).
+constexpr unsigned long long kScottArraysVoteLines = 65536, kScottArraysNearLines = 300000;
+constexpr unsigned long long kScottArraysSmallRkf45 = 300000, kScottArraysSmallRk4 = 180000;
+constexpr unsigned long long kScottSmallBytes = 16ull << 20;  // 64^3 float nodes are 3, 256 x 200 x 160 94 MiB
 
 // FP64 lines up to which a launch may go by quads, four a resident quad: above it
 // the quads' extra instructions cost more than their shorter chain gives where
@@ -1823,13 +1840,13 @@ constexpr int kScottSpread = 2;
 constexpr int kScottQuadRefillFp32 = 1, kScottQuadRefillFp64 = 2;
 
 template <typename R, class F, class FJ, typename X>
-static int scott_stepping(ScottStepping<R, F, FJ, X>* st, const F& f, int method, unsigned long long n) {
+static int scott_stepping(ScottStepping<R, F, FJ, X>* st, const F& f, int method, unsigned long long n, bool pairs) {
     const int pct = g_tune[FQSL_TUNE_GRID_PCT];
+    const unsigned long long bytes = 3ull * sizeof(R) * f.n[0] * f.n[1] * f.n[2];
     bool lanes = !std::is_same<R, X>::value, quads = !lanes;
     st->work = 0;
     if (sizeof(R) == 8 && method == kRK4) {
-        const unsigned long long nodes = (unsigned long long)f.n[0] * f.n[1] * f.n[2];
-        const unsigned long long work = scott_fp64_quad_work(3ull * sizeof(R) * nodes);
+        const unsigned long long work = scott_fp64_quad_work(bytes);
         if (n > work) {
             lanes = true;
             st->work = work;
@@ -1842,13 +1859,31 @@ static int scott_stepping(ScottStepping<R, F, FJ, X>* st, const F& f, int method
     }
     st->kern = nullptr;
     st->grid = st->quads = 0;
-    st->dense = false;
+    st->reach = 0.f;
+    st->both = false;
+    st->far = 0;
+    bool arrays = false;
     if constexpr (!std::is_same<R, X>::value) st->kern = k_scott_persistent_w2<R, F, FJ, X>;
     else if constexpr (sizeof(R) == 8) {
         if (lanes) st->kern = k_scott_persistent<R, F, FJ, X>;
     } else if constexpr (std::is_same<F, FieldCell32>::value && !has_current<FJ>()) {
-        st->dense = method == kRK4 && n > kScottDenseLines;
-        if (st->dense) st->kern = k_scott_persistent_w3<R, F, FJ, X>;
+        st->both = method == kRK4 && n > kScottDenseLines;
+        if (st->both) st->reach = kDenseCells;
+    } else if constexpr (std::is_same<F, FieldSoA<float>>::value) {
+        arrays = !pairs;
+        if (arrays && bytes <= kScottSmallBytes) {
+            lanes = n > (method == kRK4 ? kScottArraysSmallRk4 : kScottArraysSmallRkf45);
+            quads = !lanes;
+        } else if (arrays && n > kScottArraysVoteLines) {
+            st->both = method == kRK4 && n > kScottArraysNearLines;
+            st->reach = kNearCells;
+        }
+    }
+    if constexpr (sizeof(R) == 4 && std::is_same<R, X>::value) {
+        if (lanes || st->both) {
+            if constexpr (rollable_stages<R, X, FJ>()) st->kern = k_scott_persistent_w3<R, F, FJ, X>;
+            else st->kern = k_scott_persistent_w2<R, F, FJ, X>;
+        }
     }
     int rc = st->kern ? persistent_grid(st->kern, &st->grid) : FQSL_OK;
     if constexpr (std::is_same<R, X>::value)
@@ -1857,7 +1892,11 @@ static int scott_stepping(ScottStepping<R, F, FJ, X>* st, const F& f, int method
     for (int* g : {&st->grid, &st->quads})
         if (*g) *g = std::max(1, (int)((long)*g * pct / 100));
     st->lines = st->quads ? 64ull * st->quads : 256ull * st->grid;
-    st->ordered_up_to = st->quads && !st->dense ? 16ull * st->lines : 64ull * 256ull * st->grid;
+    st->ordered_up_to = st->quads && !st->both ? 16ull * st->lines : 64ull * 256ull * st->grid;
+    if (arrays && st->quads) {
+        st->far = st->reach > 0.f ? std::max(1, st->quads / 4) : 0;
+        st->quads = std::max(1, st->quads / 2);
+    }
     return FQSL_OK;
 }
 
@@ -1896,21 +1935,24 @@ static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, co
     if (e != hipSuccess) return e;
     if (timed && record_start(st)) return hipErrorUnknown;
     k_scott_prep<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(f, P, s, n, frames, o, ds,
-                                                                    step.dense ? q + kSlotVotes : nullptr);
-    // dense lines go by lanes, ordered; by quads such a launch is not
-    const Pick dense{step.dense ? q + kSlotVotes : nullptr};
+                                                                    step.reach > 0.f ? q + kSlotVotes : nullptr,
+                                                                    step.reach);
+    // the order that only near lines by lanes need is left out where they are not
+    const bool quads_ordered = ordered && n_hint <= 16ull * step.lines;
+    const Pick near{step.both && !quads_ordered ? q + kSlotVotes : nullptr};
     if (ordered) {
         k_zero_u32<<<1, 256, 0, st>>>(counts, kOrderBuckets);
         k_order_predict<R, F><<<grid_for((long)n_hint, 256), 256, 0, st>>>(
-            f, s, n, g_tune[FQSL_TUNE_ORDER_BUCKETS], key, counts, dense);
+            f, s, n, g_tune[FQSL_TUNE_ORDER_BUCKETS], key, counts, near);
         k_order_scan<<<1, kOrderBuckets, 0, st>>>(counts, g_tune[FQSL_TUNE_ORDER_BUCKETS],
                                                   step.work ? q + kSlotVotes : nullptr, step.work);
         const int sg = grid_for((long)n_hint, 256) < 4096 ? grid_for((long)n_hint, 256) : 4096;
-        k_order_scatter<<<sg, 256, 0, st>>>(key, n, counts, order, dense);
+        k_order_scatter<<<sg, 256, 0, st>>>(key, n, counts, order, near);
     }
     if (timed) e = hipEventRecord(g_evs0, st);
     // without the estimated lengths nothing tells which of two kernels is the faster one
-    const Pick pick{(step.work && ordered) || step.dense ? q + kSlotVotes : nullptr};
+    const Pick pick{(step.work && ordered) || step.both ? q + kSlotVotes : nullptr};
+    const FarGrid far{step.far ? q + kSlotVotes : nullptr, step.far};
     if constexpr (std::is_same<R, X>::value) {
         if (step.quads) {
             const QuadGrid g = quad_grid(n_hint, step.quads, kScottSpread, quad_min<R>());
@@ -1921,13 +1963,13 @@ static hipError_t scott_persistent_launches(const F& f, const ScottParams& P, co
                 if (pairs) {
                     k_scott_quads<R, FieldPairs, FJ><<<grid, 256, 0, st>>>(
                         FieldPairs{pairs, {f.n[0], f.n[1], f.n[2]}}, P, s, n, frames, recs, ds, q, waves, refill, order, fj,
-                        pick);
+                        pick, far);
                     done = true;
                 }
             }
             if (!done)
                 k_scott_quads<R, F, FJ><<<grid, 256, 0, st>>>(f, P, s, n, frames, recs, ds, q, waves, refill,
-                                                              step.dense ? nullptr : order, fj, pick);
+                                                              near.votes ? nullptr : order, fj, pick, far);
         }
     }
     if (step.kern && (pick.votes || !step.quads))
@@ -1965,7 +2007,7 @@ static int launch_scott(const F& f, const ScottParams& P, const Seeds& s, unsign
         // n_hint: number of lines, known on the host (sizes the workspace)
         if (n_hint == 0) return FQSL_OK;
         ScottStepping<R, F, FJ, X> step;
-        int rc = scott_stepping<R, F, FJ, X>(&step, f, P.method, n_hint);
+        int rc = scott_stepping<R, F, FJ, X>(&step, f, P.method, n_hint, pairs != nullptr);
         if (rc) return rc;
         const bool ordered = scott_ordered<R, F, FJ, X>(ds, f, n_hint, step);
         const ScottWs w = scott_ws_layout<R>(n_hint, ordered);

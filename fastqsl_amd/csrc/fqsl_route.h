@@ -69,8 +69,8 @@ inline bool plain_by_lines(bool in_place, bool per_line, bool capturing) {
 
 // Most FP64 RK4 Scott lines' worth of work, counted in longest lines of the launch
 // by the queue order's estimate, that go by quads of lanes.  By lanes a launch that
-// fits the chip takes as long as its longest line (3.3 us an evaluation on a field
-// that the L2 caches hold, 5.0 on a larger one); by quads the chip does an
+// fits the chip takes as long as its longest line (3.3 us an evaluation on a field of
+// 6 or 9 MiB, 5.0 on one of 50 or 90); by quads the chip does an
 // evaluation every 0.12-0.15 ns, so the two meet where the work is that many longest
 // lines.  ms by quads / by lanes: 64^3 seeds anywhere, 24,576 lines (14,500 longest)
 // 3.8 / 4.3, 32,768 (19,400) 4.5 / 4.4, 65,536 (38,600) 6.6 / 4.4, a 256^2 map (13,300)

@@ -98,7 +98,7 @@ def test_every_device_allocation_may_find_kept_memory():
 def test_fp64_work_that_goes_by_quads(route):
     f = route.rt_scott_fp64_quad_work
     f.restype, f.argtypes = ctypes.c_ulonglong, [ctypes.c_ulonglong]
-    assert f(24 * 64 ** 3) == f(32 << 20) == 19000      # fields that the eight 4 MiB L2 caches hold
+    assert f(24 * 64 ** 3) == f(32 << 20) == 19000
     assert f((32 << 20) + 1) == f(24 * 256 ** 3) == 34000
 
 
