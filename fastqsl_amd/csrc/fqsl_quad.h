@@ -423,10 +423,10 @@ FQSL_COLD double plain_tol(double bn, double tol_coef) {
 
 // Step control (TraceBlineAdaptive.cu:365-370) with the hardware's estimates: scales s,
 // false when the step is rejected.
-__device__ __forceinline__ bool next_step(double& s, double tol, double e2) {
+__device__ __forceinline__ bool next_step(double& s, double tol, double e2, double limit) {
     double q;
     float g;
-    if (step_is_plain(s, tol, e2)) {
+    if (step_is_plain(tol, e2, limit)) {
         q = scale_argument(tol, e2, __builtin_amdgcn_rsq(e2));
         g = __builtin_amdgcn_exp2f(0.2f * __builtin_amdgcn_logf((float)q));
     } else {
@@ -443,11 +443,12 @@ struct SideTracer {
     SideField<K, F> f;
     SideGeom<K, G, R> geo;
     const PlainParams& P;
-    double len_lim;
+    double len_lim, tol_limit;
     int step_lim;
 
     __device__ __forceinline__ SideTracer(const F& ff, const G& g, const PlainParams& p, int a)
-        : f(ff, a), geo(g, ff.n, a), P(p), len_lim(geo.len_lim(p.method)), step_lim(geo.step_lim(p.method)) {}
+        : f(ff, a), geo(g, ff.n, a), P(p), len_lim(geo.len_lim(p.method)),
+          tol_limit(step_tol_limit(p.s0)), step_lim(geo.step_lim(p.method)) {}
 
     __device__ __forceinline__ void unit(const Coord<R>* x, const R* d, R b[K]) const {
         int c[K];
@@ -556,7 +557,7 @@ struct SideTracer {
             L.evals += 6;
             bool accept;
             if constexpr (sizeof(R) == 4) {
-                accept = next_step(L.s, L.tol, e2);
+                accept = next_step(L.s, L.tol, e2, tol_limit);
             } else {
                 const double scale = pow(L.tol / sqrt(e2) / 11.09, 0.2);
                 accept = !(scale < 0.618);

@@ -55,12 +55,13 @@ FQSL_HD Step step_of_scale(double s, double scale) {
     if (s < 1. / 10.) s = 1. / 10.;
     return Step{s, true};
 }
-// Where the estimates hold, s being the attempt's step: nothing under- or overflows, in
-// double nor in the float of q (below 1e35), and a step beyond its upper bound was not
-// rejected.  Zero, infinite, NaN and extreme values, and first steps of 160 and more, go
-// as written.
-FQSL_HD bool step_is_plain(double s, double tol, double e2) {
-    return e2 > 1e-60 && e2 < 1e60 && tol > 1e-60 && tol < 1e6 && s < 160.0;
+// Where the estimates hold: nothing under- or overflows, in double nor in the float of
+// q (below 1e35), and a step beyond its upper bound was not rejected.  Zero, infinite, NaN
+// and extreme values go as written, and so does a trace with a first step s0 of 160 or
+// more (later ones are at most 100 or smaller than it): `limit` is step_tol_limit(s0).
+FQSL_HD double step_tol_limit(double s0) { return s0 < 160.0 ? 1e6 : 0.0; }
+FQSL_HD bool step_is_plain(double tol, double e2, double limit) {
+    return e2 > 1e-60 && e2 < 1e60 && tol > 1e-60 && tol < limit;
 }
 
 // The step after an attempt with step s, from q = tol / err / 11.09 and g, which is q^0.2
