@@ -528,7 +528,7 @@ def bench_neighbour(args, fq, torch, log):
                                "(tol_coef 0.1) + Qcut; K maps over %d streams" % (n, n, nstreams),
                    "pixels_per_step": n * n, "pseudo_pixels": npseudo, "precision": args.precision,
                    "schedule": args.schedule, "parallelism": "single GPU"},
-        "roofline": hbm_roofline("neighbour", "k_plain_%s (main trace)" % args.schedule, k, evals, bpe,
+        "roofline": hbm_roofline("neighbour", plain_kernel(n * n) + " (main trace)", k, evals, bpe,
                                  (args.precision, args.schedule, n) == ("fp32c", "persistent", 1024)),
         "cpu_baseline": cpu,
         **extra,
@@ -631,8 +631,7 @@ def bench_twist(args, fq, torch, log):
                                "twist, RKF45 tol 1e-6, z=0 plane %dx%d" % (n, n),
                    "lines_per_step": nlines, "precision": args.precision, "schedule": args.schedule,
                    "parallelism": "single GPU"},
-        "roofline": dict(hbm_roofline("twist", ("stepping kernel k_scott_persistent_w2 (twist)" if persistent
-                                                 else "k_scott_per_line (twist)"), k, evals, bpe),
+        "roofline": dict(hbm_roofline("twist", "stepping kernel %s (twist)" % scott_kernel(args, nlines), k, evals, bpe),
                          note="HBM traffic not profiled; stage evaluations only (the two J and B "
                               "interpolations per accepted step for the twist are not counted)"),
         "cpu_baseline": cpu,
@@ -660,10 +659,10 @@ def bench_stretch(args, fq, torch, log):
     cells 0.055-0.13) and z spacing growing with height (geometric, strength
     3; cells 0.013-0.24), box [-10,10]^2 x [0,20]; 1024^2 seeds on z = 1e-3
     over [-9.5, 9.5]^2, s_len 0.01, tol_coef 1e-2, the reference's bisection
-    cell rule (flag_uni false).  FP32c (one thread per line by default:
-    these lines are short, ~200 evaluations, and adjacent seeds in one
-    wavefront share cache lines) against FP64 one thread per line on the
-    same GPU, and the FP64 oracle on the host."""
+    cell rule (flag_uni false).  FP32c against FP64 on the same GPU (the
+    per-line schedule of both; either traces the sides nearly tangent to the
+    plane by quads of lanes and the rest one side a lane), and the FP64 oracle
+    on the host."""
     dev = torch.device("cuda", 0)
     steps = args.steps or 5
     warm = args.warmup if args.warmup is not None else 1
@@ -756,7 +755,7 @@ def bench_stretch(args, fq, torch, log):
                                "%dx%d" % (n, n),
                    "lines_per_step": nlines, "precision": args.precision, "schedule": args.schedule,
                    "parallelism": "single GPU"},
-        "roofline": hbm_roofline("stretch", "k_plain_%s (stretched)" % args.schedule, k, evals, bpe,
+        "roofline": hbm_roofline("stretch", plain_kernel(nlines) + " (stretched)", k, evals, bpe,
                                  (args.precision, args.schedule, n) == ("fp32c", "per_line", 1024)),
         "cpu_baseline": cpu,
         "classes": {str(int(c)): int(v) for c, v in zip(classes, counts)},
@@ -785,18 +784,34 @@ def profile_values(workload):
     return vals
 
 
+def scott_kernel(args, lines):
+    """The kernel that traces an RKF45 launch of so many lines on a cell field."""
+    if args.schedule != "persistent":
+        return "k_scott_per_line"
+    quads = args.precision == "fp32c" or (args.precision == "fp64" and lines <= 65536)
+    return "k_scott_quads" if quads else "k_scott_persistent"
+
+
+def plain_kernel(lines):
+    """The kernel that traces a plain RKF45 launch of so many lines: tangent
+    lines by quads and the rest by lanes, or few lines all by quads."""
+    return "k_plain_sides" if lines > 65536 else "k_plain_quads"
+
+
 def valu_roofline(workload, kernel_ms, evals, bpe, oracle_evals=None, kernel="", flops_per_eval=FLOPS_PER_EVAL):
-    """Roofline of a stepping kernel bound by VALU issue.  achieved / peak is
-    the issue rate of VALU wave instructions (4 cycles per wave64 instruction
-    on a SIMD16) against the chip's (1,024 SIMDs at the engine clock); the
-    instruction count per launch comes from the workload's rocprofv3 profile
-    (SQ_INSTS_VALU), the kernel time is measured live.  Beside it: HBM
+    """Roofline of a stepping kernel whose nearest limit is VALU issue.  achieved
+    / peak is the issue rate of VALU wave instructions against the chip's at
+    its highest engine clock, 1,024 SIMDs at one instruction per 4 cycles (a
+    model: SIMD16 and wave64); the clock of the run is not known, so the share
+    of the slots it really had is larger.  The instruction count per launch
+    comes from the workload's rocprofv3 profile (SQ_INSTS_VALU), the kernel
+    time is measured live.  Beside it: HBM
     traffic (profile) and algorithmic flops against their peaks, and the
     no-reuse stencil model (96 B per stage evaluation)."""
     pv = profile_values(workload)
     t = kernel_ms * 1e-3
     insts = pv.get("valu_insts_per_launch")
-    clk = pv.get("sclk_mhz", SCLK_PEAK_MHZ) * 1e6
+    clk = SCLK_PEAK_MHZ * 1e6
     peak = N_SIMDS * clk / 4.0
     traffic = pv.get("traffic_bytes_per_launch")
     rec = {"bound": "valu", "kernel": kernel, "kernel_ms": kernel_ms,
@@ -994,8 +1009,7 @@ def bench_trace(args, fq, torch, log, volume):
     classes, counts = np.unique(flags, return_counts=True)
     prof = "volume" if volume else "plane"
     roof = valu_roofline(prof, kms, evals, bpe, oracle_evals,
-                         kernel=("k_scott_per_line" if args.schedule != "persistent" else
-                                 "stepping kernel " + ("k_scott_quads" if args.precision == "fp32c" else "k_scott_persistent")))
+                         kernel="stepping kernel " + scott_kernel(args, nlines))
     if not (args.precision == "fp32c" and args.schedule == "persistent" and (volume or args.pixels == 1024)):
         roof.update(achieved=None, frac=None, valu_insts_per_launch=None, traffic=None,
                     note="the profile covers the default FP32c persistent workload only")

@@ -4,8 +4,9 @@
 //   k_build_cells          SoA float field -> 128-byte cells of trilinear coefficients
 //   k_scott_quads          Scott tracer, persistent grid, lines refilled from a
 //                          device work queue, one line per quad of lanes
-//   k_scott_persistent     the same with one line per lane: the mixed variant
-//                          and large FP64 launches
+//   k_scott_persistent     the same with one line per lane: the mixed variant,
+//                          large FP64 launches, dense RK4 maps, many lines on
+//                          component arrays
 //   k_scott_per_line       Scott tracer, one thread per line
 //   k_plain_quads / k_plain_sides   position-only tracer (grid-index
 //                          coordinates, or a stretched grid's own coordinates)
@@ -1125,7 +1126,7 @@ k_scott_persistent_w3(F f, ScottParams P, Seeds s, unsigned long long n, const R
 // when the line is done.  Ended sides are landed, second sides
 // begun and free quads refilled together, once `refill_min` quads wait or none
 // is tracing; free quads take lines from the wavefront's own run, claimed a
-// share of the rest at a time (see trace_sides).
+// part of the rest at a time (1/8 to 1/4 of its even share, as in trace_sides).
 template <typename R, class F, class FJ, class Src>
 __device__ __forceinline__ void scott_quads_body(const F& f, Src src, unsigned long long n,
                                                  const R* __restrict__ frames, ScottRec<R>* __restrict__ recs,
@@ -1274,12 +1275,14 @@ struct ScottLines {
 // does a stage's three components in turn: a line's chain took 1.3 us an
 // evaluation, its six cell loads touch 384 cache lines a wavefront.  By quads
 // 0.5 us and a third of the cache lines, for 1.5 times the instructions a line;
-// FP32c launches of every size gain or stay (multipole 256^3, RKF45 1e-6, ms
+// FP32c RKF45 launches on cells of every size gain or stay (multipole 256^3, 1e-6, ms
 // before and after: 64 lines 1.87 / 0.78, 256^2 4.5 / 2.05, 512^2 5.9 / 3.0,
 // 1024^2 9.2 / 8.7; 512^2 with twist 5.2 / 3.1; cell cube of 8.4 M lines
-// 217 / 193).  Four wavefronts a SIMD: from 512^2 lines on bound by vector
-// instruction issue (98 instructions a stage of 16 lines, all issue slots
-// taken).  `spread` wavefronts share few lines before one takes a second.
+// 217 / 193), but for maps of 1.7-4 M lines on 64^3 (0.93-0.95).  Dense RK4 maps, FP64
+// and component arrays: see scott_stepping.  Four wavefronts a SIMD: from 512^2
+// lines on vector instruction issue is nearest its limit (125 instructions an
+// evaluation of 16 lines, 0.95-0.98 of the slots at four cycles each, counts and
+// clock of one launch).  `spread` wavefronts share few lines before one takes a second.
 template <typename R, class F, class FJ>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1)))
 k_scott_quads(F f, ScottParams P, Seeds s, unsigned long long n, const R* frames, ScottRec<R>* recs, DevScalars ds,
@@ -1499,7 +1502,8 @@ __device__ __forceinline__ void trace_sides(const F& f, const PlainParams& P, co
     const bool mine = (K == 3 ? lane : lane >> 2) < width;
     const unsigned long long below = (1ull << (K == 3 ? lane : lane & ~3)) - 1ull;
     const unsigned long long tasks = 2ull * n;
-    // a claim takes 1/4 of a wavefront's even share of the rest
+    // a claim takes between 1/8 and 1/4 of a wavefront's even share of the rest: with a
+    // power of two a shift stands for the quotient
     const int share_shift = 66 - __clzll((long long)gridDim.x * (blockDim.x >> 6));
     unsigned long long line = 0, next = 0, end = 0;
     bool drained = false;
